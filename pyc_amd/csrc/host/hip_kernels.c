@@ -30,7 +30,7 @@ int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int tile, int M, int N, 
                               void* stream);
 int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C,
                                float alpha, float beta, const float* bias, int epi, void* stream);
-int pyc_hip_gemm_nn_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C,
+int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N, int K, const void* A, const void* B, void* C,
                                float alpha, float beta, const float* bias, int epi, void* stream);
 int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A, const void* B,
                             void* C, float alpha, float beta, const float* bias, int epi,
@@ -241,7 +241,7 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
      * large NN shapes; the _lds symbols name it alone (-1 outside its
      * preconditions), the shape-chosen symbols fall back to the tiled kernels. */
     if (!v->b_trans && (v->tile == -1 || (v->tile == 0 && pick_half_tile(M, N) == 256))) {
-        const int rc = pyc_hip_gemm_nn_lds_launch(v->dtype == VT_BF16, M, N, K, A, B, C, alpha, beta, bias,
+        const int rc = pyc_hip_gemm_nn_lds_launch(v->dtype == VT_BF16, v->tile == 0, M, N, K, A, B, C, alpha, beta, bias,
                                                   epilogue, stream);
         if (rc != 1) {
             return rc;

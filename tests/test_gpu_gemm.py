@@ -384,3 +384,39 @@ def test_reference_bf16_symbol_8192_row_major_b(gpu):
     colsum = Cd.float().sum(0).double()
     pred = (A.double().sum(0, keepdim=True) @ B.double()).squeeze(0)
     assert (colsum - pred).abs().max().item() <= 1e-2 * pred.abs().max().item()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("m,n,k,epi", [
+    (4095, 4096, 64, 3),    # one row short of whole tiles, a single k stage
+    (3841, 4104, 128, 0),   # 1 row and 8 columns into the last tiles, more tiles than CUs
+    (257, 32768, 64, 1),    # two tile rows, the second of one row
+])
+def test_ragged_persistent_gemm(gpu, m, n, k, epi, layout, dtype):
+    """At least one 256 x 256 tile per CU with M or N no multiple of 256: the
+    persistent kernel's ragged form. Every element against the oracle, and
+    nothing is written past the end of C."""
+    torch = gpu
+    bt = layout == "nt"
+    r = np.random.default_rng(m + n + k)
+    t = torch.bfloat16 if dtype == "bf16" else torch.float16
+    a32 = (r.standard_normal((m, k)) / np.sqrt(k)).astype(np.float32)
+    b32 = r.standard_normal((n, k) if bt else (k, n)).astype(np.float32)
+    bias = r.standard_normal(n).astype(np.float32)
+    A, B, Bd = torch.from_numpy(a32).cuda().to(t), torch.from_numpy(b32).cuda().to(t), dev_f32(torch, bias)
+    Cd = torch.full((m * n + 4096,), 7.0, dtype=t, device="cuda")
+    pyc_amd.gemm(f"hip_gemm_{dtype}_{layout}", A, B, Cd, m, n, k, bias=Bd, epilogue=epi)
+    torch.cuda.synchronize()
+    assert bool((Cd[m * n:] == 7.0).all())
+    a, b = A.float(), B.float()
+    ref = (a @ (b.t() if bt else b)).cpu().numpy()
+    if epi & 1:
+        ref = ref + bias
+    if epi & 2:
+        ref = np.maximum(ref, 0.0)
+    got = Cd[:m * n].float().cpu().numpy().reshape(m, n)
+    # one rounding of the result (2^-8 or 2^-11 relative) plus fp32 summation order
+    bound = 2.0 ** (-8 if dtype == "bf16" else -11) * np.abs(ref) + 4e-6 * np.sqrt(k) * np.abs(ref).max()
+    bad = np.abs(got - ref) > bound
+    assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
