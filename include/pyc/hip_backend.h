@@ -68,7 +68,9 @@ int pyc_hip_attention_dispatch(
  * C_in % 8 == 0. The symbol fixes the element type and the kernel path:
  *   hip_conv2d_bf16 / _f16          by shape: whole 256 x 256 tiles on the
  *                                   persistent kernel, a second partial round
- *                                   on 160-pixel tail tiles, else the tiles below
+ *                                   on 144-pixel tail tiles, or LDS-DMA tiles of
+ *                                   32 to 128 pixels, whichever is estimated
+ *                                   fastest, else the tiles below
  *   hip_conv2d_bf16_persist / _f16_persist   every tile on the persistent kernel
  *                                   (no tail kernel), else the tiles below
  *   hip_conv2d_bf16_tiled / _f16_tiled       the register-staged implicit-GEMM

@@ -25,7 +25,7 @@
 int pyc_hip_gemm_half_launch(int is_bf16, int b_trans, int tile, int M, int N, int K,
                              const void* A, const void* B, void* C, float alpha, float beta,
                              const float* bias, int epi, void* stream);
-int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int tile, int M, int N, int K, const void* A,
+int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
                               const void* B, void* C, float alpha, float beta, const float* bias, int epi,
                               void* stream);
 int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C,
@@ -37,6 +37,12 @@ int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A, con
                             void* stream);
 int pyc_hip_attention_launch(int is_bf16, int B, int H, int S, int D, int causal, const void* Q,
                              const void* K, const void* V, void* O, float scale, void* stream);
+int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg, int H, int W, int C, int Kout, int R, int S,
+                                int ph, int pw, int sh, int sw, const void* x, const void* w, const float* bias,
+                                int relu, void* y, void* stream);
+int pyc_hip_conv2d_persist_launch(int is_bf16, int tail, int Nimg, int H, int W, int C, int Kout, int R, int S, int ph,
+                                  int pw, int sh, int sw, const void* x, const void* w, const float* bias, int relu,
+                                  void* y, void* stream);
 int pyc_hip_conv2d_launch(int is_bf16, int path, int N, int H, int W, int C, int K, int R, int S, int ph,
                           int pw, int sh, int sw, const void* x, const void* w, const float* bias,
                           int relu, void* y, void* stream);
@@ -204,14 +210,72 @@ int pyc_hip_kernel_symbol_count(const char* op_key) {
 
 /* ---------------------------------------------------------------- GEMM */
 
-/* Tile choice for shape-generic symbols: the 256x256 tile when it still gives
- * at least one workgroup per CU (256 CUs on MI355X), else 128x128 when that
- * gives at least half as many, else 64x64 (small shapes: more workgroups
- * walking K side by side). */
+/* Tile choice among the general register-staged tiles: the 256x256 tile when it
+ * still gives at least one workgroup per CU (256 CUs on MI355X), else 128x128
+ * when that gives at least half as many, else 64x64. */
 static int pick_half_tile(int M, int N) {
     const long t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256);
     const long t128 = (long)((M + 127) / 128) * (long)((N + 127) / 128);
     return t256 >= 256 ? 256 : t128 >= 128 ? 128 : 64;
+}
+
+/* The LDS-DMA tiles and what a product costs on each, in microseconds: a
+ * launch, then for every round of one tile per CU a start and end and K / 64
+ * stages. A stage takes longer the more CUs fetch at once (stage[0] with few of
+ * them busy, stage[1] with all 256), and `many` times as long when there is more
+ * than one round (the operands of the small tiles then come from beyond L2 more
+ * often; the persistent 256 x 256 tile hides its next tile's start). Measured on
+ * the MI355X over products of 0.01 to 180 GFLOP: the tile it picks is within
+ * about 10 % of the best one. Examples, in us, of 32x32 / 64x64 / 128x128 /
+ * 128x256 / 256x256: 512^3 3.7 / 4.4 / 8.0 / 12.4 / 16.6; [N,K] 128 x 1024 x 8192
+ * 13.8 / 22.4 / 50 / 82 / 147; 2048^3 82 / 40 / 21 / 28 / 46; 1024 x 8192 x 4096
+ * - / 158 / 117 / 62 / 86; 1999 x 11008 x 4096 - / 414 / 293 / 223 / 185. */
+typedef struct {
+    int bm, bn;
+    double launch, round, stage[2], many;
+} dma_tile;
+
+enum { DT_32 = 0, DT_64, DT_128, DT_128X256, DT_256, DT_COUNT };
+
+static const dma_tile k_dma_tiles[DT_COUNT] = {
+    {32, 32, 1.0, 2.0, {0.085, 0.15}, 1.0},   {64, 64, 1.0, 2.2, {0.17, 0.19}, 1.4},
+    {128, 128, 1.0, 4.2, {0.34, 0.52}, 1.1},  {128, 256, 1.0, 7.0, {0.57, 0.90}, 1.15},
+    {256, 256, 7.5, 2.0, {1.12, 1.50}, 0.93},
+};
+
+/* `k_rows`: B stored [K,N]; the 32 x 32 tile reads half lines of it, which costs
+ * it up to twice the time once B no longer fits an XCD's 4 MiB L2. `tail`: a
+ * second round on the convolution's tail kernel takes about 0.65 of a round. */
+static double dma_tile_cost(int t, long M, long N, long K, int k_rows, int tail) {
+    const dma_tile* d = &k_dma_tiles[t];
+    const double tiles = (double)((M + d->bm - 1) / d->bm) * (double)((N + d->bn - 1) / d->bn);
+    const double busy = tiles < 256.0 ? tiles / 256.0 : 1.0;
+    double rounds = (double)(long)((tiles + 255.0) / 256.0);
+    double stage = d->stage[0] + (d->stage[1] - d->stage[0]) * busy;
+    if (t == DT_32 && k_rows && (double)K * (double)N * 2.0 > 4194304.0) {
+        stage *= 1.3 + 0.7 * busy;
+    }
+    if (rounds > 1.0) {
+        stage *= d->many;
+    }
+    if (t == DT_256 && tail && rounds == 2.0) {
+        rounds = 1.65;
+    }
+    return d->launch + rounds * (d->round + (double)((K + 63) / 64) * stage);
+}
+
+/* The cheapest of the tiles 0 .. last. */
+static int pick_dma_tile(long M, long N, long K, int k_rows, int tail, int last) {
+    int t, best = 0;
+    double c, cb = dma_tile_cost(0, M, N, K, k_rows, tail);
+    for (t = 1; t <= last; ++t) {
+        c = dma_tile_cost(t, M, N, K, k_rows, tail);
+        if (c < cb) {
+            cb = c;
+            best = t;
+        }
+    }
+    return best;
 }
 
 static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, const void* B,
@@ -228,36 +292,39 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
     if (v->dtype == VT_F32) {
         return pyc_hip_gemm_f32_launch(v->b_trans, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
     }
-    /* The direct-LDS NT kernel takes large NT shapes with K % 64 == 0 (its
-     * launcher answers 1 when the shape is outside its preconditions). */
-    if (v->b_trans && (v->tile == -1 || (v->tile == 0 && pick_half_tile(M, N) == 256))) {
-        const int rc = pyc_hip_gemm_nt_lds_launch(v->dtype == VT_BF16, M, N, K, A, B, C, alpha, beta, bias,
-                                                  epilogue, stream);
+    /* The _lds symbols name the persistent LDS-DMA kernel alone: [N,K] shapes
+     * outside its preconditions (its launcher answers 1) take the tiles below,
+     * [K,N] ones are refused. */
+    if (v->tile == -1) {
+        const int bf = v->dtype == VT_BF16;
+        const int rc = v->b_trans
+                           ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
+                           : pyc_hip_gemm_nn_lds_launch(bf, 0, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
         if (rc != 1) {
             return rc;
         }
-    }
-    /* The persistent LDS kernel with a [K,N] operand (transpose reads) takes
-     * large NN shapes; the _lds symbols name it alone (-1 outside its
-     * preconditions), the shape-chosen symbols fall back to the tiled kernels. */
-    if (!v->b_trans && (v->tile == -1 || (v->tile == 0 && pick_half_tile(M, N) == 256))) {
-        const int rc = pyc_hip_gemm_nn_lds_launch(v->dtype == VT_BF16, v->tile == 0, M, N, K, A, B, C, alpha, beta, bias,
-                                                  epilogue, stream);
-        if (rc != 1) {
-            return rc;
-        }
-        if (v->tile == -1) {
+        if (!v->b_trans) {
             return -1;
         }
     }
-    /* Below the persistent kernel's range: the LDS-DMA ring kernel when the
-     * shape is whole tiles (it answers 1 otherwise), with 64 x 64 tiles while
-     * 128 x 128 ones would not fill the chip (bf16 1536^3: 46 against 54 us
-     * per call with 128 x 128 tiles), else 128 x 128. */
-    if (v->tile == 0 && pick_half_tile(M, N) <= 128) {
-        const int small = (long)((M + 127) / 128) * (long)((N + 127) / 128) < 256;
-        const int rc = pyc_hip_gemm_small_launch(v->dtype == VT_BF16, v->b_trans, small ? 64 : 128, M, N, K, A, B,
-                                                 C, alpha, beta, bias, epilogue, stream);
+    /* The shape-chosen symbols: the LDS-DMA tile that the table above makes the
+     * cheapest. A launcher answers 1 when the shape is outside its kernel's
+     * preconditions (alignment, K % 64 and beta == 0 for the persistent 256 x 256
+     * tile, K % 8 for the others); then the next smaller kind is asked. */
+    if (v->tile == 0) {
+        const int bf = v->dtype == VT_BF16;
+        int t = pick_dma_tile(M, N, K, !v->b_trans, 0, DT_256);
+        if (t == DT_256) {
+            const int rc =
+                v->b_trans ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
+                           : pyc_hip_gemm_nn_lds_launch(bf, 1, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
+            if (rc != 1) {
+                return rc;
+            }
+            t = pick_dma_tile(M, N, K, !v->b_trans, 0, DT_128X256);
+        }
+        const int rc = pyc_hip_gemm_small_launch(bf, v->b_trans, k_dma_tiles[t].bm, k_dma_tiles[t].bn, M, N, K, A, B, C,
+                                                 alpha, beta, bias, epilogue, stream);
         if (rc != 1) {
             return rc;
         }
@@ -316,6 +383,27 @@ int pyc_hip_conv2d_dispatch(const char* symbol, int N, int H, int W, int C_in, i
     }
     if (H + 2 * pad_h < R || W + 2 * pad_w < S) {
         return -1;
+    }
+    if (v->tile == CONV_AUTO) {
+        /* The implicit GEMM [N*P*Q, R*S*C] x [K, R*S*C]: the persistent 256 x 256
+         * tiles (and their tail kernel) for shapes inside their preconditions
+         * where they are the cheapest, else the best of the smaller tiles. */
+        const int bf = v->dtype == VT_BF16;
+        const long P = (H + 2L * pad_h - R) / stride_h + 1, Q = (W + 2L * pad_w - S) / stride_w + 1;
+        const long Mg = (long)N * P * Q, Kg = (long)R * S * C_in;
+        int rc = 1, t = pick_dma_tile(Mg, K, Kg, 0, 1, DT_256);
+        if (t == DT_256) {
+            rc = pyc_hip_conv2d_persist_launch(bf, 1, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h, stride_w, x, w,
+                                               bias, relu ? 1 : 0, y, stream);
+            t = pick_dma_tile(Mg, K, Kg, 0, 1, DT_128X256);
+        }
+        if (rc == 1) {
+            rc = pyc_hip_conv2d_small_launch(bf, k_dma_tiles[t].bm, k_dma_tiles[t].bn, N, H, W, C_in, K, R, S, pad_h,
+                                             pad_w, stride_h, stride_w, x, w, bias, relu ? 1 : 0, y, stream);
+        }
+        if (rc != 1) {
+            return rc;
+        }
     }
     return pyc_hip_conv2d_launch(v->dtype == VT_BF16, v->tile, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h,
                                  stride_w, x, w, bias, relu ? 1 : 0, y, stream);

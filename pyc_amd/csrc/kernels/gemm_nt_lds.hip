@@ -965,7 +965,8 @@ extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, cons
 // NN form (B stored [K,N]) of the persistent kernel: returns 1 when the shape
 // is outside its preconditions (M, N multiples of 256, K of 64, beta == 0,
 // 16-byte aligned C and bias, M*K*2 and K*N*2 below 2^32, at least as many
-// 256 x 256 tiles as CUs), 0 on launch, -2 on a launch error.
+// 256 x 256 tiles as CUs; with `ragged` those of ragged_ok instead of the
+// first, and any number of tiles), 0 on launch, -2 on a launch error.
 extern "C" int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N, int K, const void* A,
                                           const void* B, void* C, float alpha, float beta, const float* bias,
                                           int epi, void* stream) {
@@ -986,11 +987,12 @@ extern "C" int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N,
     }
     const int tiles_m = (M + kD_BM - 1) / kD_BM, tiles_n = (N + kD_BN - 1) / kD_BN;
     const int ntiles = tiles_m * tiles_n;
-    if (ntiles < n_cu) return 1;  // fewer tiles than CUs: the 128 x 128 kernels fill the chip better
+    // the symbol that names this kernel alone takes no fewer tiles than CUs
+    if (!ragged && ntiles < n_cu) return 1;
     if (!whole) return launch_ragged<true>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, n_cu, (hipStream_t)stream);
     hipStream_t s = (hipStream_t)stream;
     const int pepi = (((epi & 1) && bias != nullptr) ? 1 : 0) | (epi & 2);
-    const dim3 grid(n_cu), block(4 * kWave);
+    const dim3 grid(ntiles < n_cu ? ntiles : n_cu), block(4 * kWave);
     const uint16_t* a = (const uint16_t*)A;
     const uint16_t* b = (const uint16_t*)B;
     uint16_t* c = (uint16_t*)C;

@@ -1,4 +1,5 @@
-// gemm_small.hip — bf16/fp16 GEMM for small and medium shapes on gfx950.
+// gemm_small.hip — bf16/fp16 GEMM for small and medium shapes on gfx950, and
+// the implicit-GEMM convolution of the shapes the persistent kernel does not take.
 //
 // C[M,N] = epi(alpha * A[M,K] * op(B) + beta * C), fp32 accumulation, B stored
 // [N,K] ("nt") or [K,N] ("nn", the layout of the reference's default bf16
@@ -7,19 +8,40 @@
 // persistent 256 x 256 kernel's range. A register-staged kernel that prefetches
 // one k-step pays a global round trip per step: 17 us for a 512^3 bf16 GEMM on
 // 16 workgroups. Here the tile's operands move global -> LDS by LDS-DMA
-// through a 128 KB ring: 64 x 64 tiles (16 KB stages, 8 of them, seven k-steps
-// in flight, so a K of up to 512 is in flight after the first issue) or
-// 128 x 128 tiles (32 KB stages, 4, three in flight).
+// through a ring of up to 160 KB of LDS.
 //
-// 4 waves as 2 x 2, each (BM/2) x (BN/2) in 16 x 16 fragments of
-// v_mfma_f32_16x16x32_{bf16,f16}, with the B fragment as the first operand so
-// each lane ends with four adjacent columns of C (8-byte stores).
+// 8 waves, two per SIMD: two groups of four, each group 2 x 2 over the tile
+// ((BM/2) x (BN/2) per wave, 16 x 16 fragments of v_mfma_f32_16x16x32_{bf16,f16})
+// and each on half the k of every ring slot, so that one group's MFMAs run
+// while the other waits at the barrier, on its LDS reads or on its DMA issue;
+// the two sums are added through LDS at the end in a fixed order. A slot is one
+// 64-k stage of a 128-wide tile (each group takes 32 of its k) or 2 or 4 stages
+// of the smaller ones (each group takes half the stages).
+// The B fragment is the first operand of the MFMA, so each lane ends with four
+// adjacent columns of C.
 // A and [N,K] B stage rows are 128 bytes (64 k), 16-byte chunk c of row r at
 // c ^ (r & 7). [K,N] B stages are 64 k-rows of BN columns, 32-byte segment s
 // (16 columns) of k-row k at s ^ f(k): a transpose read (ds_read_b64_tr_b16)
 // by 32 lanes touches 32 bytes of k-rows k0..k0+3 and k0+8..k0+11, which f
-// spreads over the eight 32-byte slots of a 256-byte bank window (two 128-byte
-// rows per window for BN = 64, one 256-byte row for BN = 128).
+// spreads over the eight 32-byte slots of a 256-byte bank window.
+//
+// Code that runs once per tile is kept short (rolled prologue, results through
+// LDS into a rolled store loop): a launch starts with a cold instruction cache,
+// and straight-line code cost about 0.35 us per KiB of it (a 128 x 128 tile with
+// an unrolled epilogue, 13 KiB: 7.1 us for K = 128, where a 3 KiB kernel took 3.1).
+//
+// SRC: where a stage's operands come from.
+//  kDense  K a multiple of 64: a load's offset is the lane's row offset plus a
+//          scalar advance per stage.
+//  kTail   K a multiple of 8: chunks past K (and [K,N] k-rows past K) get an
+//          offset past the buffer's end, which the descriptor reads as zeros
+//          (both operands: a neighbouring row may hold an infinity).
+//  kConv   NHWC convolution, A row = output pixel, k = (r, s, c), B = the KRSC
+//          filter [K_out, R*S*C], C % 8 == 0: a lane's 16-byte chunk is 8
+//          channels of one tap. It is the same k for every row the lane loads,
+//          so a stage's tap is found once per lane (two multiplications by
+//          rounded-up reciprocals); taps in the padding, pixels past the last
+//          and k past R*S*C get the past-the-end offset.
 #include <stdint.h>
 
 #include "common.hpp"
@@ -28,35 +50,56 @@
 namespace pyc {
 
 constexpr int kSmBK = 64;
-constexpr uint32_t kSmRingBytes = 128 * 1024;
+enum { kDense = 0, kTail = 1, kConv = 2 };
+constexpr uint32_t kSmPastEnd = 0xFFFFFFF0u;  // not below any descriptor's byte count
 
-// segment swizzle of a [K,N] k-row: 64-column tiles (128-byte rows, two rows
-// per 256-byte bank window) and 128-column tiles (256-byte rows)
+struct SmConv {
+    int H, W, C, S, P, Q, ph, pw, sh, sw;
+    uint32_t rc, rs;    // ceil(2^32 / C), ceil(2^32 / S) (0 for S == 1)
+    uint32_t x_bytes;
+};
+
+// Ring slots of a BM x BN tile (KS stages of 64 k per slot): as many as fit.
+constexpr int sm_slots(int bm, int bn, int ks) { return 160 * 1024 / (ks * (bm + bn) * 128); }
+constexpr size_t sm_lds_bytes(int bm, int bn, int ks) { return (size_t)sm_slots(bm, bn, ks) * ks * (bm + bn) * 128; }
+
+// segment swizzle f of a [K,N] k-row: (k * BN / 16 + (s ^ f(k))) % 8 differs
+// over k0..k0+3 and k0+8..k0+11
 template <int BN> __device__ inline int sm_kswz(int k) {
-    if constexpr (BN == 64) return ((k >> 1) & 1) | (((k >> 3) & 1) << 1);
+    if constexpr (BN == 32) return (k >> 3) & 1;
+    else if constexpr (BN == 64) return ((k >> 1) & 1) | (((k >> 3) & 1) << 1);
     else return (k & 3) | (((k >> 3) & 1) << 2);
 }
 
-template <typename T, bool BT, int BM>
-__global__ void __launch_bounds__(256, 1)
+template <typename T, bool BT, int BM, int BN, int KS, int SRC>
+__global__ void __launch_bounds__(512, 1)
 gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C,
                   int M, int N, int K, float alpha, float beta, const float* __restrict__ bias, int epi,
-                  int tiles_n) {
-    constexpr int BN = BM;
-    constexpr uint32_t TILE_BYTES = BM * 128;                // one operand's stage: BM rows of 64 k
-    constexpr int STAGES = kSmRingBytes / (2 * TILE_BYTES);  // 8 (64 x 64) or 4 (128 x 128)
-    constexpr int NQ = BM / 32;                              // DMA instructions per wave and operand
-    constexpr int LOADS = 2 * NQ;
+                  int tiles_n, int vec_c, SmConv cg) {
+    constexpr uint32_t A_BYTES = BM * 128, B_BYTES = BN * 128;  // one stage: 64 k of BM and of BN rows
+    constexpr uint32_t STAGE_BYTES = A_BYTES + B_BYTES;
+    constexpr uint32_t SLOT_BYTES = KS * STAGE_BYTES;
+    constexpr int SLOTS = sm_slots(BM, BN, KS);
+    constexpr bool HALF = KS == 1;                           // a group takes 32 k of each stage, else KS/2 stages
+    constexpr int NST = HALF ? 1 : KS / 2;                   // stages a wave loads and multiplies per slot
+    constexpr int NLW = HALF ? 8 : 4;                        // waves that load a stage
+    constexpr int NQA = BM / 8 / NLW, NQB = BN / 8 / NLW;    // DMA instructions per wave, operand and stage
+    constexpr int LOADS = NQA + NQB;
     constexpr int FM = BM / 32, FN = BN / 32;                // fragments per wave
     constexpr int SEGS = BN / 16;                            // 32-byte segments per [K,N] k-row
-    static_assert(STAGES >= 3, "ring");
-    __shared__ __attribute__((aligned(1024))) uint16_t smem[kSmRingBytes / 2];
-    static_assert(sizeof(smem) == kSmRingBytes, "registered LDS figure");
+    constexpr int CH = BN / 8;                               // 16-byte chunks of a wave's row of fp32 results
+    static_assert(SLOTS >= 3 && (SLOTS - 2) * NST * LOADS <= 60, "ring");
+    static_assert(SRC != kConv || BT, "the filter is the [N,K] operand");
+    static_assert(BM * BN * 4 <= SLOTS * SLOT_BYTES, "results through the ring's LDS");
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[SLOTS * SLOT_BYTES / 2];
+    static_assert(sizeof(smem) == sm_lds_bytes(BM, BN, KS), "registered LDS figure");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int kh = wave >> 2, quad = wave & 3;               // group (k half), place in the tile
+    const int lw = HALF ? wave : quad;
+    const int wm = quad >> 1, wn = quad & 1;
     const int lrow = lane & 15, lgrp = lane >> 4;
     // tiles in groups of 4 tile rows, column by column (neighbouring workgroups share B columns)
     const int tiles_m = (M + BM - 1) / BM;
@@ -68,21 +111,37 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     const int in = blockIdx.x - grp * span;
     const int m0 = (first_m + in % gsz) * BM;
     const int n0 = (in / gsz) * BN;
-    const int KT = K / kSmBK;
+    const int KT = (K + kSmBK - 1) / kSmBK;
 
-    const i32x4 ra = make_buf_rsrc(A, (uint32_t)((size_t)M * K * 2));
+    const i32x4 ra = make_buf_rsrc(A, SRC == kConv ? cg.x_bytes : (uint32_t)((size_t)M * K * 2));
     const i32x4 rb = make_buf_rsrc(B, (uint32_t)((size_t)N * K * 2));
-    // DMA instruction q = NQ wave + h of an operand fills LDS bytes
-    // 1024 q .. +1023: 8 rows of 128 bytes (A, [N,K] B; lane i at 16-byte
-    // position i % 8 of row i / 8) or 1024 / (2 BN) k-rows of [K,N] B
-    uint32_t va[NQ], vb[NQ];
+    // DMA instruction q = NQ lw + h of an operand fills LDS bytes
+    // 1024 q .. +1023 of its stage: 8 rows of 128 bytes (A, [N,K] B; lane i at
+    // 16-byte position i % 8 of row i / 8) or 1024 / (2 BN) k-rows of [K,N] B
+    const int lch = (lane & 7) ^ (lane >> 3);  // logical chunk of this lane, the same in every row it loads
+    uint32_t va[NQA], vb[NQB];
+    int ih0[SRC == kConv ? NQA : 1], iw0[SRC == kConv ? NQA : 1];
 #pragma unroll
-    for (int h = 0; h < NQ; ++h) {
-        const int q = NQ * wave + h;
-        const int row = 8 * q + lane / 8, p = lane % 8;
-        va[h] = (uint32_t)(((size_t)(m0 + row) * K + 8 * (p ^ (row & 7))) * 2);
+    for (int h = 0; h < NQA; ++h) {
+        const int m = m0 + 8 * (NQA * lw + h) + lane / 8;
+        if constexpr (SRC == kConv) {
+            const int pq = cg.P * cg.Q;
+            const int n = m / pq, r = m - n * pq;
+            const int p = r / cg.Q, q = r - p * cg.Q;
+            ih0[h] = m < M ? p * cg.sh - cg.ph : -(1 << 30);  // no tap of a pixel past the last is inside
+            iw0[h] = q * cg.sw - cg.pw;
+            va[h] = ((uint32_t)(n * cg.H + p * cg.sh - cg.ph) * (uint32_t)cg.W + (uint32_t)iw0[h]) * (uint32_t)cg.C;
+            asm volatile("" : "+v"(ih0[h]), "+v"(iw0[h]));
+        } else {
+            va[h] = (uint32_t)(((size_t)m * K + 8 * lch) * 2);
+        }
+        asm volatile("" : "+v"(va[h]));
+    }
+#pragma unroll
+    for (int h = 0; h < NQB; ++h) {
+        const int q = NQB * lw + h;
         if constexpr (BT) {
-            vb[h] = (uint32_t)(((size_t)(n0 + row) * K + 8 * (p ^ (row & 7))) * 2);
+            vb[h] = (uint32_t)(((size_t)(n0 + 8 * q + lane / 8) * K + 8 * lch) * 2);
         } else {
             // k-row kr, 16-byte position pp: chunk pair (segment) pp / 2 holds segment (pp / 2) ^ f(kr)
             constexpr int CPR = BN / 8;  // 16-byte chunks per k-row
@@ -90,18 +149,64 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
             const int c = ((((pp >> 1) ^ sm_kswz<BN>(kr)) << 1) | (pp & 1));
             vb[h] = (uint32_t)(((size_t)kr * N + n0 + 8 * c) * 2);
         }
-        asm volatile("" : "+v"(va[h]), "+v"(vb[h]));
+        asm volatile("" : "+v"(vb[h]));
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
-    auto issue = [&](int kt) {
-        const uint32_t slot = lds0 + (uint32_t)(kt % STAGES) * (2 * TILE_BYTES);
-        const uint32_t sa = (uint32_t)kt * kSmBK * 2;
-        const uint32_t sb = BT ? sa : (uint32_t)kt * kSmBK * (uint32_t)N * 2;
-#pragma unroll
-        for (int h = 0; h < NQ; ++h) {
-            const uint32_t off = (uint32_t)(NQ * wave + h) * 1024;
-            lds_dma_buf_b128_u(ra, va[h], sa, slot + off);
-            lds_dma_buf_b128_u(rb, vb[h], sb, slot + TILE_BYTES + off);
+
+    // What one stage's loads share: scalar advances (kDense), or whether the
+    // lane's chunk is inside K and (kConv) the tap it belongs to. Stages past
+    // the last are issued too, so that the count of outstanding loads is the
+    // same every step; they read past the buffer's end and cost no traffic.
+    struct Src {
+        uint32_t sa, sb;
+        bool in;
+        int r, s;
+        uint32_t tap;
+    };
+    auto src_of = [&](int kt) {
+        Src x{};
+        x.sa = (uint32_t)kt * (kSmBK * 2);
+        x.sb = BT ? x.sa : (uint32_t)kt * kSmBK * (uint32_t)N * 2;
+        if constexpr (SRC == kDense) {
+            x.in = kt < KT;
+        } else {
+            const uint32_t k = (uint32_t)(kt * kSmBK + 8 * lch);
+            x.in = k < (uint32_t)K;
+            if constexpr (SRC == kConv) {
+                const uint32_t t = __umulhi(k, cg.rc);
+                const uint32_t c = k - t * (uint32_t)cg.C;
+                x.r = cg.rs ? (int)__umulhi(t, cg.rs) : (int)t;
+                x.s = (int)t - x.r * cg.S;
+                x.tap = (uint32_t)(x.r * cg.W + x.s) * (uint32_t)cg.C + c;
+            }
+        }
+        return x;
+    };
+    // load d (< NQA: A, else B) of a stage whose slot part starts at LDS byte `base`
+    auto dma = [&](int d, const Src& x, uint32_t base) {
+        i32x4 r = d < NQA ? ra : rb;
+        if constexpr (SRC == kDense) r.z = x.in ? r.z : 0;  // a stage past the last: an empty buffer
+        if (d < NQA) {
+            const int h = d;
+            const uint32_t lds = base + (uint32_t)(NQA * lw + h) * 1024;
+            if constexpr (SRC == kDense) {
+                lds_dma_buf_b128_u(r, va[h], x.sa, lds);
+            } else if constexpr (SRC == kTail) {
+                lds_dma_buf_b128_u(r, x.in ? va[h] + x.sa : kSmPastEnd, 0u, lds);
+            } else {
+                const bool ok = x.in & ((unsigned)(ih0[h] + x.r) < (unsigned)cg.H) &
+                                ((unsigned)(iw0[h] + x.s) < (unsigned)cg.W);
+                lds_dma_buf_b128_u(r, ok ? (va[h] + x.tap) * 2u : kSmPastEnd, 0u, lds);
+            }
+        } else {
+            const int h = d - NQA;
+            const uint32_t lds = base + A_BYTES + (uint32_t)(NQB * lw + h) * 1024;
+            // [K,N]: the whole offset goes through the range check (a scalar
+            // offset would not), which columns past N of the last k-row and
+            // k-rows past K need
+            if constexpr (!BT) lds_dma_buf_b128_u(r, vb[h] + x.sb, 0u, lds);
+            else if constexpr (SRC == kDense) lds_dma_buf_b128_u(r, vb[h], x.sb, lds);
+            else lds_dma_buf_b128_u(r, x.in ? vb[h] + x.sb : kSmPastEnd, 0u, lds);
         }
     };
 
@@ -117,165 +222,230 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     const int tr_k = 8 * lgrp + (lrow >> 2);
     const int tr_c = 4 * (lrow & 3);
 
-    // Every step issues one stage, clamped to the last (a duplicate into the
-    // slot the previous step freed), so each wave has STAGES - 2 stages of
-    // loads outstanding at the top of every step. Per step, the MFMAs go out
-    // in program order (sched_barrier) in groups of two, with the second
-    // k-step's fragment reads on the first groups and the DMAs of stage
-    // kt + STAGES - 1 on the following ones, so neither stalls the MFMAs.
-    constexpr int NF = FM + FN;            // fragment reads per k-step
-    constexpr int NG = FM * FN;            // groups of two MFMAs per step (2 k-steps)
-    // the second k-step's MFMAs start at group NG / 2: its fragment reads ride
-    // on the first NF groups when they fit before it, else they go out with
-    // the first k-step's reads (64 x 64 tiles: 4 reads, 2 groups)
-    constexpr bool PRE = NF > NG / 2;
-    constexpr int G_DMA = PRE ? 0 : (NF < NG - LOADS ? NF : NG - LOADS);
-    static_assert(G_DMA + LOADS <= NG && (PRE || NF <= NG / 2), "schedule");
+    // stage t (< NST) of this wave's share of a slot, and its first k stage
+    auto own = [&](int t) { return HALF ? 0 : kh * NST + t; };
+    auto issue_stage = [&](int st, int t, uint32_t slot_base, auto&& each) {
+        const Src x = src_of(st * KS + own(t));
+        each(x, slot_base + (uint32_t)own(t) * STAGE_BYTES);
+    };
+    const int steps = (KT + KS - 1) / KS;
+    // The prologue fills all slots but one; then every step issues one slot
+    // into the place the previous step freed, so each wave has SLOTS - 2 slots
+    // of its loads outstanding at the top of every step.
+#pragma unroll 1
+    for (int p = 0; p < SLOTS - 1; ++p)
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) issue(min(s, KT - 1));
-    for (int kt = 0; kt < KT; ++kt) {
-        wait_vmem_le<(STAGES - 2) * LOADS>();  // own loads of stage kt landed
-        __syncthreads();  // every wave's part of stage kt is in LDS; slot kt-1 is consumed
-        const int kn = min(kt + STAGES - 1, KT - 1);
-        const uint32_t nslot = lds0 + (uint32_t)((kt + STAGES - 1) % STAGES) * (2 * TILE_BYTES);
-        const uint32_t nsa = (uint32_t)kn * kSmBK * 2;
-        const uint32_t nsb = BT ? nsa : (uint32_t)kn * kSmBK * (uint32_t)N * 2;
-        const uint16_t* As = smem + (kt % STAGES) * TILE_BYTES;  // uint16_t units: 2 tiles per stage
-        const uint16_t* Bs = As + TILE_BYTES / 2;
-        u32x4 fa[2][FM], fb[2][FN];
-        auto rd = [&](int ks, int f) {
-            if (f < FM) {
-                const int r = wm * (BM / 2) + 16 * f + lrow;
-                fa[ks][f] = *reinterpret_cast<const u32x4*>(As + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
-            } else {
-                const int j = f - FM;
-                if constexpr (BT) {
-                    const int r = wn * (BN / 2) + 16 * j + lrow;
-                    fb[ks][j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
-                } else {
-                    const int seg = wn * (SEGS / 2) + j;  // the fragment's 16 columns
-                    const int k0 = 32 * ks + tr_k, k1 = k0 + 4;
-                    const u32x2 lo = lds_read_tr16(Bs + k0 * BN + 16 * (seg ^ sm_kswz<BN>(k0)) + tr_c);
-                    const u32x2 hi = lds_read_tr16(Bs + k1 * BN + 16 * (seg ^ sm_kswz<BN>(k1)) + tr_c);
-                    fb[ks][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        for (int t = 0; t < NST; ++t)
+            issue_stage(p, t, lds0 + (uint32_t)p * SLOT_BYTES, [&](const Src& x, uint32_t base) {
+#pragma unroll
+                for (int d = 0; d < LOADS; ++d) dma(d, x, base);
+            });
+    constexpr int KSTEPS = HALF ? 1 : 2;               // 32-k steps a wave multiplies per stage
+    constexpr int NM = FM * FN * KSTEPS;               // MFMAs per stage and wave
+    constexpr int GAP = NM / LOADS > 0 ? NM / LOADS : 1;  // MFMAs between two DMAs
+    int cur = 0, nxt = SLOTS - 1;  // slot of this step, slot that is issued now
+    for (int st = 0; st < steps; ++st) {
+        wait_vmem_le<(SLOTS - 2) * NST * LOADS>();  // own loads of this step's slot landed
+        __syncthreads();  // every wave's part of it is in LDS; the previous step's slot is consumed
+#pragma unroll
+        for (int t = 0; t < NST; ++t) {
+            const uint16_t* As = smem + (uint32_t)cur * (SLOT_BYTES / 2) + (uint32_t)own(t) * (STAGE_BYTES / 2);
+            const uint16_t* Bs = As + A_BYTES / 2;
+            u32x4 fa[KSTEPS][FM], fb[KSTEPS][FN];
+#pragma unroll
+            for (int u = 0; u < KSTEPS; ++u) {
+                const int ks = HALF ? kh : u;  // which 32 k of the stage
+#pragma unroll
+                for (int i = 0; i < FM; ++i) {
+                    const int r = wm * (BM / 2) + 16 * i + lrow;
+                    fa[u][i] = *reinterpret_cast<const u32x4*>(As + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
+                }
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    if constexpr (BT) {
+                        const int r = wn * (BN / 2) + 16 * j + lrow;
+                        fb[u][j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
+                    } else {
+                        const int seg = wn * (SEGS / 2) + j;  // the fragment's 16 columns
+                        const int k0 = 32 * ks + tr_k, k1 = k0 + 4;
+                        const u32x2 lo = lds_read_tr16(Bs + k0 * BN + 16 * (seg ^ sm_kswz<BN>(k0)) + tr_c);
+                        const u32x2 hi = lds_read_tr16(Bs + k1 * BN + 16 * (seg ^ sm_kswz<BN>(k1)) + tr_c);
+                        fb[u][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                    }
                 }
             }
-        };
-        auto dma = [&](int d) {  // d < NQ: A, else B
-            const int h = d % NQ;
-            const uint32_t off = (uint32_t)(NQ * wave + h) * 1024;
-            if (d < NQ) lds_dma_buf_b128_u(ra, va[h], nsa, nslot + off);
-            else lds_dma_buf_b128_u(rb, vb[h], nsb, nslot + TILE_BYTES + off);
-        };
+            issue_stage(st + SLOTS - 1, t, lds0 + (uint32_t)nxt * SLOT_BYTES, [&](const Src& x, uint32_t base) {
+                int d = 0;
 #pragma unroll
-        for (int f = 0; f < NF; ++f) rd(0, f);
-        if constexpr (PRE) {
+                for (int m = 0; m < NM; ++m) {
+                    const int u = m / (FM * FN), q = m % (FM * FN);
+                    acc[q / FN][q % FN] = mfma16x16x32(fb[u][q % FN], fa[u][q / FN], acc[q / FN][q % FN], T{});
+                    if (m % GAP == GAP - 1 && d < LOADS) dma(d++, x, base);
+                    if (GAP > 1) __builtin_amdgcn_sched_barrier(0);
+                }
 #pragma unroll
-            for (int f = 0; f < NF; ++f) rd(1, f);
+                for (; d < LOADS; ++d) dma(d, x, base);
+            });
         }
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int p = 2 * g + u;
-                const int ks = p / (FM * FN), q = p % (FM * FN);
-                acc[q / FN][q % FN] = mfma16x16x32(fb[ks][q % FN], fa[ks][q / FN], acc[q / FN][q % FN], T{});
-            }
-            if (!PRE && g < NF) rd(1, g);
-            if (g >= G_DMA && g < G_DMA + LOADS) dma(g - G_DMA);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        nxt = cur;
+        cur = cur + 1 == SLOTS ? 0 : cur + 1;
     }
-    wait_vmem_le<0>();  // the clamped duplicates have landed too
+    wait_vmem_le<0>();  // the loads past the last stage have landed too
+    __syncthreads();    // every wave is done with the ring; it takes the results
 
-    // lane's acc[i][j][e] is C[m0 + BM/2 wm + 16 i + lrow][n0 + BN/2 wn + 16 j + 4 lgrp + e]
-    const bool has_bias = (epi & 1) && bias != nullptr;
-    const bool relu = (epi & 2) != 0;
+    // Results as fp32 in LDS, BM/2 x BN/2 per quadrant, 16-byte chunk c of row
+    // r at c ^ (r % CH): acc[i][j] is row 16 i + lrow, columns 16 j + 4 lgrp .. +3.
+    // Group 1 hands over its sums, group 0 adds them to its own, and all eight
+    // waves write C, half a quadrant's rows each, CH lanes to a row segment.
+    f32x4* const res = reinterpret_cast<f32x4*>(smem) + quad * (BM / 2) * CH;
+    auto at = [&](int r, int c) { return r * CH + (c ^ (r & (CH - 1))); };
+    if (kh) {
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const int gn = n0 + wn * (BN / 2) + 16 * j + 4 * lgrp;
-        if (gn >= N) continue;  // N % 4 == 0: a lane's 4 columns are all in or all out
-        float bv[4];
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) bv[e] = has_bias ? bias[gn + e] : 0.f;
+            for (int j = 0; j < FN; ++j) res[at(16 * i + lrow, 4 * j + lgrp)] = acc[i][j];
+    }
+    __syncthreads();
+    if (!kh) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const int gm = m0 + wm * (BM / 2) + 16 * i + lrow;
-            if (gm >= M) continue;
-            uint16_t* cp = C + (size_t)gm * N + gn;
-            float v[4];
-            u32x2 old = u32x2{0u, 0u};
-            if (beta != 0.f) old = *reinterpret_cast<const u32x2*>(cp);
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = alpha * acc[i][j][e];
-                if (beta != 0.f) v[e] += beta * elem<T>::to_f32((uint16_t)(old[e >> 1] >> (16 * (e & 1))));
-                v[e] += bv[e];
-                if (relu) v[e] = v[e] > 0.f ? v[e] : 0.f;
+            for (int j = 0; j < FN; ++j) {
+                f32x4* p = &res[at(16 * i + lrow, 4 * j + lgrp)];
+                *p = acc[i][j] + *p;
             }
-            u32x2 packed;
-            packed[0] = (uint32_t)elem<T>::from_f32(v[0]) | ((uint32_t)elem<T>::from_f32(v[1]) << 16);
-            packed[1] = (uint32_t)elem<T>::from_f32(v[2]) | ((uint32_t)elem<T>::from_f32(v[3]) << 16);
-            *reinterpret_cast<u32x2*>(cp) = packed;
+    }
+    __syncthreads();
+    constexpr int RPI = kWave / CH;  // rows per pass of a wave
+    static_assert(BM / 4 % RPI == 0 || BM / 4 < RPI, "row passes");
+    const bool relu = (epi & 2) != 0;
+    const int c = lane % CH;
+    const int gn = n0 + wn * (BN / 2) + 4 * c;
+    f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
+    if ((epi & 1) && bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (gn + e < N) bv[e] = bias[gn + e];
+    }
+#pragma unroll 1
+    for (int r = kh * (BM / 4) + lane / CH; r < (kh + 1) * (BM / 4); r += RPI) {
+        const int gm = m0 + wm * (BM / 2) + r;
+        if (gm >= M || gn >= N) break;
+        f32x4 v = res[at(r, c)];
+        uint16_t* cp = C + (size_t)gm * N + gn;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = alpha * v[e];
+        if (beta != 0.f) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (gn + e < N) v[e] += beta * elem<T>::to_f32(cp[e]);
+        }
+        uint16_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float x = v[e] + bv[e];
+            if (relu) x = x > 0.f ? x : 0.f;
+            o[e] = elem<T>::from_f32(x);
+        }
+        if (vec_c) {  // N % 4 == 0: a lane's 4 columns are all in or all out
+            *reinterpret_cast<u32x2*>(cp) =
+                u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (gn + e < N) cp[e] = o[e];
         }
     }
 }
 
-}  // namespace pyc
-
-// tile: 64 or 128 (square tiles). Returns 1 when the shape is outside this
-// kernel's preconditions (N a multiple of 4, K of 64; A, B, C 16-byte
-// aligned; A and B below 4 GiB), 0 on launch, -2 on a launch error. Ragged M
-// and N: rows of A (and of [N,K] B) past the end are read as zeros through the
-// buffer descriptors, [K,N] B columns past N read neighbouring data, and only
-// the rows and columns of C inside M x N are written.
-extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int tile, int M, int N, int K, const void* A,
-                                         const void* B, void* C, float alpha, float beta, const float* bias,
-                                         int epi, void* stream) {
-    using namespace pyc;
-    if (tile != 64 && tile != 128) return 1;
-    if (M <= 0 || N <= 0 || K <= 0 || N % 4 || K % kSmBK) return 1;
-    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
-    if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) return 1;
-    const int tiles_n = (N + tile - 1) / tile;
-    const long tiles = (long)((M + tile - 1) / tile) * tiles_n;
+template <typename T, bool BT, int SRC>
+static int launch_small(int bm, int bn, int M, int N, int K, const void* A, const void* B, void* C, float alpha,
+                        float beta, const float* bias, int epi, hipStream_t s, const SmConv& cg) {
+    const int tiles_n = (N + bn - 1) / bn;
+    const long tiles = (long)((M + bm - 1) / bm) * tiles_n;
     if (tiles > 0x7FFFFFFFL) return 1;
-    hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)tiles), block(4 * kWave);
+    const dim3 grid((unsigned)tiles), block(8 * kWave);
     const uint16_t* a = (const uint16_t*)A;
     const uint16_t* b = (const uint16_t*)B;
     uint16_t* c = (uint16_t*)C;
-#define PYC_SMALL(TY, BT)                                                                                       \
-    do {                                                                                                        \
-        if (tile == 64)                                                                                         \
-            hipLaunchKernelGGL((gemm_small_kernel<TY, BT, 64>), grid, block, 0, s, a, b, c, M, N, K, alpha, beta, \
-                               bias, epi, tiles_n);                                                             \
-        else                                                                                                    \
-            hipLaunchKernelGGL((gemm_small_kernel<TY, BT, 128>), grid, block, 0, s, a, b, c, M, N, K, alpha,    \
-                               beta, bias, epi, tiles_n);                                                       \
-    } while (0)
-    if (is_bf16) {
-        if (b_trans) PYC_SMALL(bf16_t, true);
-        else PYC_SMALL(bf16_t, false);
-    } else {
-        if (b_trans) PYC_SMALL(f16_t, true);
-        else PYC_SMALL(f16_t, false);
-    }
+    const int vec_c = N % 4 == 0 && ((uintptr_t)C & 7) == 0;
+#define PYC_SMALL(BM, BN, KS)                                                                                  \
+    hipLaunchKernelGGL((gemm_small_kernel<T, BT, BM, BN, KS, SRC>), grid, block, 0, s, a, b, c, M, N, K, alpha, \
+                       beta, bias, epi, tiles_n, vec_c, cg)
+    if (bm == 32 && bn == 32) PYC_SMALL(32, 32, 4);
+    else if (bm == 64 && bn == 64) PYC_SMALL(64, 64, 2);
+    else if (bm == 128 && bn == 128) PYC_SMALL(128, 128, 1);
+    else if (bm == 128 && bn == 256) PYC_SMALL(128, 256, 1);
+    else return 1;
 #undef PYC_SMALL
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// Registry figures: the 128 KB ring allows one 4-wave workgroup per CU.
+}  // namespace pyc
+
+// bm x bn: one of the tiles above. Returns 1 when the shape is outside this
+// kernel's preconditions (K a multiple of 8 and, for [K,N] B, N of 4; A and B
+// 16-byte aligned and below 4 GiB), 0 on launch, -2 on a launch error. Ragged M
+// and N: rows of A (and of [N,K] B) past the end are read as zeros through the
+// buffer descriptors, [K,N] B columns past N read neighbouring data, and only
+// the rows and columns of C inside M x N are written.
+extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
+                                         const void* B, void* C, float alpha, float beta, const float* bias,
+                                         int epi, void* stream) {
+    using namespace pyc;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 8 || (!b_trans && N % 4)) return 1;
+    const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
+    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
+    if ((K % kSmBK || !b_trans) && ((size_t)M * K * 2 > kSmPastEnd || (size_t)N * kpad * 2 > kSmPastEnd)) return 1;
+    if (((uintptr_t)A | (uintptr_t)B) & 15) return 1;
+    hipStream_t s = (hipStream_t)stream;
+    const SmConv cg{};
+    const bool tail = K % kSmBK != 0;
+#define PYC_GO(TY, BT)                                                                                              \
+    (tail ? launch_small<TY, BT, kTail>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                    \
+          : launch_small<TY, BT, kDense>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg))
+    if (is_bf16) return b_trans ? PYC_GO(bf16_t, true) : PYC_GO(bf16_t, false);
+    return b_trans ? PYC_GO(f16_t, true) : PYC_GO(f16_t, false);
+#undef PYC_GO
+}
+
+// NHWC convolution on the same tiles (bm output pixels x bn output channels).
+// Returns 1 outside its preconditions (C % 8 == 0, x and w 16-byte aligned and
+// below 4 GiB, reciprocals exact: R*S*C * C < 2^32), 0 on launch, -2 on a
+// launch error.
+extern "C" int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg, int H, int W, int C, int Kout,
+                                           int R, int S, int ph, int pw, int sh, int sw, const void* x,
+                                           const void* w, const float* bias, int relu, void* y, void* stream) {
+    using namespace pyc;
+    const long long P = (H + 2LL * ph - R) / sh + 1, Q = (W + 2LL * pw - S) / sw + 1;
+    const long long M = (long long)Nimg * P * Q, Kg = (long long)R * S * C;
+    const unsigned long long lim = kSmPastEnd;
+    if (C % 8 || P <= 0 || Q <= 0 || M > 0x7FFFFF00LL || Kg > 0x7FFFFF00LL) return 1;
+    if ((unsigned long long)Kg * C >= (1ull << 32)) return 1;
+    if ((unsigned long long)Nimg * H * W * C * 2 > lim || (unsigned long long)Kout * Kg * 2 > lim) return 1;
+    if (H >= (1 << 28) || W >= (1 << 28) || ph >= (1 << 28) || pw >= (1 << 28)) return 1;
+    if (((uintptr_t)x | (uintptr_t)w) & 15) return 1;
+    const SmConv cg{H, W, C, S, (int)P, (int)Q, ph, pw, sh, sw, (uint32_t)(((1ull << 32) + C - 1) / C),
+                    S == 1 ? 0u : (uint32_t)(((1ull << 32) + S - 1) / S),
+                    (uint32_t)((size_t)Nimg * H * W * C * 2)};
+    const int epi = (bias ? 1 : 0) | (relu ? 2 : 0);
+    hipStream_t st = (hipStream_t)stream;
+    if (is_bf16)
+        return launch_small<bf16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, st, cg);
+    return launch_small<f16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, st, cg);
+}
+
+// Registry figures: the ring allows one 8-wave workgroup per CU.
 extern "C" int pyc_hip_kinfo_small(int tile, int b_trans, int is_bf16, pyc_hip_kinfo* out) {
     using namespace pyc;
     if (!out || (tile != 64 && tile != 128)) return -1;
-    out->threads = 256;
-    out->waves_per_simd = 1;
-    out->lds_bytes = kSmRingBytes;
+    out->threads = 512;
+    out->waves_per_simd = 2;
+    out->lds_bytes = sm_lds_bytes(tile, tile, tile == 64 ? 2 : 1);
     out->name = tile == 64 ? "gemm_small_kernel<64>" : "gemm_small_kernel<128>";
 #define PYC_KI(TY, BT) \
-    out->fn = tile == 64 ? reinterpret_cast<const void*>(&gemm_small_kernel<TY, BT, 64>) \
-                         : reinterpret_cast<const void*>(&gemm_small_kernel<TY, BT, 128>)
+    out->fn = tile == 64 ? reinterpret_cast<const void*>(&gemm_small_kernel<TY, BT, 64, 64, 2, kDense>) \
+                         : reinterpret_cast<const void*>(&gemm_small_kernel<TY, BT, 128, 128, 1, kDense>)
     if (is_bf16) {
         if (b_trans) PYC_KI(bf16_t, true); else PYC_KI(bf16_t, false);
     } else {

@@ -183,3 +183,39 @@ def test_conv_unaligned_bias_takes_general_kernel(gpu):
     _check(oracle.bf16_to_f32(host_bits16(Y1[:1])), ref, 9 * C)
     d = (Y1.float() - Y2.float()).abs().max().item()
     assert d <= 2e-2 * Y2.float().abs().max().item()
+
+
+@pytest.mark.parametrize("bm,bn", [(32, 32), (64, 64), (128, 128), (128, 256)])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("N,H,W,C,K,R,S,pad,stride", [
+    (2, 9, 7, 8, 33, 3, 3, (1, 1), (1, 1)),     # 8 channels: a stage spans 8 taps, one odd output channel
+    (3, 13, 11, 24, 260, 3, 2, (1, 0), (2, 1)),  # taps that begin inside a stage, an even filter, a k tail
+    (1, 12, 12, 192, 64, 1, 1, (0, 0), (2, 2)),  # 1x1: the reciprocal of S = 1
+    (5, 8, 9, 64, 130, 5, 3, (2, 1), (1, 1)),    # more padding than a 3x3 has
+])
+def test_conv_lds_tiles(gpu, bm, bn, dt, N, H, W, C, K, R, S, pad, stride):
+    """The implicit GEMM on each LDS-DMA tile: ragged pixels and channels,
+    padding, strides, against the oracle."""
+    import ctypes
+    torch = gpu
+    r = np.random.default_rng(N + H + C + K)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float16
+    X = torch.from_numpy(r.uniform(0, 1, (N, H, W, C)).astype(np.float32)).cuda().to(tdt)
+    Wd = torch.from_numpy(r.normal(0, np.sqrt(2.0 / (R * S * C)), (K, R, S, C)).astype(np.float32)).cuda().to(tdt)
+    bias = r.normal(0, 0.1, K).astype(np.float32)
+    P = (H + 2 * pad[0] - R) // stride[0] + 1
+    Q = (W + 2 * pad[1] - S) // stride[1] + 1
+    Bd = dev_f32(torch, bias)
+    Y = torch.full((N * P * Q * K + 512,), 7.0, dtype=tdt, device="cuda")
+    launch = pyc_amd.lib().pyc_hip_conv2d_small_launch
+    launch.argtypes = [ctypes.c_int] * 14 + [ctypes.c_void_p] * 3 + [ctypes.c_int] + [ctypes.c_void_p] * 2
+    assert launch(int(dt == "bf16"), bm, bn, N, H, W, C, K, R, S, pad[0], pad[1], stride[0], stride[1], X.data_ptr(),
+                  Wd.data_ptr(), Bd.data_ptr(), 1, Y.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    assert bool((Y[N * P * Q * K:] == 7.0).all())
+    ref = oracle.conv2d_nhwc_f32(X.float().cpu().numpy(), Wd.float().cpu().numpy(), bias, pad, stride, relu=True)
+    got = Y[:N * P * Q * K].float().cpu().numpy().reshape(ref.shape)
+    # one rounding of the result (2^-8 or 2^-11 relative) plus fp32 summation order
+    eps = 2.0 ** (-8 if dt == "bf16" else -11)
+    bad = ~(np.abs(got - ref) <= eps * np.abs(ref) + 4e-6 * np.sqrt(R * S * C) * np.abs(ref).max())
+    assert not bad.any(), f"{bad.sum()} off, first at {np.argwhere(bad)[0]}"

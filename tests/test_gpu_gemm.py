@@ -7,6 +7,8 @@ Tolerances:
     (2^-8 relative for bf16) plus a K-dependent accumulation-order term, which
     a dropped k-tile or a transposed operand would break.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -420,3 +422,69 @@ def test_ragged_persistent_gemm(gpu, m, n, k, epi, layout, dtype):
     bound = 2.0 ** (-8 if dtype == "bf16" else -11) * np.abs(ref) + 4e-6 * np.sqrt(k) * np.abs(ref).max()
     bad = np.abs(got - ref) > bound
     assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
+
+
+LDS_TILES = [(32, 32), (64, 64), (128, 128), (128, 256)]
+
+
+@pytest.mark.parametrize("bm,bn", LDS_TILES)
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("k,beta,epi", [(8, 0.0, 0),        # one chunk of one stage
+                                        (64, 0.5, 3),       # one whole stage, every epilogue term
+                                        (136, 0.0, 1),      # a tail of one chunk in the third stage
+                                        (1416, 0.0, 2)])    # 23 stages: every ring wraps
+def test_lds_tiles_ragged(gpu, bm, bn, layout, dtype, k, beta, epi):
+    """Each LDS-DMA tile by itself: one row and four columns into a second tile
+    each way ([N,K] B: one column, so C's rows are not 8-byte aligned), k tails
+    that are chunks of 8, infinities in the row after each k tail (which must
+    stay in their own row and column), nothing written past C."""
+    torch = gpu
+    bt = layout == "nt"
+    m, n = bm + 1, bn + (1 if bt else 4)
+    r = np.random.default_rng(bm + bn + k)
+    t = torch.bfloat16 if dtype == "bf16" else torch.float16
+    A = torch.from_numpy((r.standard_normal((m, k)) / np.sqrt(k)).astype(np.float32)).cuda().to(t)
+    B = torch.from_numpy(r.standard_normal((n, k) if bt else (k, n)).astype(np.float32)).cuda().to(t)
+    bias = torch.from_numpy(r.standard_normal(n).astype(np.float32)).cuda()
+    A[1, 0] = float("inf")
+    C0 = torch.from_numpy(r.standard_normal(m * n + 512).astype(np.float32)).cuda().to(t)
+    Cd = C0.clone()
+    L = pyc_amd.lib()
+    launch = L.pyc_hip_gemm_small_launch
+    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p, C.c_int, C.c_void_p]
+    assert launch(int(dtype == "bf16"), int(bt), bm, bn, m, n, k, A.data_ptr(), B.data_ptr(), Cd.data_ptr(), 0.75,
+                  beta, bias.data_ptr(), epi, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(Cd[m * n:], C0[m * n:])
+    a, b = A.float().cpu().numpy(), B.float().cpu().numpy()
+    a[1] = 0
+    ref = 0.75 * (a @ (b.T if bt else b)) + beta * C0[:m * n].float().cpu().numpy().reshape(m, n)
+    if epi & 1:
+        ref = ref + bias.cpu().numpy()
+    if epi & 2:
+        ref = np.maximum(ref, 0.0)
+    got = Cd[:m * n].float().cpu().numpy().reshape(m, n)
+    keep = np.arange(m) != 1
+    # one rounding of the result (2^-8 or 2^-11 relative) plus fp32 summation order
+    bound = 2.0 ** (-8 if dtype == "bf16" else -11) * np.abs(ref) + 4e-6 * np.sqrt(k) * np.abs(ref).max()
+    bad = ~(np.abs(got - ref) <= bound) & keep[:, None]
+    assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
+
+
+def test_lds_tile_choice_covers_shapes(gpu):
+    """The shape-chosen symbols over sizes on both sides of every tile choice
+    (and K and N that only the register-staged tiles take), against fp32."""
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(4)
+    for m, n, k in [(1, 8, 8), (60, 500, 4096), (128, 1024, 1000), (512, 4096, 512), (900, 900, 904), (2047, 2044, 64),
+                    (1023, 8192, 128), (3000, 2000, 256), (2304, 5000, 192), (77, 130, 33), (200, 301, 250)]:
+        for bt in (True, False):
+            A = (torch.randn((m, k), generator=g, device="cuda") / np.sqrt(k)).bfloat16()
+            B = torch.randn((n, k) if bt else (k, n), generator=g, device="cuda").bfloat16()
+            Cd = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            pyc_amd.gemm("hip_gemm_bf16_nt" if bt else "hip_gemm_bf16_nn", A, B, Cd, m, n, k)
+            ref = A.float() @ (B.float().t() if bt else B.float())
+            bound = 2.0 ** -8 * ref.abs() + 4e-6 * np.sqrt(k) * ref.abs().max()
+            bad = ~((Cd.float() - ref).abs() <= bound)
+            assert not bool(bad.any()), (m, n, k, bt, int(bad.sum()))
