@@ -601,6 +601,277 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp,
     wait_vmem_le<0>();  // no LDS-DMA write may still be pending
 }
 
+// ---------------------------------------------------------------------------
+// Few heads or short sequences: the kernel above gives a CU 256 queries of one
+// head, so 32 heads of 1000 queries leave half the chip idle and every
+// workgroup walks all keys by itself. Here a workgroup owns 32 QW queries, and
+// its 8 waves are QW query groups x KW = 8 / QW key groups: a step covers 32 KW
+// keys, 32 for each wave, and the KW partial results (reference m, sum l and
+// O, each against the wave's own m) are joined through LDS at the end. One
+// workgroup per (head, query block); with a causal mask the long blocks start
+// first.
+// K and V halves of a step (32 KW rows) stream through one LDS ring by
+// LDS-DMA in the order K0 V0 K1 V1 ...; step i has one barrier, after which
+// V(i-1) and K(i) are visible and the two halves consumed in the step before
+// are refilled: O += V(i-1)^T P(i-1)^T, S(i) = K(i) Q^T, softmax of S(i). The
+// other wave of the SIMD (at head dim 64 the other three: two workgroups fit a
+// CU) fills the softmax with its MFMAs. Halves past the last are issued from an
+// empty buffer, so the count of outstanding loads is the same every step.
+// A query's softmax reference m is the maximum of the first block with an
+// unmasked key (m = -inf, l = 0 until then); later blocks exponentiate against
+// it without a maximum, and only when a lane's sum passes 2^14 is m raised where
+// the block's maximum is more than 2^8 above it.
+template <int D, int QW> struct AttnSmall {
+    static constexpr int KW = 8 / QW;
+    static constexpr int ROWS = 32 * KW;                  // keys of a step
+    static constexpr uint32_t HALF = ROWS * D * 2;        // LDS bytes of the step's K (or V)
+    // D = 64: half of the LDS, for two workgroups per CU
+    static constexpr int SLOTS_FIT = (int)((D == 64 ? 80 : 160) * 1024 / HALF);
+    static constexpr int SLOTS = SLOTS_FIT < 9 ? SLOTS_FIT : 9;
+    static constexpr size_t RING = (size_t)SLOTS * HALF;
+    static constexpr size_t JOIN = (size_t)8 * 32 * D * 4;  // the partial O, after the last step
+    static constexpr size_t LDS = RING;
+    static_assert(JOIN + 8 * 32 * 8 <= RING, "partial O, m and l in the ring's LDS");
+};
+
+template <typename T, int D, int QW>
+__global__ void __launch_bounds__(512, D == 64 ? 4 : 2)
+attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+                  uint16_t* __restrict__ O, int BH, int S, int causal, float scale_log2) {
+    using Cfg = AttnSmall<D, QW>;
+    constexpr int KW = Cfg::KW, ROWS = Cfg::ROWS, SLOTS = Cfg::SLOTS;
+    constexpr int CH = D / 8;                         // 16-byte chunks per row
+    constexpr int DT = D / 32, KK = D / 16;
+    constexpr int RPD = kWave / CH;                   // rows one wave-load fills
+    constexpr int L = ROWS / RPD / 8;                 // wave-loads per half and wave
+    constexpr float kRaise = 8.0f;
+    static_assert(L * RPD * 8 == ROWS && SLOTS >= 5, "ring");
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[Cfg::LDS / 2];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qg = wave % QW, kg = wave / QW;
+    const int l32 = lane & 31, h = lane >> 5;
+    const int xaddr = (lane ^ 32) * 4;
+
+    // head and query block: an XCD walks the blocks of its own heads (their
+    // K/V in its L2), the longest (last) blocks of a causal head first
+    const int nqb = (S + 32 * QW - 1) / (32 * QW);
+    int bh, qb;
+    if ((BH & 7) == 0) {
+        const int x = blockIdx.x & 7, i = blockIdx.x >> 3, per = BH >> 3;
+        bh = x * per + i % per;
+        qb = nqb - 1 - i / per;
+    } else {
+        bh = blockIdx.x % BH;
+        qb = nqb - 1 - blockIdx.x / BH;
+    }
+    const int q0 = qb * 32 * QW + qg * 32;            // this wave's first query
+    const int qi = q0 + l32;                          // this lane's query
+    const int kend = causal ? min((qb + 1) * 32 * QW, S) : S;
+    const int n = (kend + ROWS - 1) / ROWS;           // steps
+    const int k_last = causal ? min(q0 + 31, S - 1) : S - 1;  // last key any query of this wave sees
+    const size_t base = (size_t)bh * S * D;
+
+    // Q fragments (B operand of S^T = K Q^T); queries past S load row S-1 and are never stored
+    u32x4 qf[KK];
+    {
+        const uint16_t* src = Q + base + (size_t)min(qi, S - 1) * D + h * 8;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) qf[kk] = *reinterpret_cast<const u32x4*>(src + kk * 16);
+    }
+
+    const uint32_t head_bytes = (uint32_t)((size_t)S * D * 2);
+    const i32x4 krs = make_buf_rsrc(Kp + base, head_bytes), vrs = make_buf_rsrc(Vp + base, head_bytes);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    // wave-load j of a half fills rows (8 j + wave) RPD ..; the swizzles see
+    // only row bits that j does not change
+    const int r0 = wave * RPD + lane / CH;
+    uint32_t ko[L], vo[L];
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+        const int row = j * 8 * RPD + r0;
+        ko[j] = (uint32_t)((row * CH + k_swz<CH>(row, lane % CH)) * 16);
+        vo[j] = (uint32_t)((row * CH + v_swz<CH>(row, lane % CH)) * 16);
+    }
+    // half x = 2 i (K of step i) or 2 i + 1 (V of step i) into ring slot `slot`
+    auto issue = [&](int x, int slot) {
+        const bool is_v = x & 1;
+        i32x4 rs = is_v ? vrs : krs;
+        rs.z = (x >> 1) < n ? rs.z : 0;
+        const uint32_t adv = (uint32_t)(x >> 1) * Cfg::HALF;  // whole offset in the lane: range-checked
+        const uint32_t lb = lds0 + (uint32_t)slot * Cfg::HALF + (uint32_t)wave * 1024u;
+#pragma unroll
+        for (int j = 0; j < L; ++j) lds_dma_buf_b128_u(rs, (is_v ? vo[j] : ko[j]) + adv, 0u, lb + j * 8192u);
+    };
+
+    const int gl = lane & 15;
+    const int vcol = 16 * ((lane >> 4) & 1) + 4 * (gl & 3);
+    const int vrow = 4 * h + (gl >> 2);
+    int v_off[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+        const int col = t * 32 + vcol;
+        v_off[t] = (kg * 32 + vrow) * D + v_swz<CH>(vrow, col / 8) * 8 + col % 8;
+    }
+    int k_off[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) k_off[kk] = (kg * 32 + l32) * D + k_swz<CH>(l32, kk * 2 + h) * 8;
+
+    f32x16 acc[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    u32x4 pf[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
+
+#pragma unroll 1
+    for (int x = 0; x < SLOTS - 3; ++x) issue(x, x);
+    // the compiler's wait for the Q loads lands here, once, instead of in every
+    // step (where it would drain the ring, whose loads it does not see)
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
+    int sk = 0;             // ring slot of K(i) (V(i) in the next one)
+    auto next = [&](int s) { return s + 1 == SLOTS ? 0 : s + 1; };
+    int sv = -1;            // ring slot of V(i-1)
+    int sf = SLOTS - 3;     // ring slot the next half goes into
+#pragma unroll 1
+    for (int i = 0; i <= n; ++i) {
+        // own loads up to K(i) landed: SLOTS - 3 + 2 i halves were issued, 2 i + 1 are needed
+        wait_vmem_le<(SLOTS - 4) * L>();
+        // every wave's part of V(i-1) and K(i) is in LDS; V(i-2) and K(i-1),
+        // halves 2 i - 3 and 2 i - 2, are consumed and their slots refilled
+        __syncthreads();
+        issue(2 * i + SLOTS - 3, sf);
+        sf = next(sf);
+        issue(2 * i + SLOTS - 2, sf);
+        sf = next(sf);
+        const int key0 = i * ROWS + kg * 32;
+        if (i > 0 && key0 - ROWS <= k_last) {         // wave-uniform: some of the keys of step i-1 count
+            const uint16_t* vs = smem + (uint32_t)sv * (Cfg::HALF / 2);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int t = 0; t < DT; ++t) {
+                    const u32x2 a0 = lds_read_tr16(vs + v_off[t] + ks * 16 * D);
+                    const u32x2 a1 = lds_read_tr16(vs + v_off[t] + (ks * 16 + 8) * D);
+                    acc[t] = mfma32x32x16(u32x4{a0[0], a0[1], a1[0], a1[1]}, pf[ks], acc[t], T{});
+                }
+        }
+        if (i < n && key0 <= k_last) {
+            const uint16_t* ks = smem + (uint32_t)sk * (Cfg::HALF / 2);
+            f32x16 sc;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk)
+                sc = mfma32x32x16(*reinterpret_cast<const u32x4*>(ks + k_off[kk]), qf[kk], sc, T{});
+            // exponents against m (0 while every key so far was masked); lane
+            // holds keys key0 + 8 (r / 4) + 4 h + r % 4 of query qi
+            const bool fresh = m_run == -INFINITY;
+            const float mref = fresh ? 0.f : m_run;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = fmaf(sc[r], scale_log2, -mref);
+            if ((causal && key0 + 31 > q0) || key0 + 32 > S) {
+                const int thr = (causal ? min(qi, S - 1) : S - 1) - key0 - 4 * h;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float x = 8 * (r >> 2) + (r & 3) > thr ? -INFINITY : sc[r];
+                    asm volatile("" : "+v"(x));  // keeps the masking inside this branch
+                    sc[r] = x;
+                }
+            }
+            // raises m to the block's maximum where that is far above it, or
+            // where m is not set yet and the block has an unmasked key
+            auto raise = [&](bool unset) {
+                float mb = vmax(sc[0], sc[1]);
+#pragma unroll
+                for (int r = 2; r < 16; r += 2) mb = vmax(vmax(mb, sc[r]), sc[r + 1]);
+                mb = vmax(mb, other_half(mb, xaddr));
+                const bool up = unset ? mb > -INFINITY : mb > kRaise;
+                const float shift = up ? mb : 0.f;
+                const float alpha = unset ? 0.f : __builtin_amdgcn_exp2f(-shift);
+                m_run = up ? mref + mb : m_run;
+                l_run *= alpha;
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] -= shift;
+            };
+            auto exponentiate = [&]() {
+                float ls[2] = {0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r < 16; r += 2) {
+                    const float p0 = __builtin_amdgcn_exp2f(sc[r]);
+                    const float p1 = __builtin_amdgcn_exp2f(sc[r + 1]);
+                    pf[r >> 3][(r & 7) >> 1] = pack2(p0, p1, T{});
+                    ls[0] += p0;
+                    ls[1] += p1;
+                }
+                return ls[0] + ls[1];
+            };
+            const bool any_fresh = __any(fresh);
+            if (any_fresh) raise(fresh);
+            float lsum = exponentiate();
+            if (!any_fresh && __any(!(lsum <= kAttnFastSumMax))) {
+                raise(false);
+                lsum = exponentiate();
+            }
+            l_run += lsum;
+        }
+        sv = next(sk);
+        sk = next(sv);
+    }
+    wait_vmem_le<0>();
+    __syncthreads();        // the ring is free; it takes (m, l) of each wave's queries and the partial O
+    float2(*const s_ml)[32] = reinterpret_cast<float2(*)[32]>(smem + Cfg::JOIN / 2);
+    const float l_wave = l_run + other_half(l_run, xaddr);
+    if (h == 0) s_ml[wave][l32] = float2{m_run, l_wave};
+    __syncthreads();
+
+    // Join the KW key groups of a query: factor exp2(m_kg - max) / sum
+    float mmax = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < KW; ++g) mmax = fmaxf(mmax, s_ml[g * QW + qg][l32].x);
+    const float mz = mmax == -INFINITY ? 0.f : mmax;
+    float lsum = 0.f;
+#pragma unroll
+    for (int g = 0; g < KW; ++g) {
+        const float2 ml = s_ml[g * QW + qg][l32];
+        lsum += ml.y * __builtin_amdgcn_exp2f(ml.x - mz);
+    }
+    // m and l of a query with a NaN score are NaN in some group; the sum carries it
+    const float f = __builtin_amdgcn_exp2f(m_run - mz) * (lsum > 0.f || lsum != lsum ? 1.f / lsum : 0.f);
+    // partial O of wave w: 32 rows (queries) of D floats, 16-byte chunk c of row q at c ^ (q & 15)
+    f32x4* part = reinterpret_cast<f32x4*>(smem);
+    constexpr int CW = D / 4;  // chunks per row
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 v = f32x4{acc[t][4 * g] * f, acc[t][4 * g + 1] * f, acc[t][4 * g + 2] * f, acc[t][4 * g + 3] * f};
+            part[(wave * 32 + l32) * CW + ((t * 8 + 2 * g + h) ^ (l32 & 15))] = v;
+        }
+    __syncthreads();
+    // thread: chunk c of rows tid / CW, + 512 / CW, ...
+    const int c = tid % CW;
+    uint16_t* ob = O + base;
+#pragma unroll 1
+    for (int r = tid / CW; r < 32 * QW; r += 512 / CW) {
+        const int q = qb * 32 * QW + r;
+        if (q >= S) break;
+        const f32x4* src = part + r * CW + (c ^ (r & 15));
+        f32x4 v = src[0];
+#pragma unroll
+        for (int g = 1; g < KW; ++g) v += src[(size_t)g * QW * 32 * CW];
+        *reinterpret_cast<u32x2*>(ob + (size_t)q * D + c * 4) = u32x2{pack2(v[0], v[1], T{}), pack2(v[2], v[3], T{})};
+    }
+}
+
 static int attn_cu_count() {
     static int n = 0;
     if (n == 0) {
@@ -614,8 +885,57 @@ static int attn_cu_count() {
     return n;
 }
 
+template <typename T, int D, int QW>
+static hipError_t launch_attn_small(int BH, int S, int causal, const void* q, const void* k, const void* v, void* o,
+                                    float scale_log2, hipStream_t s) {
+    const int nqb = (S + 32 * QW - 1) / (32 * QW);
+    hipLaunchKernelGGL((attn_small_kernel<T, D, QW>), dim3(BH * nqb), dim3(512), 0, s, (const uint16_t*)q,
+                       (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, BH, S, causal, scale_log2);
+    return hipGetLastError();
+}
+
+// Estimated microseconds of each form, from measurements on the MI355X (warm, back
+// to back; [B,H,S,D], persistent / QW = 2 / QW = 4): [2,16,1000,64] 22.8 / 17.1 /
+// 16.7, [1,8,1917,128] causal 57.5 / 24.2 / 37, [1,8,1917,64] causal 44 / 15.8 /
+// 25, [4,16,954,64] causal 29.6 / 21 / 18.6, [3,32,473,128] 21.5 / 32 / 29,
+// [8,32,300,128] causal 29.4 / 42 / 35, [8,32,2048,64] causal 190 / 312 / 207,
+// [1,12,64,64] 5.8 / 4.9 / 4.7. The persistent form takes a fixed part, then
+// one time per 64-key block of its longest workgroup; the others one per step
+// of the longest workgroup or of the average CU, and a start and end per round
+// of workgroups.
+static double attn_cost_persist(int BH, int S, int D, int causal) {
+    const int nqb = (S + 255) / 256;
+    const bool pair = causal && nqb > 1;
+    const long units = (long)BH * (pair ? (nqb + 1) / 2 : nqb);
+    const double rounds = (double)((units + 255) / 256), busy = units < 256 ? (double)units / 256.0 : 1.0;
+    // a pair's blocks: its first q-block (ragged) and q-block 0, or any other pair's 4 (nqb + 1)
+    const double top = (double)((S + 63) / 64), rest = nqb >= 4 ? 4.0 * (nqb + 1) : nqb == 3 ? 8.0 : 0.0;
+    const double blocks = !pair ? top : top + 4.0 > rest ? top + 4.0 : rest;
+    const double block = D == 128 ? 1.45 + 0.65 * busy : 1.1 + 0.2 * busy;
+    return 4.5 + rounds * blocks * block + (pair ? 3.0 : 0.0) * rounds;
+}
+
+static double attn_cost_small(int BH, int S, int D, int causal, int qw) {
+    const int bq = 32 * qw, rows = 256 / qw, nqb = (S + bq - 1) / bq;
+    const double wgs = (double)BH * nqb, n = (double)((S + rows - 1) / rows);
+    const double step = D == 128 ? (qw == 2 ? 1.28 : 1.1) : (qw == 2 ? 0.77 : 0.74);
+    const double at_once = D == 128 ? 256.0 : 512.0;
+    const double rounds = (double)(long)((wgs + at_once - 1.0) / at_once);
+    double steps;
+    if (causal) {
+        // block q of nqb walks (q + 1) bq keys; the long ones start first
+        const double mean = 0.5 * ((double)bq / rows) * (nqb + 1) + 0.5 * (1.0 - 1.0 / qw);
+        const double avg = wgs * (mean < n ? mean : n) / 256.0;
+        steps = n > avg ? n : avg;
+    } else {
+        steps = rounds * n * (D == 64 && wgs > 256.0 ? 2.0 : 1.0);
+    }
+    return (D == 128 ? 0.0 : 2.5) + (D == 128 ? (qw == 2 ? 4.5 : 5.0) : 2.0) * rounds + steps * step;
+}
+
+// form: 0 = the cheapest by estimate, 1 = persistent, 2 / 4 = small with that QW
 template <typename T, int D>
-static hipError_t launch_attn(int B, int H, int S, int causal, const void* q, const void* k,
+static hipError_t launch_attn(int form, int B, int H, int S, int causal, const void* q, const void* k,
                               const void* v, void* o, float scale, hipStream_t s) {
     const int BH = B * H;
     const float scale_log2 = scale * 1.4426950408889634f;
@@ -623,6 +943,13 @@ static hipError_t launch_attn(int B, int H, int S, int causal, const void* q, co
     const uint16_t* kk = (const uint16_t*)k;
     const uint16_t* vv = (const uint16_t*)v;
     uint16_t* oo = (uint16_t*)o;
+    if (form == 0) {
+        const double c1 = attn_cost_persist(BH, S, D, causal), c2 = attn_cost_small(BH, S, D, causal, 2),
+                     c4 = attn_cost_small(BH, S, D, causal, 4);
+        form = c1 <= c2 && c1 <= c4 ? 1 : c2 <= c4 ? 2 : 4;
+    }
+    if (form == 2) return launch_attn_small<T, D, 2>(BH, S, causal, q, k, v, o, scale_log2, s);
+    if (form == 4) return launch_attn_small<T, D, 4>(BH, S, causal, q, k, v, o, scale_log2, s);
     const int bq = kAttnWaves * 32;
     const int nqb = (S + bq - 1) / bq;
     const int units = (causal && nqb > 1) ? (nqb + 1) / 2 : nqb;
@@ -640,22 +967,30 @@ static hipError_t launch_attn(int B, int H, int S, int causal, const void* q, co
 
 }  // namespace pyc
 
-extern "C" int pyc_hip_attention_launch(int is_bf16, int B, int H, int S, int D, int causal,
-                                        const void* Q, const void* K, const void* V, void* O,
-                                        float scale, void* stream) {
+// form: see launch_attn; -1 for an unknown form or head dim
+extern "C" int pyc_hip_attention_launch_form(int form, int is_bf16, int B, int H, int S, int D, int causal,
+                                             const void* Q, const void* K, const void* V, void* O, float scale,
+                                             void* stream) {
     using namespace pyc;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
+    if (form != 0 && form != 1 && form != 2 && form != 4) return -1;
     if (D == 128) {
-        e = is_bf16 ? launch_attn<bf16_t, 128>(B, H, S, causal, Q, K, V, O, scale, s)
-                    : launch_attn<f16_t, 128>(B, H, S, causal, Q, K, V, O, scale, s);
+        e = is_bf16 ? launch_attn<bf16_t, 128>(form, B, H, S, causal, Q, K, V, O, scale, s)
+                    : launch_attn<f16_t, 128>(form, B, H, S, causal, Q, K, V, O, scale, s);
     } else if (D == 64) {
-        e = is_bf16 ? launch_attn<bf16_t, 64>(B, H, S, causal, Q, K, V, O, scale, s)
-                    : launch_attn<f16_t, 64>(B, H, S, causal, Q, K, V, O, scale, s);
+        e = is_bf16 ? launch_attn<bf16_t, 64>(form, B, H, S, causal, Q, K, V, O, scale, s)
+                    : launch_attn<f16_t, 64>(form, B, H, S, causal, Q, K, V, O, scale, s);
     } else {
         return -1;
     }
     return e == hipSuccess ? 0 : -2;
+}
+
+extern "C" int pyc_hip_attention_launch(int is_bf16, int B, int H, int S, int D, int causal,
+                                        const void* Q, const void* K, const void* V, void* O,
+                                        float scale, void* stream) {
+    return pyc_hip_attention_launch_form(0, is_bf16, B, H, S, D, causal, Q, K, V, O, scale, stream);
 }
 
 // Registry figures: one 8-wave workgroup per CU (the LDS ring; at d = 64 the

@@ -622,7 +622,7 @@ gemm_nt_persist_kernel(const uint16_t* __restrict__ A, const uint16_t* __restric
                 const int gm = cm0 + wm * 128 + pass * STAGE_ROWS + r;
                 if constexpr (RAG) {
                     const int gn = cn0 + wn * 128 + lrow * 8;
-                    const uint32_t off = (gm < M) & (gn < N) ? ((uint32_t)gm * (uint32_t)N + (uint32_t)gn) * 2u : kPastEnd;
+                    const uint32_t off = gm < M && gn < N ? ((uint32_t)gm * (uint32_t)N + (uint32_t)gn) * 2u : kPastEnd;
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, val), c_rsrc, off, 0, 0);
                 } else {
                     *reinterpret_cast<uint4*>(C + (size_t)gm * N + cn0 + wn * 128 + lrow * 8) = val;

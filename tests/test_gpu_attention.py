@@ -192,3 +192,43 @@ def test_attention_f16_persistent_rounds(gpu):
         q, k, v = (t[b:b + 1, h:h + 1].float().cpu().numpy() for t in (Q, K, V))
         ref = oracle.attention_f32(q, k, v, True, scale)
         _check(O[b:b + 1, h:h + 1].float().cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("form", [1, 2, 4])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("case,S", [("normal", 1), ("normal", 33), ("normal", 129), ("normal", 517),
+                                    ("large_logits", 300), ("growing_keys", 700), ("negative_scale", 300),
+                                    ("zero_scale", 300), ("all_underflow", 300)])
+def test_attention_forms(gpu, form, D, causal, case, S):
+    """Each kernel form by itself, whatever the shape rule picks: one query, one
+    key past a wave's 32 and a step's 128, several steps of the K/V ring with
+    a ragged end, and the softmax paths of test_attention_online_softmax_paths;
+    f16 too. Heads of an odd count, so that the head order is not the XCD one."""
+    torch = gpu
+    B, H = 1, 3
+    r = np.random.default_rng(S * 10 + D + causal)
+    q, k, v = (r.standard_normal((B, H, S, D)).astype(np.float32) for _ in range(3))
+    scale = 1.0 / np.sqrt(D)
+    if case == "large_logits":
+        q *= 30.0
+    elif case == "growing_keys":
+        k *= 1.0 + np.arange(S, dtype=np.float32)[:, None] / 32.0
+    elif case == "negative_scale":
+        scale = -scale
+    elif case == "zero_scale":
+        scale = 0.0
+    elif case == "all_underflow":
+        q, k, scale = np.abs(q), np.abs(k), -4.0
+    for t in (torch.bfloat16, torch.float16):
+        Q, K, V = (torch.from_numpy(x).cuda().to(t) for x in (q, k, v))
+        O = torch.full((B * H * S * D + 256,), 3.0, dtype=t, device="cuda")
+        launch = pyc_amd.lib().pyc_hip_attention_launch_form
+        import ctypes as C
+        launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 4 + [C.c_float, C.c_void_p]
+        assert launch(form, int(t == torch.bfloat16), B, H, S, D, int(causal), Q.data_ptr(), K.data_ptr(),
+                      V.data_ptr(), O.data_ptr(), scale, None) == 0
+        torch.cuda.synchronize()
+        assert bool((O[B * H * S * D:] == 3.0).all())
+        ref = oracle.attention_f32(*(x.float().cpu().numpy() for x in (Q, K, V)), causal, scale)
+        _check(O[:B * H * S * D].float().cpu().numpy().reshape(ref.shape), ref)
