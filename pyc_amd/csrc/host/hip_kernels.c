@@ -309,24 +309,32 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
     }
     /* The shape-chosen symbols: the LDS-DMA tile that the table above makes the
      * cheapest. A launcher answers 1 when the shape is outside its kernel's
-     * preconditions (alignment, K % 64 and beta == 0 for the persistent 256 x 256
-     * tile, K % 8 for the others); then the next smaller kind is asked. */
+     * preconditions (K % 64 and beta == 0 for the persistent 256 x 256 tile,
+     * operands that LDS-DMA can move for 128 x 256); then the next smaller kind
+     * is asked. Operands off a 16-byte boundary go to the persistent tile only
+     * where they always did, with a tile for every CU. */
     if (v->tile == 0) {
         const int bf = v->dtype == VT_BF16;
-        int t = pick_dma_tile(M, N, K, !v->b_trans, 0, DT_256);
-        if (t == DT_256) {
-            const int rc =
-                v->b_trans ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
-                           : pyc_hip_gemm_nn_lds_launch(bf, 1, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
+        const int off16 = (int)(((uintptr_t)A | (uintptr_t)B) & 15) != 0;
+        int last = off16 && pick_half_tile(M, N) != 256 ? DT_128X256 : DT_256;
+        for (; last >= DT_128; --last) {
+            const int t = pick_dma_tile(M, N, K, !v->b_trans, 0, last);
+            int rc;
+            if (t == DT_256) {
+                rc = v->b_trans
+                         ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
+                         : pyc_hip_gemm_nn_lds_launch(bf, 1, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
+            } else {
+                rc = pyc_hip_gemm_small_launch(bf, v->b_trans, k_dma_tiles[t].bm, k_dma_tiles[t].bn, M, N, K, A, B, C,
+                                               alpha, beta, bias, epilogue, stream);
+            }
             if (rc != 1) {
                 return rc;
             }
-            t = pick_dma_tile(M, N, K, !v->b_trans, 0, DT_128X256);
-        }
-        const int rc = pyc_hip_gemm_small_launch(bf, v->b_trans, k_dma_tiles[t].bm, k_dma_tiles[t].bn, M, N, K, A, B, C,
-                                                 alpha, beta, bias, epilogue, stream);
-        if (rc != 1) {
-            return rc;
+            if (t < DT_128X256) {
+                break;
+            }
+            last = t;
         }
     }
     return pyc_hip_gemm_half_launch(v->dtype == VT_BF16, v->b_trans, v->tile > 0 ? v->tile : pick_half_tile(M, N),

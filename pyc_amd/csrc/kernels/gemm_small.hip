@@ -42,6 +42,13 @@
 //          so a stage's tap is found once per lane (two multiplications by
 //          rounded-up reciprocals); taps in the padding, pixels past the last
 //          and k past R*S*C get the past-the-end offset.
+//  kAny    any K, N, alignment and size: rows that are no whole 16-byte chunks
+//          on 16-byte boundaries cannot go by LDS-DMA, so a wave loads its
+//          chunks into registers (unaligned 16-byte loads, those that would
+//          cross the end of their row moved back to end there and shifted), two
+//          slots ahead, and writes them to one of two LDS slots. Rows of at
+//          least 8 elements. f16 [3218,7424] x [7424,922]:
+//          470 us on register-staged tiles that loaded such rows by elements.
 #include <stdint.h>
 
 #include "common.hpp"
@@ -50,7 +57,7 @@
 namespace pyc {
 
 constexpr int kSmBK = 64;
-enum { kDense = 0, kTail = 1, kConv = 2 };
+enum { kDense = 0, kTail = 1, kConv = 2, kAny = 3 };
 constexpr uint32_t kSmPastEnd = 0xFFFFFFF0u;  // not below any descriptor's byte count
 
 struct SmConv {
@@ -59,9 +66,14 @@ struct SmConv {
     uint32_t x_bytes;
 };
 
-// Ring slots of a BM x BN tile (KS stages of 64 k per slot): as many as fit.
-constexpr int sm_slots(int bm, int bn, int ks) { return 160 * 1024 / (ks * (bm + bn) * 128); }
-constexpr size_t sm_lds_bytes(int bm, int bn, int ks) { return (size_t)sm_slots(bm, bn, ks) * ks * (bm + bn) * 128; }
+// Ring slots of a BM x BN tile (KS stages of 64 k per slot): as many as fit, or
+// the two that register staging alternates between.
+constexpr int sm_slots(int bm, int bn, int ks, int src) {
+    return src == kAny ? 2 : 160 * 1024 / (ks * (bm + bn) * 128);
+}
+constexpr size_t sm_lds_bytes(int bm, int bn, int ks, int src) {
+    return (size_t)sm_slots(bm, bn, ks, src) * ks * (bm + bn) * 128;
+}
 
 // segment swizzle f of a [K,N] k-row: (k * BN / 16 + (s ^ f(k))) % 8 differs
 // over k0..k0+3 and k0+8..k0+11
@@ -72,14 +84,14 @@ template <int BN> __device__ inline int sm_kswz(int k) {
 }
 
 template <typename T, bool BT, int BM, int BN, int KS, int SRC>
-__global__ void __launch_bounds__(512, 1)
+__global__ void __launch_bounds__(512, SRC == kAny && BM < 128 ? 4 : 2)
 gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C,
                   int M, int N, int K, float alpha, float beta, const float* __restrict__ bias, int epi,
                   int tiles_n, int vec_c, SmConv cg) {
     constexpr uint32_t A_BYTES = BM * 128, B_BYTES = BN * 128;  // one stage: 64 k of BM and of BN rows
     constexpr uint32_t STAGE_BYTES = A_BYTES + B_BYTES;
     constexpr uint32_t SLOT_BYTES = KS * STAGE_BYTES;
-    constexpr int SLOTS = sm_slots(BM, BN, KS);
+    constexpr int SLOTS = sm_slots(BM, BN, KS, SRC);
     constexpr bool HALF = KS == 1;                           // a group takes 32 k of each stage, else KS/2 stages
     constexpr int NST = HALF ? 1 : KS / 2;                   // stages a wave loads and multiplies per slot
     constexpr int NLW = HALF ? 8 : 4;                        // waves that load a stage
@@ -88,11 +100,11 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     constexpr int FM = BM / 32, FN = BN / 32;                // fragments per wave
     constexpr int SEGS = BN / 16;                            // 32-byte segments per [K,N] k-row
     constexpr int CH = BN / 8;                               // 16-byte chunks of a wave's row of fp32 results
-    static_assert(SLOTS >= 3 && (SLOTS - 2) * NST * LOADS <= 60, "ring");
+    static_assert(SRC == kAny || SLOTS >= 3 && (SLOTS - 2) * NST * LOADS <= 60, "ring");
     static_assert(SRC != kConv || BT, "the filter is the [N,K] operand");
     static_assert(BM * BN * 4 <= SLOTS * SLOT_BYTES, "results through the ring's LDS");
     __shared__ __attribute__((aligned(1024))) uint16_t smem[SLOTS * SLOT_BYTES / 2];
-    static_assert(sizeof(smem) == sm_lds_bytes(BM, BN, KS), "registered LDS figure");
+    static_assert(sizeof(smem) == sm_lds_bytes(BM, BN, KS, SRC), "registered LDS figure");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -210,6 +222,43 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
         }
     };
 
+    // kAny: chunk d of stage kt, as dma() would move it. Rows past the end are
+    // read from the last valid row (never stored), columns and k past it are
+    // 0. `edge` (uniform): some chunk of the stage reaches past its row.
+    auto load_any = [&](int d, int kt, bool edge) {
+        const uint16_t* row;
+        int c, end;  // first element of the chunk in its row, elements in the row
+        bool in = true;
+        if (d < NQA || BT) {
+            const bool a = d < NQA;
+            const int r = a ? m0 + 8 * (NQA * lw + d) + lane / 8 : n0 + 8 * (NQB * lw + d - NQA) + lane / 8;
+            row = a ? A + (size_t)min(r, M - 1) * K : B + (size_t)min(r, N - 1) * K;
+            c = kt * kSmBK + 8 * lch;
+            end = K;
+        } else {
+            constexpr int CPR = BN / 8;
+            const int kr = (1024 * (NQB * lw + d - NQA) + 16 * lane) / (2 * BN), pp = lane % CPR;
+            in = kt * kSmBK + kr < K;
+            row = B + (size_t)min(kt * kSmBK + kr, K - 1) * N;
+            c = n0 + 8 * ((((pp >> 1) ^ sm_kswz<BN>(kr)) << 1) | (pp & 1));
+            end = N;
+        }
+        u32x4 v;
+        __builtin_memcpy(&v, row + (edge ? min(c, end - 8) : c), 16);  // the device runs with unaligned access on
+        if (edge) {
+            const int sh = in ? c + 8 - min(c + 8, end) : 8;  // elements past the end
+            uint64_t lo = (uint64_t)v[0] | ((uint64_t)v[1] << 32), hi = (uint64_t)v[2] | ((uint64_t)v[3] << 32);
+            lo = sh >= 4 ? hi : lo;
+            hi = sh >= 4 ? 0 : hi;
+            const int b = 16 * (sh & 3);
+            lo = (lo >> b) | ((hi << 1) << (63 - b));
+            hi >>= b;
+            if (sh >= 8) lo = hi = 0;
+            v = u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+        }
+        return v;
+    };
+
     f32x4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -224,73 +273,121 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
 
     // stage t (< NST) of this wave's share of a slot, and its first k stage
     auto own = [&](int t) { return HALF ? 0 : kh * NST + t; };
-    auto issue_stage = [&](int st, int t, uint32_t slot_base, auto&& each) {
-        const Src x = src_of(st * KS + own(t));
-        each(x, slot_base + (uint32_t)own(t) * STAGE_BYTES);
-    };
     const int steps = (KT + KS - 1) / KS;
-    // The prologue fills all slots but one; then every step issues one slot
-    // into the place the previous step freed, so each wave has SLOTS - 2 slots
-    // of its loads outstanding at the top of every step.
-#pragma unroll 1
-    for (int p = 0; p < SLOTS - 1; ++p)
-#pragma unroll
-        for (int t = 0; t < NST; ++t)
-            issue_stage(p, t, lds0 + (uint32_t)p * SLOT_BYTES, [&](const Src& x, uint32_t base) {
-#pragma unroll
-                for (int d = 0; d < LOADS; ++d) dma(d, x, base);
-            });
     constexpr int KSTEPS = HALF ? 1 : 2;               // 32-k steps a wave multiplies per stage
     constexpr int NM = FM * FN * KSTEPS;               // MFMAs per stage and wave
     constexpr int GAP = NM / LOADS > 0 ? NM / LOADS : 1;  // MFMAs between two DMAs
-    int cur = 0, nxt = SLOTS - 1;  // slot of this step, slot that is issued now
-    for (int st = 0; st < steps; ++st) {
-        wait_vmem_le<(SLOTS - 2) * NST * LOADS>();  // own loads of this step's slot landed
-        __syncthreads();  // every wave's part of it is in LDS; the previous step's slot is consumed
+    // this wave's MFMAs on stage t of its share of slot `cur`; each(d) is called
+    // for d < LOADS with MFMAs in between
+    auto multiply = [&](int cur, int t, auto&& each) {
+        const uint16_t* As = smem + (uint32_t)cur * (SLOT_BYTES / 2) + (uint32_t)own(t) * (STAGE_BYTES / 2);
+        const uint16_t* Bs = As + A_BYTES / 2;
+        u32x4 fa[KSTEPS][FM], fb[KSTEPS][FN];
 #pragma unroll
-        for (int t = 0; t < NST; ++t) {
-            const uint16_t* As = smem + (uint32_t)cur * (SLOT_BYTES / 2) + (uint32_t)own(t) * (STAGE_BYTES / 2);
-            const uint16_t* Bs = As + A_BYTES / 2;
-            u32x4 fa[KSTEPS][FM], fb[KSTEPS][FN];
+        for (int u = 0; u < KSTEPS; ++u) {
+            const int ks = HALF ? kh : u;  // which 32 k of the stage
 #pragma unroll
-            for (int u = 0; u < KSTEPS; ++u) {
-                const int ks = HALF ? kh : u;  // which 32 k of the stage
+            for (int i = 0; i < FM; ++i) {
+                const int r = wm * (BM / 2) + 16 * i + lrow;
+                fa[u][i] = *reinterpret_cast<const u32x4*>(As + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
+            }
 #pragma unroll
-                for (int i = 0; i < FM; ++i) {
-                    const int r = wm * (BM / 2) + 16 * i + lrow;
-                    fa[u][i] = *reinterpret_cast<const u32x4*>(As + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
-                }
-#pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    if constexpr (BT) {
-                        const int r = wn * (BN / 2) + 16 * j + lrow;
-                        fb[u][j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
-                    } else {
-                        const int seg = wn * (SEGS / 2) + j;  // the fragment's 16 columns
-                        const int k0 = 32 * ks + tr_k, k1 = k0 + 4;
-                        const u32x2 lo = lds_read_tr16(Bs + k0 * BN + 16 * (seg ^ sm_kswz<BN>(k0)) + tr_c);
-                        const u32x2 hi = lds_read_tr16(Bs + k1 * BN + 16 * (seg ^ sm_kswz<BN>(k1)) + tr_c);
-                        fb[u][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-                    }
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (BT) {
+                    const int r = wn * (BN / 2) + 16 * j + lrow;
+                    fb[u][j] = *reinterpret_cast<const u32x4*>(Bs + r * 64 + 8 * ((4 * ks + lgrp) ^ (r & 7)));
+                } else {
+                    const int seg = wn * (SEGS / 2) + j;  // the fragment's 16 columns
+                    const int k0 = 32 * ks + tr_k, k1 = k0 + 4;
+                    const u32x2 lo = lds_read_tr16(Bs + k0 * BN + 16 * (seg ^ sm_kswz<BN>(k0)) + tr_c);
+                    const u32x2 hi = lds_read_tr16(Bs + k1 * BN + 16 * (seg ^ sm_kswz<BN>(k1)) + tr_c);
+                    fb[u][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
                 }
             }
-            issue_stage(st + SLOTS - 1, t, lds0 + (uint32_t)nxt * SLOT_BYTES, [&](const Src& x, uint32_t base) {
-                int d = 0;
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    const int u = m / (FM * FN), q = m % (FM * FN);
-                    acc[q / FN][q % FN] = mfma16x16x32(fb[u][q % FN], fa[u][q / FN], acc[q / FN][q % FN], T{});
-                    if (m % GAP == GAP - 1 && d < LOADS) dma(d++, x, base);
-                    if (GAP > 1) __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (; d < LOADS; ++d) dma(d, x, base);
-            });
         }
-        nxt = cur;
-        cur = cur + 1 == SLOTS ? 0 : cur + 1;
+        int d = 0;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int u = m / (FM * FN), q = m % (FM * FN);
+            acc[q / FN][q % FN] = mfma16x16x32(fb[u][q % FN], fa[u][q / FN], acc[q / FN][q % FN], T{});
+            if (m % GAP == GAP - 1 && d < LOADS) each(d++);
+            if (GAP > 1 && SRC != kAny) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (; d < LOADS; ++d) each(d);
+    };
+    if constexpr (SRC == kAny) {
+        // rg[s & 1] is slot s in registers; slot s + 1 goes to LDS and slot
+        // s + 3 starts loading while slot s is multiplied
+        u32x4 rg[2][NST * LOADS];
+        const bool edge_n = !BT && n0 + BN > N;
+        auto fetch = [&](int st, u32x4 (&r)[NST * LOADS]) {
+            if (edge_n || (st + 1) * KS * kSmBK > K) {
+#pragma unroll
+                for (int t = 0; t < NST; ++t)
+#pragma unroll
+                    for (int d = 0; d < LOADS; ++d) r[t * LOADS + d] = load_any(d, st * KS + own(t), true);
+            } else {
+#pragma unroll
+                for (int t = 0; t < NST; ++t)
+#pragma unroll
+                    for (int d = 0; d < LOADS; ++d) r[t * LOADS + d] = load_any(d, st * KS + own(t), false);
+            }
+        };
+        auto put = [&](int st, const u32x4 (&r)[NST * LOADS]) {
+#pragma unroll
+            for (int t = 0; t < NST; ++t)
+#pragma unroll
+                for (int d = 0; d < LOADS; ++d) {
+                    const uint32_t off = d < NQA ? (uint32_t)(NQA * lw + d) * 1024
+                                                 : A_BYTES + (uint32_t)(NQB * lw + d - NQA) * 1024;
+                    *reinterpret_cast<u32x4*>(smem + (((st & 1) * SLOT_BYTES + own(t) * STAGE_BYTES + off) / 2 +
+                                                      lane * 8)) = r[t * LOADS + d];
+                }
+        };
+        fetch(0, rg[0]);
+        fetch(1, rg[1]);
+        put(0, rg[0]);
+        fetch(2, rg[0]);
+        __syncthreads();
+        for (int st = 0; st < steps; st += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {  // slots past the last are zeros
+                put(st + u + 1, rg[(u + 1) & 1]);
+                fetch(st + u + 3, rg[(u + 1) & 1]);
+#pragma unroll
+                for (int t = 0; t < NST; ++t) multiply(u, t, [](int) {});
+                __syncthreads();
+            }
+        }
+    } else {
+        // The prologue fills all slots but one; then every step issues one slot
+        // into the place the previous step freed, so each wave has SLOTS - 2
+        // slots of its loads outstanding at the top of every step.
+#pragma unroll 1
+        for (int p = 0; p < SLOTS - 1; ++p)
+#pragma unroll
+            for (int t = 0; t < NST; ++t) {
+                const Src x = src_of(p * KS + own(t));
+#pragma unroll
+                for (int d = 0; d < LOADS; ++d)
+                    dma(d, x, lds0 + (uint32_t)p * SLOT_BYTES + (uint32_t)own(t) * STAGE_BYTES);
+            }
+        int cur = 0, nxt = SLOTS - 1;  // slot of this step, slot that is issued now
+        for (int st = 0; st < steps; ++st) {
+            wait_vmem_le<(SLOTS >= 2 ? SLOTS - 2 : 0) * NST * LOADS>();  // own loads of this step's slot landed
+            __syncthreads();  // every wave's part of it is in LDS; the previous step's slot is consumed
+#pragma unroll
+            for (int t = 0; t < NST; ++t) {
+                const Src x = src_of((st + SLOTS - 1) * KS + own(t));
+                const uint32_t base = lds0 + (uint32_t)nxt * SLOT_BYTES + (uint32_t)own(t) * STAGE_BYTES;
+                multiply(cur, t, [&](int d) { dma(d, x, base); });
+            }
+            nxt = cur;
+            cur = cur + 1 == SLOTS ? 0 : cur + 1;
+        }
     }
-    wait_vmem_le<0>();  // the loads past the last stage have landed too
+    if constexpr (SRC != kAny) wait_vmem_le<0>();  // the loads past the last stage have landed too
     __syncthreads();    // every wave is done with the ring; it takes the results
 
     // Results as fp32 in LDS, BM/2 x BN/2 per quadrant, 16-byte chunk c of row
@@ -375,35 +472,41 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
     if (bm == 32 && bn == 32) PYC_SMALL(32, 32, 4);
     else if (bm == 64 && bn == 64) PYC_SMALL(64, 64, 2);
     else if (bm == 128 && bn == 128) PYC_SMALL(128, 128, 1);
-    else if (bm == 128 && bn == 256) PYC_SMALL(128, 256, 1);
-    else return 1;
+    else if constexpr (SRC != kAny) {
+        if (bm == 128 && bn == 256) PYC_SMALL(128, 256, 1);
+        else return 1;
+    } else return 1;
 #undef PYC_SMALL
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 }  // namespace pyc
 
-// bm x bn: one of the tiles above. Returns 1 when the shape is outside this
-// kernel's preconditions (K a multiple of 8 and, for [K,N] B, N of 4; A and B
-// 16-byte aligned and below 4 GiB), 0 on launch, -2 on a launch error. Ragged M
-// and N: rows of A (and of [N,K] B) past the end are read as zeros through the
-// buffer descriptors, [K,N] B columns past N read neighbouring data, and only
-// the rows and columns of C inside M x N are written.
+// bm x bn: one of the tiles above. Rows of A (and of [N,K] B) past the end are
+// read as zeros through the buffer descriptors, [K,N] B columns past N read
+// neighbouring data, and only the rows and columns of C inside M x N are
+// written. LDS-DMA takes K a multiple of 8 and, for [K,N] B, N of 4, with A and
+// B 16-byte aligned and below 4 GiB; other shapes are staged through registers,
+// up to 128 x 128 tiles, with rows of at least 8 elements. Returns 1 for an
+// unknown tile (128 x 256 for a shape that is register-staged) and for shorter
+// rows, 0 on launch, -2 on a launch error.
 extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
                                          const void* B, void* C, float alpha, float beta, const float* bias,
                                          int epi, void* stream) {
     using namespace pyc;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 8 || (!b_trans && N % 4)) return 1;
+    if (M <= 0 || N <= 0 || K <= 0) return 1;
     const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
-    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
-    if ((K % kSmBK || !b_trans) && ((size_t)M * K * 2 > kSmPastEnd || (size_t)N * kpad * 2 > kSmPastEnd)) return 1;
-    if (((uintptr_t)A | (uintptr_t)B) & 15) return 1;
+    const bool tail = K % kSmBK != 0;
+    const bool any = K % 8 || (!b_trans && N % 4) || (((uintptr_t)A | (uintptr_t)B) & 15) ||
+                     (size_t)M * K * 2 > kSmPastEnd || (size_t)N * K * 2 > kSmPastEnd ||
+                     ((tail || !b_trans) && (size_t)N * kpad * 2 > kSmPastEnd);
+    if (any && (K < 8 || (!b_trans && N < 8))) return 1;
     hipStream_t s = (hipStream_t)stream;
     const SmConv cg{};
-    const bool tail = K % kSmBK != 0;
 #define PYC_GO(TY, BT)                                                                                              \
-    (tail ? launch_small<TY, BT, kTail>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                    \
-          : launch_small<TY, BT, kDense>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg))
+    (any    ? launch_small<TY, BT, kAny>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                   \
+     : tail ? launch_small<TY, BT, kTail>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                  \
+            : launch_small<TY, BT, kDense>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg))
     if (is_bf16) return b_trans ? PYC_GO(bf16_t, true) : PYC_GO(bf16_t, false);
     return b_trans ? PYC_GO(f16_t, true) : PYC_GO(f16_t, false);
 #undef PYC_GO
@@ -441,7 +544,7 @@ extern "C" int pyc_hip_kinfo_small(int tile, int b_trans, int is_bf16, pyc_hip_k
     if (!out || (tile != 64 && tile != 128)) return -1;
     out->threads = 512;
     out->waves_per_simd = 2;
-    out->lds_bytes = sm_lds_bytes(tile, tile, tile == 64 ? 2 : 1);
+    out->lds_bytes = sm_lds_bytes(tile, tile, tile == 64 ? 2 : 1, kDense);
     out->name = tile == 64 ? "gemm_small_kernel<64>" : "gemm_small_kernel<128>";
 #define PYC_KI(TY, BT) \
     out->fn = tile == 64 ? reinterpret_cast<const void*>(&gemm_small_kernel<TY, BT, 64, 64, 2, kDense>) \

@@ -488,3 +488,46 @@ def test_lds_tile_choice_covers_shapes(gpu):
             bound = 2.0 ** -8 * ref.abs() + 4e-6 * np.sqrt(k) * ref.abs().max()
             bad = ~((Cd.float() - ref).abs() <= bound)
             assert not bool(bad.any()), (m, n, k, bt, int(bad.sum()))
+
+
+@pytest.mark.parametrize("bt", [32, 64, 128])
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("dn,k,off", [(1, 9, 0),       # the shortest rows: one chunk and one element over
+                                      (3, 65, 1),      # operands one element off a 16-byte boundary
+                                      (8, 64, 3),      # whole chunks, off the boundary
+                                      (-7, 1415, 0),   # one partial tile each way, every slot pair wraps
+                                      (2, 1416, 0)])   # [K,N]: rows of 4-byte alignment
+def test_register_staged_tiles(gpu, bt, layout, dtype, dn, k, off):
+    """Shapes LDS-DMA cannot move (rows that are no whole 16-byte chunks, bases
+    off a 16-byte boundary), on each tile: chunks that cross the end of a row
+    are loaded from inside it and shifted, so an infinity in the element after
+    the row's end must not show; nothing is written past C."""
+    torch = gpu
+    nt = layout == "nt"
+    m, n = bt + 1, bt + dn
+    r = np.random.default_rng(bt + k + dn)
+    t = torch.bfloat16 if dtype == "bf16" else torch.float16
+
+    def place(x):  # x in the middle of infinities, off elements past a boundary
+        buf = torch.full((x.size + 64,), float("inf"), dtype=t, device="cuda")
+        buf[8 + off:8 + off + x.size] = torch.from_numpy(x.reshape(-1)).cuda().to(t)
+        return buf, buf.data_ptr() + 2 * (8 + off), buf[8 + off:8 + off + x.size].float().cpu().numpy().reshape(x.shape)
+
+    ab, ap, a = place((r.standard_normal((m, k)) / np.sqrt(k)).astype(np.float32))
+    bb, bp, b = place(r.standard_normal((n, k) if nt else (k, n)).astype(np.float32))
+    bias = r.standard_normal(n).astype(np.float32)
+    Bd = dev_f32(torch, bias)
+    Cd = torch.full((m * n + 256,), 7.0, dtype=t, device="cuda")
+    launch = pyc_amd.lib().pyc_hip_gemm_small_launch
+    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p, C.c_int, C.c_void_p]
+    assert launch(int(dtype == "bf16"), int(nt), bt, bt, m, n, k, ap, bp, Cd.data_ptr(), -0.5, 0.0, Bd.data_ptr(), 1,
+                  None) == 0
+    torch.cuda.synchronize()
+    assert bool((Cd[m * n:] == 7.0).all())
+    ref = -0.5 * (a @ (b.T if nt else b)) + bias
+    got = Cd[:m * n].float().cpu().numpy().reshape(m, n)
+    # one rounding of the result (2^-8 or 2^-11 relative) plus fp32 summation order
+    bad = ~(np.abs(got - ref) <= 2.0 ** (-8 if dtype == "bf16" else -11) * np.abs(ref) +
+            4e-6 * np.sqrt(k) * np.abs(ref).max())
+    assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
