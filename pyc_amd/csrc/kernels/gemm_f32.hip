@@ -201,8 +201,22 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B, float*
 // c ^ 4((k >> 2) & 3), and read one element per lane (ds_read_b32): the 16
 // lanes of each k slot read 16 consecutive n of rows 4 apart, which the
 // swizzle puts in four different 16-bank groups.
-constexpr int kF32Stages = 4;
+//
+// RAG: any M, N, K (fp32 rows start on 4-byte boundaries, which is what a
+// dword-multiple load needs; the rows of the whole-tile form are 16-byte
+// aligned). Every load carries its whole offset in the vector register, so that
+// the descriptor's range check, which works dword by dword, zeroes what lies
+// past the operand: rows past M (or N), [K,N] k-rows past K, and the 16-byte
+// chunks past K of an A or [N,K] row get an offset past its end. A chunk that
+// crosses the end of its row brings the next row's first elements along: they
+// are overwritten with zeros in LDS before the last k-tile is read. k-tiles past
+// the last are issued too, all past the end (no traffic).
+// TILE 32: the same kernel with a quarter of the tile (each wave one 16x16
+// block of a k half, a ring of 8 stages), for products with few 64x64 tiles:
+// a k-tile takes about 0.4 us instead of 1.0.
+constexpr int kF32Stages = 4, kF32Stages32 = 8;
 constexpr size_t kF32DmaLds = (size_t)kF32Stages * 2 * kF32BM * kF32BK * 4;
+constexpr uint32_t kF32PastEnd = 0xFFFFFFF0u;  // not below any descriptor's byte count
 
 // SIG: the launch ends a synchronous run, and the kernel itself tells the host
 // when its results are complete (instead of a separate one-lane kernel behind
@@ -212,13 +226,21 @@ constexpr size_t kF32DmaLds = (size_t)kF32Stages * 2 * kF32BM * kF32BK * 4;
 // arrival re-arms the counters and stores `done_seq` into the pinned host
 // word. A kernel on any stream that the host starts after seeing the word
 // reads the whole of C, although the grid's last waves may still be exiting.
-template <bool BT, bool SIG>
+template <bool BT, bool SIG, int TILE, bool RAG>
 __global__ void __launch_bounds__(512, 1)
 gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
                     int M, int N, int K, float alpha, float beta, const float* __restrict__ bias,
                     int epi, int group_m, uint32_t* __restrict__ done_word, uint32_t* __restrict__ done_count,
                     uint32_t done_seq) {
-    __shared__ __attribute__((aligned(1024))) float smem[kF32Stages * 2 * kF32BM * kF32BK];
+    constexpr int BK = kF32BK;
+    constexpr int STAGES = TILE == 64 ? kF32Stages : kF32Stages32;
+    constexpr int F = TILE / 32;                       // 16-wide fragments per wave and operand
+    constexpr int NH = TILE / 32;                      // DMA instructions per wave and operand per k-tile
+    constexpr int NDMA = 2 * NH;
+    constexpr uint32_t OP_BYTES = TILE * BK * 4;       // one operand's part of a stage
+    constexpr int CPR = TILE / 4;                      // 16-byte chunks per [K,N] k-row
+    constexpr int NSWZ = TILE == 64 ? 3 : 1;           // k-row groups that its swizzle tells apart, minus one
+    __shared__ __attribute__((aligned(1024))) float smem[STAGES * 2 * TILE * BK];
     static_assert(sizeof(smem) == kF32DmaLds, "registered LDS figure");
 
     const int tid = threadIdx.x;
@@ -232,7 +254,7 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     // tile indices are given to one XCD; tiles are numbered in groups of
     // group_m tile rows, column by column, so the tiles an XCD holds at once
     // share a few A row panels and B column panels in its L2.
-    const int tiles_n = N / kF32BN, tiles_m = M / kF32BM;
+    const int tiles_n = (N + TILE - 1) / TILE, tiles_m = (M + TILE - 1) / TILE;
     int bid = blockIdx.x;
     const int nblk = gridDim.x;
     if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
@@ -241,142 +263,172 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     const int first_m = grp * group_m;
     const int gsz = min(tiles_m - first_m, group_m);
     const int in = bid - grp * span;
-    const int m0 = (first_m + in % gsz) * kF32BM;
-    const int n0 = (in / gsz) * kF32BN;
-    const int KT = K / kF32BK;
+    const int m0 = (first_m + in % gsz) * TILE;
+    const int n0 = (in / gsz) * TILE;
+    const int KT = (K + BK - 1) / BK;
 
     const i32x4 ra = make_buf_rsrc(A, (uint32_t)((size_t)M * K * 4));
     const i32x4 rb = make_buf_rsrc(B, (uint32_t)((size_t)N * K * 4));
-    // wave w issues rows 8w .. 8w+7 of the A tile and of the B tile (two
-    // instructions each, four rows per instruction); lane i writes chunk
-    // position p = i % 16 of row 4j + i / 16
-    uint32_t va[2], vb[2];
+    // wave w issues TILE / 8 rows of the A tile and of the [N,K] B tile (four
+    // rows of 16 chunks per instruction; lane i writes chunk position p = i % 16
+    // of row i / 16) and 8 k-rows of a [K,N] B tile
+    uint32_t va[NH], vb[NH];
+    int lch[NH];  // the lane's logical chunk in those rows
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int row = 8 * wave + 4 * h + (lane >> 4), p = lane & 15;
-        va[h] = (uint32_t)(((size_t)(m0 + row) * K + 4 * (p ^ (row & 7))) * 4);
-        if constexpr (BT) vb[h] = (uint32_t)(((size_t)(n0 + row) * K + 4 * (p ^ (row & 7))) * 4);
-        else vb[h] = (uint32_t)(((size_t)row * N + n0 + 4 * (p ^ (4 * ((row >> 2) & 3)))) * 4);
+    for (int h = 0; h < NH; ++h) {
+        const int row = TILE / 8 * wave + 4 * h + (lane >> 4), p = lane & 15;
+        lch[h] = p ^ (row & 7);
+        va[h] = (uint32_t)(((size_t)(m0 + row) * K + 4 * lch[h]) * 4);
+        if constexpr (BT) {
+            vb[h] = (uint32_t)(((size_t)(n0 + row) * K + 4 * lch[h]) * 4);
+        } else {
+            const int kr = 8 * wave + h * (64 / CPR) + lane / CPR;
+            vb[h] = (uint32_t)(((size_t)kr * N + n0 + 4 * ((lane % CPR) ^ (4 * ((kr >> 2) & NSWZ)))) * 4);
+        }
         asm volatile("" : "+v"(va[h]), "+v"(vb[h]));
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
-    // DMA d (0..3) of k-tile kt into ring slot `slot`: d / 2 = h, A if d even
+    // DMA d (< NDMA) of k-tile kt into ring slot `slot`: d / 2 = h, A if d even
     auto issue_one = [&](int kt, int slot_i, int d) {
-        const uint32_t slot = lds0 + (uint32_t)(slot_i * 2 * kF32BM * kF32BK * 4);
-        const uint32_t sa = (uint32_t)kt * kF32BK * 4;
-        const uint32_t sb = BT ? sa : (uint32_t)kt * kF32BK * (uint32_t)N * 4;
+        const uint32_t slot = lds0 + (uint32_t)slot_i * 2 * OP_BYTES;
+        const uint32_t sa = (uint32_t)kt * BK * 4;
+        const uint32_t sb = BT ? sa : (uint32_t)kt * BK * (uint32_t)N * 4;
         const int h = d >> 1;
-        const uint32_t off = (uint32_t)(8 * wave + 4 * h) * kF32BK * 4;
-        if ((d & 1) == 0) lds_dma_buf_b128_u(ra, va[h], sa, slot + off);
-        else lds_dma_buf_b128_u(rb, vb[h], sb, slot + kF32BM * kF32BK * 4 + off);
+        const uint32_t off = (uint32_t)(TILE / 8 * wave + 4 * h) * BK * 4;  // = (8 wave + h 64 / CPR) TILE 4
+        const bool inside = !RAG || kt * BK + 4 * lch[h] < K;
+        if ((d & 1) == 0) {
+            if constexpr (RAG) lds_dma_buf_b128_u(ra, inside ? va[h] + sa : kF32PastEnd, 0u, slot + off);
+            else lds_dma_buf_b128_u(ra, va[h], sa, slot + off);
+        } else {
+            if constexpr (RAG) lds_dma_buf_b128_u(rb, !BT || inside ? vb[h] + sb : kF32PastEnd, 0u, slot + OP_BYTES + off);
+            else lds_dma_buf_b128_u(rb, vb[h], sb, slot + OP_BYTES + off);
+        }
     };
-    // k-tile kt, all four DMAs, into slot kt % 4 (the prologue)
-    auto issue = [&](int kt) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) issue_one(kt, kt % kF32Stages, d);
-    };
+    static_assert(TILE / 8 * BK == 8 * TILE && 4 * BK == 64 / CPR * TILE, "one LDS offset for both B layouts");
 
-    f32x4 acc[2][2];
+    f32x4 acc[F][F];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < F; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int lrow = lane & 15, lgrp = lane >> 4;
     // fragment f of half kk (16 k: 4 per k slot) of the k-tile in ring slot
-    // kt % 4: f = 0, 1 the A rows 16 f.., f = 2, 3 the B columns 16 (f - 2)..
-    auto rd = [&](int kt, int kk, int f, f32x4 (&af)[2], f32x4 (&bfr)[2]) {
-        const float* As = smem + (kt % kF32Stages) * 2 * kF32BM * kF32BK;
-        const float* Bs = As + kF32BM * kF32BK;
+    // kt % STAGES: f < F the A rows 16 f.., f >= F the B columns 16 (f - F)..
+    auto rd = [&](int kt, int kk, int f, f32x4 (&af)[F], f32x4 (&bfr)[F]) {
+        const float* As = smem + (kt % STAGES) * 2 * TILE * BK;
+        const float* Bs = As + TILE * BK;
         const int ch = (kh * 2 + kk) * 4 + lgrp;
-        const int i = f & 1;
-        if (f < 2) {
-            const int r = wm * 32 + i * 16 + lrow;
-            af[i] = *reinterpret_cast<const f32x4*>(&As[r * kF32BK + swz8(r, ch) * 4]);
+        const int i = f % F;
+        if (f < F) {
+            const int r = wm * (TILE / 2) + i * 16 + lrow;
+            af[i] = *reinterpret_cast<const f32x4*>(&As[r * BK + swz8(r, ch) * 4]);
         } else {
-            const int n = wn * 32 + i * 16 + lrow;
+            const int n = wn * (TILE / 2) + i * 16 + lrow;
             if constexpr (BT) {
-                bfr[i] = *reinterpret_cast<const f32x4*>(&Bs[n * kF32BK + swz8(n, ch) * 4]);
+                bfr[i] = *reinterpret_cast<const f32x4*>(&Bs[n * BK + swz8(n, ch) * 4]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int k = 4 * ch + e;  // (k >> 2) & 3 == lgrp
-                    bfr[i][e] = Bs[k * kF32BN + (((n >> 2) ^ (4 * lgrp)) << 2) + (n & 3)];
+                    bfr[i][e] = Bs[k * TILE + (((n >> 2) ^ (4 * (lgrp & NSWZ))) << 2) + (n & 3)];
                 }
             }
         }
     };
+    // RAG: zeros over the elements of the last k-tile that its row-crossing
+    // chunks brought from the next row (K % 4 of them are real)
+    auto clear_crossing = [&]() {
+        float* As = smem + ((KT - 1) % STAGES) * 2 * TILE * BK;
+        const int c = (K % BK) / 4;
+        if (tid < (BT ? 2 : 1) * TILE) {
+            float* row = (tid < TILE ? As : As + TILE * BK) + (tid % TILE) * BK + swz8(tid % TILE, c) * 4;
+            for (int e = K % 4; e < 4; ++e) row[e] = 0.f;
+        }
+        __syncthreads();
+    };
+    const bool crossing = RAG && K % 4 != 0;
 
-    // Ring: while k-tile kt is multiplied, kt+1 has landed, kt+2 is in flight
-    // and kt+3 (clamped to the last k-tile: a duplicate into the free slot)
-    // is issued into the slot kt-1 left, so the wait count is the same every
-    // step. Per step the 32 MFMAs go out in program order (sched_barrier) in
-    // groups of two: the second half's fragment reads ride on the first four
-    // groups, the next k-tile's first-half reads on groups 8-11 (it landed
-    // before this step's barrier), and the four DMAs on groups 12-15.
+    // Ring: while k-tile kt is multiplied, kt+1 has landed, the next ones are in
+    // flight and kt+STAGES-1 (whole tiles: clamped to the last k-tile, a
+    // duplicate into the free slot) is issued into the slot kt-1 left, so the
+    // wait count is the same every step. Per step the MFMAs go out in program
+    // order (sched_barrier) in groups of two: the second half's fragment reads
+    // ride on the first groups, the next k-tile's first-half reads on the first
+    // groups of the second half (it landed before this step's barrier), and
+    // the DMAs on the last groups.
+    auto stage_of = [&](int kt) { return RAG ? kt : min(kt, KT - 1); };
+    constexpr int NGH = 2 * F * F;  // groups of two MFMAs per half
+    constexpr int NFR = 2 * F;      // fragment reads per half
 #pragma unroll
-    for (int s = 0; s < kF32Stages - 1; ++s) issue(min(s, KT - 1));
-    wait_vmem_le<8>();  // this wave's loads of k-tile 0 landed
+    for (int s = 0; s < STAGES - 1; ++s)
+#pragma unroll
+        for (int d = 0; d < NDMA; ++d) issue_one(stage_of(s), s, d);
+    wait_vmem_le<(STAGES - 2) * NDMA>();  // this wave's loads of k-tile 0 landed
     __syncthreads();
-    f32x4 af0[2], bf0[2];
+    if (crossing && KT == 1) clear_crossing();
+    f32x4 af0[F], bf0[F];
 #pragma unroll
-    for (int f = 0; f < 4; ++f) rd(0, 0, f, af0, bf0);
+    for (int f = 0; f < NFR; ++f) rd(0, 0, f, af0, bf0);
     for (int kt = 0; kt < KT; ++kt) {
-        wait_vmem_le<4>();  // own loads of k-tile kt+1 landed (kt+2's may be in flight)
+        wait_vmem_le<(STAGES - 3) * NDMA>();  // own loads of k-tile kt+1 landed (later ones may be in flight)
         // every wave's part of k-tile kt+1 is in LDS, and k-tile kt-1 (and
         // the prefetch of kt) is consumed
         __syncthreads();
-        const int kn = min(kt + kF32Stages - 1, KT - 1);
-        f32x4 af1[2], bf1[2];
+        if (crossing && kt == KT - 2) clear_crossing();
+        const int kn = stage_of(kt + STAGES - 1);
+        f32x4 af1[F], bf1[F];
 #pragma unroll
-        for (int g = 0; g < 16; ++g) {
+        for (int g = 0; g < 2 * NGH; ++g) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                const int q = (2 * g + u) & 15;  // MFMA q of the half: element e = q / 4, block (i, j) = q % 4
-                const int e = q >> 2, i = (q >> 1) & 1, j = q & 1;
-                if (g < 8) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af0[i][e], bf0[j][e], acc[i][j], 0, 0, 0);
+                const int q = (2 * g + u) % (2 * NGH);  // MFMA q of the half: element e, block (i, j)
+                const int e = q / (F * F), i = q / F % F, j = q % F;
+                if (g < NGH) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af0[i][e], bf0[j][e], acc[i][j], 0, 0, 0);
                 else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af1[i][e], bf1[j][e], acc[i][j], 0, 0, 0);
             }
-            if (g < 4) rd(kt, 1, g, af1, bf1);
-            if (g >= 8 && g < 12) rd(kt + 1, 0, g - 8, af0, bf0);  // past the last k-tile: a stale slot, unused
-            if (g >= 12) issue_one(kn, (kt + kF32Stages - 1) % kF32Stages, g - 12);
+            if (g < NFR) rd(kt, 1, g, af1, bf1);
+            if (g >= NGH && g < NGH + NFR) rd(kt + 1, 0, g - NGH, af0, bf0);  // past the last k-tile: unused
+            if (g >= 2 * NGH - NDMA) issue_one(kn, (kt + STAGES - 1) % STAGES, g - (2 * NGH - NDMA));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    wait_vmem_le<0>();  // the clamped duplicates have landed too
+    wait_vmem_le<0>();  // the loads past the last k-tile have landed too
     __syncthreads();  // every wave is done with the ring
 
     // k halves summed through LDS (waves 4-7 hand theirs to waves 0-3)
     float* red = smem;
     if (kh) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < F; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < F; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) red[(quad * 16 + (i * 2 + j) * 4 + r) * 64 + lane] = acc[i][j][r];
+                for (int r = 0; r < 4; ++r) red[(quad * 4 * F * F + (i * F + j) * 4 + r) * 64 + lane] = acc[i][j][r];
     }
     __syncthreads();
     if (!SIG && kh) return;
     if (!kh) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < F; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < F; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][j][r] += red[(quad * 16 + (i * 2 + j) * 4 + r) * 64 + lane];
+                for (int r = 0; r < 4; ++r) acc[i][j][r] += red[(quad * 4 * F * F + (i * F + j) * 4 + r) * 64 + lane];
 
         const bool has_bias = (epi & 1) && bias != nullptr;
         const bool relu = (epi & 2) != 0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int gn = n0 + wn * 32 + j * 16 + lrow;
+        for (int j = 0; j < F; ++j) {
+            const int gn = n0 + wn * (TILE / 2) + j * 16 + lrow;
+            if (RAG && gn >= N) continue;
             const float bv = has_bias ? bias[gn] : 0.f;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < F; ++i) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int gm = m0 + wm * 32 + i * 16 + lgrp * 4 + r;
+                    const int gm = m0 + wm * (TILE / 2) + i * 16 + lgrp * 4 + r;
+                    if (RAG && gm >= M) continue;
                     float* cp = C + (size_t)gm * N + gn;
                     float v = alpha * acc[i][j][r];
                     if (beta != 0.f) v += beta * *cp;
@@ -397,6 +449,20 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
 
 }  // namespace pyc
 
+// 64 or 32: the tile that takes less time, by estimated microseconds: a start
+// and end per round of one tile per CU, and a time per k-tile. Measured on the
+// MI355X, 64 / 32 (and the register-staged kernel that took ragged shapes), in
+// us, [K,N] B: 512 x 128 x 2638 52 / 20.8 (119), 440^3 13.1 / 6.7 (20.4), 512^3
+// 11.5 / 6.8, 700 x 701 x 702 18.7 / 16.5 (38), 768^3 16.4 / 23, 1000^3 24.2 / 38
+// (40), 1024^3 20.5 / 37, 2624 x 256 x 280 11 / 13.8 (15.5).
+static int tile_f32(long M, long N, long K, bool whole) {
+    const double kt = (double)((K + 63) / 64);
+    const long t64 = ((M + 63) / 64) * ((N + 63) / 64), t32 = ((M + 31) / 32) * ((N + 31) / 32);
+    const double c64 = (double)((t64 + 255) / 256) * (2.5 + kt * (whole && t64 <= 256 ? 1.0 : 1.25));
+    const double c32 = (double)((t32 + 255) / 256) * (2.2 + kt * 0.43);
+    return c32 < c64 ? 32 : 64;
+}
+
 extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A,
                                        const void* B, void* C, float alpha, float beta,
                                        const float* bias, int epi, void* stream) {
@@ -408,28 +474,41 @@ extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const v
     const float* b = (const float*)B;
     float* c = (float*)C;
     // the LDS-DMA kernel addresses each operand through a buffer descriptor
-    // (32-bit byte offsets) and moves 16-byte chunks
-    const bool dma = even && K > 0 && (size_t)M * K * 4 < (1ull << 32) && (size_t)N * K * 4 < (1ull << 32) &&
-                     ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0);
+    // (32-bit byte offsets, rows and k padded to whole tiles and ring stages)
+    // and moves 16-byte chunks, of whole tiles on 16-byte boundaries
+    const size_t pad = 16 * kF32BK;
+    const bool whole = even && ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0);
+    const bool dma = ((uintptr_t)A % 4 == 0) && ((uintptr_t)B % 4 == 0) &&
+                     (whole ? (size_t)M * K * 4 < (1ull << 32) && (size_t)N * K * 4 < (1ull << 32)
+                            : ((size_t)M + pad) * ((size_t)K + pad) * 4 < kF32PastEnd &&
+                                  ((size_t)N + pad) * ((size_t)K + pad) * 4 < kF32PastEnd);
     if (dma) {
-        const dim3 tiles((unsigned)((M / kF32BM) * (N / kF32BN)));
-        const int gm = M / kF32BM < 4 ? M / kF32BM : 4;
-        RunSignal sg;
-        if (run_signal_claim(&sg)) {
-            // this launch ends the run: it stores the completion word itself
-            if (b_trans)
-                hipLaunchKernelGGL((gemm_f32_dma_kernel<true, true>), tiles, block, 0, s, a, b, c, M, N, K, alpha,
-                                   beta, bias, epi, gm, sg.word, sg.count, sg.seq);
-            else
-                hipLaunchKernelGGL((gemm_f32_dma_kernel<false, true>), tiles, block, 0, s, a, b, c, M, N, K, alpha,
-                                   beta, bias, epi, gm, sg.word, sg.count, sg.seq);
+        const int tile = tile_f32(M, N, K, whole);
+        const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+        const dim3 tiles((unsigned)(tiles_m * tiles_n));
+        const int gm = tiles_m < 4 ? tiles_m : 4;
+        RunSignal sg{nullptr, nullptr, 0u};
+        // when this launch ends the run, it stores the completion word itself
+        const bool sig = run_signal_claim(&sg);
+#define PYC_F32(BT, SIG, TILE, RAG)                                                                                \
+    hipLaunchKernelGGL((gemm_f32_dma_kernel<BT, SIG, TILE, RAG>), tiles, block, 0, s, a, b, c, M, N, K, alpha, beta, \
+                       bias, epi, gm, sg.word, sg.count, sg.seq)
+#define PYC_F32_TILE(BT, SIG)                              \
+    do {                                                   \
+        if (tile == 32) PYC_F32(BT, SIG, 32, true);        \
+        else if (whole) PYC_F32(BT, SIG, 64, false);       \
+        else PYC_F32(BT, SIG, 64, true);                   \
+    } while (0)
+        if (sig) {
+            if (b_trans) PYC_F32_TILE(true, true);
+            else PYC_F32_TILE(false, true);
         } else if (b_trans) {
-            hipLaunchKernelGGL((gemm_f32_dma_kernel<true, false>), tiles, block, 0, s, a, b, c, M, N, K, alpha, beta,
-                               bias, epi, gm, nullptr, nullptr, 0u);
+            PYC_F32_TILE(true, false);
         } else {
-            hipLaunchKernelGGL((gemm_f32_dma_kernel<false, false>), tiles, block, 0, s, a, b, c, M, N, K, alpha, beta,
-                               bias, epi, gm, nullptr, nullptr, 0u);
+            PYC_F32_TILE(false, false);
         }
+#undef PYC_F32_TILE
+#undef PYC_F32
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }
     if (b_trans) {
@@ -451,7 +530,7 @@ extern "C" int pyc_hip_kinfo_f32(int b_trans, pyc_hip_kinfo* out) {
     out->lds_bytes = kF32DmaLds;
     out->threads = 512;
     out->waves_per_simd = 2;
-    out->fn = b_trans ? reinterpret_cast<const void*>(&gemm_f32_dma_kernel<true, false>)
-                      : reinterpret_cast<const void*>(&gemm_f32_dma_kernel<false, false>);
+    out->fn = b_trans ? reinterpret_cast<const void*>(&gemm_f32_dma_kernel<true, false, 64, false>)
+                      : reinterpret_cast<const void*>(&gemm_f32_dma_kernel<false, false, 64, false>);
     return 0;
 }

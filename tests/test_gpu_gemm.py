@@ -531,3 +531,50 @@ def test_register_staged_tiles(gpu, bt, layout, dtype, dn, k, off):
     bad = ~(np.abs(got - ref) <= 2.0 ** (-8 if dtype == "bf16" else -11) * np.abs(ref) +
             4e-6 * np.sqrt(k) * np.abs(ref).max())
     assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("m,n,k,off", [
+    (33, 31, 1, 0),      # 32 x 32 tiles, one element of k
+    (65, 130, 67, 1),    # a chunk that crosses the row's end in the second k-tile; bases off 16 bytes
+    (129, 63, 640, 0),   # ragged M and N over whole k-tiles, the 8-stage ring wraps
+    (700, 1000, 66, 0),  # 64 x 64 tiles, crossing chunks
+    (961, 1021, 129, 3), # 64 x 64 tiles, one element into the third k-tile
+    (64, 64, 257, 0),    # whole M and N
+])
+def test_f32_ragged_tiles(gpu, m, n, k, off, layout):
+    """fp32 shapes that are no whole 64 x 64 x 64 tiles, on both tiles, against
+    float64: infinities right after the operands and in their first elements
+    (which a chunk that crosses the end of the row before brings along) stay in
+    their own row and column, and nothing is written past C."""
+    torch = gpu
+    bt = layout == "nt"
+    r = np.random.default_rng(m + n + k)
+
+    def place(x):
+        buf = torch.full((x.size + 64,), float("inf"), dtype=torch.float32, device="cuda")
+        buf[16 + off:16 + off + x.size] = torch.from_numpy(x.reshape(-1)).cuda()
+        return buf, buf.data_ptr() + 4 * (16 + off)
+
+    a = r.uniform(-1, 1, (m, k)).astype(np.float32)
+    b = r.uniform(-1, 1, (n, k) if bt else (k, n)).astype(np.float32)
+    a[1, 0] = np.inf
+    bias = r.uniform(-1, 1, n).astype(np.float32)
+    ab, ap = place(a)
+    bb, bp = place(b)
+    Bd = dev_f32(torch, bias)
+    C0 = torch.from_numpy(r.uniform(-1, 1, m * n + 256).astype(np.float32)).cuda()
+    Cd = C0.clone()
+    launch = pyc_amd.lib().pyc_hip_gemm_f32_launch
+    launch.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p, C.c_int, C.c_void_p]
+    assert launch(int(bt), m, n, k, ap, bp, Cd.data_ptr(), 0.5, 0.25, Bd.data_ptr(), 3, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(Cd[m * n:], C0[m * n:])
+    a[1] = 0
+    ref = 0.5 * (a.astype(np.float64) @ (b.T if bt else b)) + 0.25 * C0[:m * n].cpu().numpy().reshape(m, n) + bias
+    ref = np.maximum(ref, 0.0)
+    got = Cd[:m * n].cpu().numpy().reshape(m, n)
+    # at most k + 4 roundings of partial sums that grow like sqrt(k) (|a b| <= 1): 2^-24 (k + 4) 4 sqrt(k)
+    bad = ~(np.abs(got - ref) <= 2.0 ** -24 * (k + 4) * 4 * np.sqrt(k))
+    bad[1] = False
+    assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
