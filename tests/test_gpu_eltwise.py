@@ -162,3 +162,21 @@ def test_run_model_layernorm_affine_device(gpu, strict):
         mdl.close()
         assert rc == 0 and st.execution_path.decode().startswith("hip_native"), st.execution_path
         assert rel_max_err(got, ref) <= tol
+
+
+def test_wrappers_follow_the_current_stream(gpu):
+    """The wrappers launch on torch's current stream: the default one, the one
+    of a stream context, each thread's own, and the one given."""
+    import threading
+    torch = gpu
+    side = torch.cuda.Stream()
+    assert pyc_amd._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert pyc_amd._stream(None) == side.cuda_stream
+        seen = []
+        t = threading.Thread(target=lambda: seen.append(pyc_amd._stream(None)))
+        t.start()
+        t.join()
+        assert seen == [torch.cuda.default_stream().cuda_stream]
+    assert pyc_amd._stream(None) == torch.cuda.current_stream().cuda_stream
+    assert pyc_amd._stream(side.cuda_stream) == side.cuda_stream
