@@ -509,6 +509,109 @@ w8a16_lds_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ Wq,
 
 
 // ---------------------------------------------------------------------------
+// One to four tokens: a weight byte feeds so few products that the matrix units
+// do not matter and any lane can take any weight. Each wave owns R whole rows:
+// a load instruction moves 1 KiB of one row (64 lanes x 16 consecutive k), the
+// next one the following KiB, so lines are fetched whole and in order, and no
+// row is split over workgroups: no partials, no counters, no workspace, and the
+// launch ends when the weight stream does. X (all M tokens, zeros past K) sits
+// in LDS as bf16; a lane reads its 16 k of each token once for all R rows, and
+// v_dot2_f32_bf16 multiplies pairs (exact products, fp32 sums). The lanes' sums
+// meet in a butterfly at the end. Two batches of kTokBatch KiB per row are in
+// flight per wave. Bound: the weight stream (HBM).
+constexpr int kTokBatch = 4;
+constexpr int kTokWaves = 8;
+constexpr size_t kTokLdsMax = 64 * 1024;
+
+typedef __attribute__((ext_vector_type(2))) __bf16 w8_bf16x2;
+__device__ inline float w8_dot16(const u32x4& w, const u32x4& x0, const u32x4& x1, float acc) {
+    const u32x4 a = fp8x8_to_bf16x8(w[0], w[1]), b = fp8x8_to_bf16x8(w[2], w[3]);
+    // (elements copied out first: a bit cast of a vector element read element 0)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t wi = i < 4 ? a[i] : b[i - 4], xi = i < 4 ? x0[i] : x1[i - 4];
+        acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(w8_bf16x2, wi), __builtin_bit_cast(w8_bf16x2, xi), acc,
+                                              false);
+    }
+    return acc;
+}
+
+template <int M, int R>
+__global__ void __launch_bounds__(kTokWaves * kWave)
+w8a16_token_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ Wq, const float* __restrict__ scale,
+                   uint16_t* __restrict__ Y, int N, int K, int relu) {
+    extern __shared__ __attribute__((aligned(16))) u32x4 xs[];  // M rows of kpad / 8 chunks
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = (blockIdx.x * kTokWaves + wave) * R;
+    const int np = K / 16;                                      // 16-k pieces of a row
+    const int nchunk = (np + kWave - 1) / kWave;                // KiB of a row
+    const uint8_t* row[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) row[r] = Wq + (size_t)min(n0 + r, N - 1) * K;
+    // piece `lane` of chunk c; lanes past the row's end repeat its last piece (against zeros of X)
+    auto load = [&](int c, u32x4 (&w)[R]) {
+        const int p = min(c * kWave + lane, np - 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row[r] + (size_t)p * 16));
+    };
+    u32x4 w[2][kTokBatch][R];
+#pragma unroll
+    for (int b = 0; b < kTokBatch; ++b) load(b, w[0][b]);
+    const int xch = nchunk * kWave * 2;                         // 8-k chunks of a padded token
+    for (int i = tid; i < M * xch; i += kTokWaves * kWave) {
+        const int m = i / xch, c = i - m * xch;
+        // the two 8-k halves of a KiB's 64 pieces in planes of 64 chunks (conflict-free reads)
+        const int p = c >> 1;
+        xs[m * xch + ((p / kWave) * 2 + (c & 1)) * kWave + p % kWave] =
+            c * 8 < K ? *reinterpret_cast<const u32x4*>(X + (size_t)m * K + c * 8) : u32x4{0, 0, 0, 0};
+    }
+    __syncthreads();
+
+    float acc[M][R];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[m][r] = 0.f;
+    for (int c0 = 0; c0 < nchunk; c0 += 2 * kTokBatch) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int c = c0 + u * kTokBatch;
+            if (c + kTokBatch < nchunk) {  // uniform
+#pragma unroll
+                for (int b = 0; b < kTokBatch; ++b) load(c + kTokBatch + b, w[u ^ 1][b]);
+            }
+#pragma unroll
+            for (int b = 0; b < kTokBatch; ++b) {
+                if (c + b < nchunk) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m) {
+                        const u32x4* x = xs + m * xch + (c + b) * 2 * kWave + lane;
+                        const u32x4 x0 = x[0], x1 = x[kWave];
+#pragma unroll
+                        for (int r = 0; r < R; ++r) acc[m][r] = w8_dot16(w[u][b][r], x0, x1, acc[m][r]);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float v = acc[m][r];
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+            if (lane == m * R + r && n0 + r < N) {
+                float y = v * scale[n0 + r];
+                if (relu) y = y > 0.f ? y : 0.f;
+                Y[(size_t)m * N + n0 + r] = elem<bf16_t>::from_f32(y);
+            }
+        }
+}
+
+// ---------------------------------------------------------------------------
 // Whole decode chain in one persistent launch. A chain is a sequence of
 // steps Y_s = relu_s?(scale_s * X_s W_s^T) with X_{s+1} = Y_s, all with M <= 32
 // tokens, K % 128 == 0 and N % 64 == 0. One workgroup per CU walks every step:
@@ -1040,6 +1143,33 @@ extern "C" int pyc_hip_w8a16_launch(int M, int N, int K, const void* X, const vo
                                     int relu, void* Y, void* stream) {
     using namespace pyc;
     hipStream_t s = (hipStream_t)stream;
+    // Up to four tokens whose X fits the token kernel's LDS: two rows per wave
+    // where that still gives every CU a workgroup, else one. In us, split-K
+    // kernel / token kernel, [N,K] 4096 x 11008: 19.4 / 11.1 (one token), 19.5 /
+    // 12.7 (two); 8192 deep 14.9 / 11.9 (four); 11008 x 4096: 18.3 / 9.7 (one),
+    // 18.6 / 16.7 (four); 14336 x 14336: 53 / 33 (6.2 TB/s); 1024 x 1024: 7.9 / 2.7.
+    const size_t xbytes = (size_t)M * ((K / 16 + kWave - 1) / kWave) * kWave * 32;
+    if (M <= 4 && xbytes <= kTokLdsMax) {
+        const int r = N >= 2 * kTokWaves * 256 ? 2 : 1;
+        const dim3 grid((N + r * kTokWaves - 1) / (r * kTokWaves)), block(kTokWaves * kWave);
+#define PYC_TOK(MM)                                                                                             \
+    do {                                                                                                        \
+        if (r == 2)                                                                                             \
+            hipLaunchKernelGGL((w8a16_token_kernel<MM, 2>), grid, block, xbytes, s, (const uint16_t*)X,         \
+                               (const uint8_t*)Wq, scale, (uint16_t*)Y, N, K, relu);                            \
+        else                                                                                                    \
+            hipLaunchKernelGGL((w8a16_token_kernel<MM, 1>), grid, block, xbytes, s, (const uint16_t*)X,         \
+                               (const uint8_t*)Wq, scale, (uint16_t*)Y, N, K, relu);                            \
+    } while (0)
+        switch (M) {
+            case 1: PYC_TOK(1); break;
+            case 2: PYC_TOK(2); break;
+            case 3: PYC_TOK(3); break;
+            default: PYC_TOK(4); break;
+        }
+#undef PYC_TOK
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    }
     W8Plan p = w8_plan(N, K, cu_count());
     float* part = nullptr;
     int* cnt = nullptr;
