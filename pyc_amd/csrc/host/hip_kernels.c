@@ -26,12 +26,14 @@ int pyc_hip_gemm_half_launch(int is_bf16, int b_trans, int tile, int M, int N, i
                              const void* A, const void* B, void* C, float alpha, float beta,
                              const float* bias, int epi, void* stream);
 int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
-                              const void* B, void* C, float alpha, float beta, const float* bias, int epi,
-                              void* stream);
+                              const void* B, void* C, float alpha, float beta, const float* bias, int epi, int m0,
+                              int m1, int n0, int n1, void* stream);
 int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C,
-                               float alpha, float beta, const float* bias, int epi, void* stream);
+                               float alpha, float beta, const float* bias, int epi, int m_end, int n_end,
+                               void* stream);
 int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N, int K, const void* A, const void* B, void* C,
-                               float alpha, float beta, const float* bias, int epi, void* stream);
+                               float alpha, float beta, const float* bias, int epi, int m_end, int n_end,
+                               void* stream);
 int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A, const void* B,
                             void* C, float alpha, float beta, const float* bias, int epi,
                             void* stream);
@@ -39,7 +41,7 @@ int pyc_hip_attention_launch(int is_bf16, int B, int H, int S, int D, int causal
                              const void* K, const void* V, void* O, float scale, void* stream);
 int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg, int H, int W, int C, int Kout, int R, int S,
                                 int ph, int pw, int sh, int sw, const void* x, const void* w, const float* bias,
-                                int relu, void* y, void* stream);
+                                int relu, void* y, int m0, int m1, void* stream);
 int pyc_hip_conv2d_persist_launch(int is_bf16, int tail, int Nimg, int H, int W, int C, int Kout, int R, int S, int ph,
                                   int pw, int sh, int sw, const void* x, const void* w, const float* bias, int relu,
                                   void* y, void* stream);
@@ -235,12 +237,12 @@ typedef struct {
     double launch, round, stage[2], many;
 } dma_tile;
 
-enum { DT_32 = 0, DT_64, DT_128, DT_128X256, DT_256, DT_COUNT };
+enum { DT_32 = 0, DT_64, DT_128X64, DT_128, DT_128X256, DT_256, DT_COUNT };
 
 static const dma_tile k_dma_tiles[DT_COUNT] = {
-    {32, 32, 1.0, 2.0, {0.085, 0.15}, 1.0},   {64, 64, 1.0, 2.2, {0.17, 0.19}, 1.4},
-    {128, 128, 1.0, 4.2, {0.34, 0.52}, 1.1},  {128, 256, 1.0, 7.0, {0.57, 0.90}, 1.15},
-    {256, 256, 7.5, 2.0, {1.12, 1.50}, 0.93},
+    {32, 32, 1.0, 2.0, {0.085, 0.15}, 1.0},  {64, 64, 1.0, 2.2, {0.17, 0.19}, 1.4},
+    {128, 64, 1.0, 3.0, {0.25, 0.33}, 1.2},  {128, 128, 1.0, 4.2, {0.34, 0.52}, 1.1},
+    {128, 256, 1.0, 7.0, {0.57, 0.90}, 1.15}, {256, 256, 7.5, 2.0, {1.12, 1.50}, 0.93},
 };
 
 /* `k_rows`: B stored [K,N]; the 32 x 32 tile reads half lines of it, which costs
@@ -264,8 +266,8 @@ static double dma_tile_cost(int t, long M, long N, long K, int k_rows, int tail)
     return d->launch + rounds * (d->round + (double)((K + 63) / 64) * stage);
 }
 
-/* The cheapest of the tiles 0 .. last. */
-static int pick_dma_tile(long M, long N, long K, int k_rows, int tail, int last) {
+/* The cheapest of the tiles 0 .. last, and its cost. */
+static int pick_dma_tile(long M, long N, long K, int k_rows, int tail, int last, double* cost) {
     int t, best = 0;
     double c, cb = dma_tile_cost(0, M, N, K, k_rows, tail);
     for (t = 1; t <= last; ++t) {
@@ -275,7 +277,59 @@ static int pick_dma_tile(long M, long N, long K, int k_rows, int tail, int last)
             best = t;
         }
     }
+    *cost = cb;
     return best;
+}
+
+/* A product in one launch, or in two: whole rounds of one tile per CU on rows
+ * 0 .. m_end - 1 and columns 0 .. n_end - 1 (one of them all of C's), and the
+ * rest on a smaller tile that fits its last round better. */
+typedef struct {
+    int t, rest; /* tiles; rest < 0: one launch */
+    int m_end, n_end;
+} dma_plan;
+
+static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_only, int first_split, int last) {
+    dma_plan p = {0, -1, M, N};
+    double best;
+    int t;
+    p.t = pick_dma_tile(M, N, K, k_rows, tail, last, &best);
+    for (t = DT_128; t <= last && t <= first_split; ++t) {
+        const dma_tile* d = &k_dma_tiles[t];
+        const long tm = (M + d->bm - 1) / d->bm, tn = (N + d->bn - 1) / d->bn;
+        const long full = tm * tn / 256 * 256;
+        int by_n;
+        if (full == 0 || full == tm * tn) {
+            continue;
+        }
+        for (by_n = rows_only ? 0 : 1; by_n >= 0; --by_n) {
+            const long part = by_n ? full / tm : full / tn; /* tile columns or rows of the first launch */
+            long m1 = M, n1 = N;
+            double c;
+            int r;
+            if (part == 0) {
+                continue;
+            }
+            if (by_n) {
+                n1 = part * d->bn;
+            } else {
+                m1 = part * d->bm;
+            }
+            if (m1 > M || n1 > N || (m1 == M && n1 == N)) {
+                continue;
+            }
+            r = pick_dma_tile(by_n ? M : M - m1, by_n ? N - n1 : N, K, k_rows, 0, t - 1, &c);
+            c += dma_tile_cost(t, m1, n1, K, k_rows, 0);
+            if (c < 0.97 * best) {
+                best = c;
+                p.t = t;
+                p.rest = r;
+                p.m_end = (int)m1;
+                p.n_end = (int)n1;
+            }
+        }
+    }
+    return p;
 }
 
 static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, const void* B,
@@ -298,8 +352,10 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
     if (v->tile == -1) {
         const int bf = v->dtype == VT_BF16;
         const int rc = v->b_trans
-                           ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
-                           : pyc_hip_gemm_nn_lds_launch(bf, 0, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
+                           ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, M, N,
+                                                        stream)
+                           : pyc_hip_gemm_nn_lds_launch(bf, 0, M, N, K, A, B, C, alpha, beta, bias, epilogue, M, N,
+                                                        stream);
         if (rc != 1) {
             return rc;
         }
@@ -318,23 +374,31 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
         const int off16 = (int)(((uintptr_t)A | (uintptr_t)B) & 15) != 0;
         int last = off16 && pick_half_tile(M, N) != 256 ? DT_128X256 : DT_256;
         for (; last >= DT_128; --last) {
-            const int t = pick_dma_tile(M, N, K, !v->b_trans, 0, last);
+            const dma_plan p = plan_dma(M, N, K, !v->b_trans, 0, 0, last, last);
+            const dma_tile* d = &k_dma_tiles[p.t];
             int rc;
-            if (t == DT_256) {
-                rc = v->b_trans
-                         ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream)
-                         : pyc_hip_gemm_nn_lds_launch(bf, 1, M, N, K, A, B, C, alpha, beta, bias, epilogue, stream);
+            if (p.t == DT_256) {
+                rc = v->b_trans ? pyc_hip_gemm_nt_lds_launch(bf, M, N, K, A, B, C, alpha, beta, bias, epilogue, p.m_end,
+                                                             p.n_end, stream)
+                                : pyc_hip_gemm_nn_lds_launch(bf, 1, M, N, K, A, B, C, alpha, beta, bias, epilogue,
+                                                             p.m_end, p.n_end, stream);
             } else {
-                rc = pyc_hip_gemm_small_launch(bf, v->b_trans, k_dma_tiles[t].bm, k_dma_tiles[t].bn, M, N, K, A, B, C,
-                                               alpha, beta, bias, epilogue, stream);
+                rc = pyc_hip_gemm_small_launch(bf, v->b_trans, d->bm, d->bn, M, N, K, A, B, C, alpha, beta, bias,
+                                               epilogue, 0, p.m_end, 0, p.n_end, stream);
+            }
+            if (rc == 0 && p.rest >= 0) {
+                d = &k_dma_tiles[p.rest];
+                rc = pyc_hip_gemm_small_launch(bf, v->b_trans, d->bm, d->bn, M, N, K, A, B, C, alpha, beta, bias,
+                                               epilogue, p.m_end < M ? p.m_end : 0, M, p.n_end < N ? p.n_end : 0, N,
+                                               stream);
             }
             if (rc != 1) {
                 return rc;
             }
-            if (t < DT_128X256) {
+            if (p.t < DT_128X256) {
                 break;
             }
-            last = t;
+            last = p.t;
         }
     }
     return pyc_hip_gemm_half_launch(v->dtype == VT_BF16, v->b_trans, v->tile > 0 ? v->tile : pick_half_tile(M, N),
@@ -399,18 +463,29 @@ int pyc_hip_conv2d_dispatch(const char* symbol, int N, int H, int W, int C_in, i
         const int bf = v->dtype == VT_BF16;
         const long P = (H + 2L * pad_h - R) / stride_h + 1, Q = (W + 2L * pad_w - S) / stride_w + 1;
         const long Mg = (long)N * P * Q, Kg = (long)R * S * C_in;
-        int rc = 1, t = pick_dma_tile(Mg, K, Kg, 0, 1, DT_256);
-        if (t == DT_256) {
-            rc = pyc_hip_conv2d_persist_launch(bf, 1, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h, stride_w, x, w,
-                                               bias, relu ? 1 : 0, y, stream);
-            t = pick_dma_tile(Mg, K, Kg, 0, 1, DT_128X256);
-        }
-        if (rc == 1) {
-            rc = pyc_hip_conv2d_small_launch(bf, k_dma_tiles[t].bm, k_dma_tiles[t].bn, N, H, W, C_in, K, R, S, pad_h,
-                                             pad_w, stride_h, stride_w, x, w, bias, relu ? 1 : 0, y, stream);
-        }
-        if (rc != 1) {
-            return rc;
+        if (Mg <= 0x7FFFFF00L && Kg <= 0x7FFFFF00L) {
+            dma_plan p = plan_dma((int)Mg, K, Kg, 0, 1, 1, DT_128X256, DT_256);
+            int rc = 1;
+            if (p.t == DT_256) {
+                rc = pyc_hip_conv2d_persist_launch(bf, 1, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h, stride_w, x,
+                                                   w, bias, relu ? 1 : 0, y, stream);
+                if (rc == 1) {
+                    p = plan_dma((int)Mg, K, Kg, 0, 0, 1, DT_128X256, DT_128X256);
+                }
+            }
+            if (rc == 1) {
+                rc = pyc_hip_conv2d_small_launch(bf, k_dma_tiles[p.t].bm, k_dma_tiles[p.t].bn, N, H, W, C_in, K, R, S,
+                                                 pad_h, pad_w, stride_h, stride_w, x, w, bias, relu ? 1 : 0, y, 0,
+                                                 p.m_end, stream);
+                if (rc == 0 && p.rest >= 0) {
+                    rc = pyc_hip_conv2d_small_launch(bf, k_dma_tiles[p.rest].bm, k_dma_tiles[p.rest].bn, N, H, W, C_in,
+                                                     K, R, S, pad_h, pad_w, stride_h, stride_w, x, w, bias,
+                                                     relu ? 1 : 0, y, p.m_end, (int)Mg, stream);
+                }
+            }
+            if (rc != 1) {
+                return rc;
+            }
         }
     }
     return pyc_hip_conv2d_launch(v->dtype == VT_BF16, v->tile, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h,

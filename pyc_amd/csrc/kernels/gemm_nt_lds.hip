@@ -867,8 +867,8 @@ static bool ragged_ok(int M, int N, int K, const void* A, const void* B, const v
 
 template <bool BNN>
 static int launch_ragged(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C, float alpha,
-                         const float* bias, int epi, int n_cu, hipStream_t s) {
-    const int tiles_m = (M + kD_BM - 1) / kD_BM, tiles_n = (N + kD_BN - 1) / kD_BN;
+                         const float* bias, int epi, int m_end, int n_end, int n_cu, hipStream_t s) {
+    const int tiles_m = (m_end + kD_BM - 1) / kD_BM, tiles_n = (n_end + kD_BN - 1) / kD_BN;
     const int ntiles = tiles_m * tiles_n;
     const int pepi = (((epi & 1) && bias != nullptr) ? 1 : 0) | (epi & 2);
     const dim3 grid(ntiles < n_cu ? ntiles : n_cu), block(4 * kWave);
@@ -895,15 +895,17 @@ static int launch_ragged(int is_bf16, int M, int N, int K, const void* A, const 
 
 }  // namespace pyc
 
+// Rows 0 .. m_end - 1 and columns 0 .. n_end - 1 of C (each whole tiles, or all).
 // Returns 1 when the shape is outside these kernels' preconditions (the caller
 // uses another variant), 0 on launch, -2 on a launch error. Full-tile shapes
 // with beta == 0 take the persistent kernel; PYC_GEMM_NT_PERSIST=0 forces the
 // one-shot kernel (for comparisons).
 extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B,
-                                          void* C, float alpha, float beta, const float* bias, int epi,
-                                          void* stream) {
+                                          void* C, float alpha, float beta, const float* bias, int epi, int m_end,
+                                          int n_end, void* stream) {
     using namespace pyc;
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 1;
+    if (m_end <= 0 || m_end > M || n_end <= 0 || n_end > N) return 1;
     // buffer descriptors hold 32-bit byte counts
     if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
     static int persist_env = -1;
@@ -920,11 +922,12 @@ extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, cons
         else
             n_cu = 256;
     }
-    const int tiles_m = (M + kD_BM - 1) / kD_BM;
-    const int tiles_n = (N + kD_BN - 1) / kD_BN;
+    const int tiles_m = (m_end + kD_BM - 1) / kD_BM;
+    const int tiles_n = (n_end + kD_BN - 1) / kD_BN;
     const int ntiles = tiles_m * tiles_n;
     if (persist_env && (M % kD_BM || N % kD_BN) && ragged_ok(M, N, K, A, B, C, beta, bias, epi))
-        return launch_ragged<false>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, n_cu, (hipStream_t)stream);
+        return launch_ragged<false>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, m_end, n_end, n_cu,
+                                    (hipStream_t)stream);
     const bool persist = persist_env && M % kD_BM == 0 && N % kD_BN == 0 && beta == 0.f &&
                          ((uintptr_t)C & 15) == 0 && ((epi & 1) == 0 || bias == nullptr || ((uintptr_t)bias & 15) == 0);
     hipStream_t s = (hipStream_t)stream;
@@ -969,9 +972,10 @@ extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, cons
 // first, and any number of tiles), 0 on launch, -2 on a launch error.
 extern "C" int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N, int K, const void* A,
                                           const void* B, void* C, float alpha, float beta, const float* bias,
-                                          int epi, void* stream) {
+                                          int epi, int m_end, int n_end, void* stream) {
     using namespace pyc;
     if (M <= 0 || N <= 0 || K <= 0 || beta != 0.f) return 1;
+    if (m_end <= 0 || m_end > M || n_end <= 0 || n_end > N) return 1;
     const bool whole = M % kD_BM == 0 && N % kD_BN == 0 && K % 64 == 0;
     if (!whole && !(ragged && ragged_ok(M, N, K, A, B, C, beta, bias, epi))) return 1;
     if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
@@ -985,11 +989,12 @@ extern "C" int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N,
         else
             n_cu = 256;
     }
-    const int tiles_m = (M + kD_BM - 1) / kD_BM, tiles_n = (N + kD_BN - 1) / kD_BN;
+    const int tiles_m = (m_end + kD_BM - 1) / kD_BM, tiles_n = (n_end + kD_BN - 1) / kD_BN;
     const int ntiles = tiles_m * tiles_n;
     // the symbol that names this kernel alone takes no fewer tiles than CUs
     if (!ragged && ntiles < n_cu) return 1;
-    if (!whole) return launch_ragged<true>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, n_cu, (hipStream_t)stream);
+    if (!whole) return launch_ragged<true>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, m_end, n_end, n_cu,
+                                    (hipStream_t)stream);
     hipStream_t s = (hipStream_t)stream;
     const int pepi = (((epi & 1) && bias != nullptr) ? 1 : 0) | (epi & 2);
     const dim3 grid(ntiles < n_cu ? ntiles : n_cu), block(4 * kWave);

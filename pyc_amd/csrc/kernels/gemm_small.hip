@@ -87,7 +87,7 @@ template <typename T, bool BT, int BM, int BN, int KS, int SRC>
 __global__ void __launch_bounds__(512, SRC == kAny && BM < 128 ? 4 : 2)
 gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C,
                   int M, int N, int K, float alpha, float beta, const float* __restrict__ bias, int epi,
-                  int tiles_n, int vec_c, SmConv cg) {
+                  int tiles_m, int tiles_n, int m_base, int n_base, int vec_c, SmConv cg) {
     constexpr uint32_t A_BYTES = BM * 128, B_BYTES = BN * 128;  // one stage: 64 k of BM and of BN rows
     constexpr uint32_t STAGE_BYTES = A_BYTES + B_BYTES;
     constexpr uint32_t SLOT_BYTES = KS * STAGE_BYTES;
@@ -114,15 +114,14 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     const int wm = quad >> 1, wn = quad & 1;
     const int lrow = lane & 15, lgrp = lane >> 4;
     // tiles in groups of 4 tile rows, column by column (neighbouring workgroups share B columns)
-    const int tiles_m = (M + BM - 1) / BM;
     const int gm = tiles_m < 4 ? tiles_m : 4;
     const int span = gm * tiles_n;
     const int grp = blockIdx.x / span;
     const int first_m = grp * gm;
     const int gsz = min(tiles_m - first_m, gm);
     const int in = blockIdx.x - grp * span;
-    const int m0 = (first_m + in % gsz) * BM;
-    const int n0 = (in / gsz) * BN;
+    const int m0 = m_base + (first_m + in % gsz) * BM;
+    const int n0 = n_base + (in / gsz) * BN;
     const int KT = (K + kSmBK - 1) / kSmBK;
 
     const i32x4 ra = make_buf_rsrc(A, SRC == kConv ? cg.x_bytes : (uint32_t)((size_t)M * K * 2));
@@ -455,11 +454,18 @@ gemm_small_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     }
 }
 
+// The part of C a launch computes: rows m0 .. m1 - 1, columns n0 .. n1 - 1 (both
+// ends whole tiles from the start, or the end of C).
+struct SmPart {
+    int m0, m1, n0, n1;
+};
+
 template <typename T, bool BT, int SRC>
 static int launch_small(int bm, int bn, int M, int N, int K, const void* A, const void* B, void* C, float alpha,
-                        float beta, const float* bias, int epi, hipStream_t s, const SmConv& cg) {
-    const int tiles_n = (N + bn - 1) / bn;
-    const long tiles = (long)((M + bm - 1) / bm) * tiles_n;
+                        float beta, const float* bias, int epi, const SmPart& pt, hipStream_t s, const SmConv& cg) {
+    if (pt.m0 < 0 || pt.m0 >= pt.m1 || pt.m1 > M || pt.n0 < 0 || pt.n0 >= pt.n1 || pt.n1 > N) return 1;
+    const int tiles_m = (pt.m1 - pt.m0 + bm - 1) / bm, tiles_n = (pt.n1 - pt.n0 + bn - 1) / bn;
+    const long tiles = (long)tiles_m * tiles_n;
     if (tiles > 0x7FFFFFFFL) return 1;
     const dim3 grid((unsigned)tiles), block(8 * kWave);
     const uint16_t* a = (const uint16_t*)A;
@@ -468,9 +474,10 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
     const int vec_c = N % 4 == 0 && ((uintptr_t)C & 7) == 0;
 #define PYC_SMALL(BM, BN, KS)                                                                                  \
     hipLaunchKernelGGL((gemm_small_kernel<T, BT, BM, BN, KS, SRC>), grid, block, 0, s, a, b, c, M, N, K, alpha, \
-                       beta, bias, epi, tiles_n, vec_c, cg)
+                       beta, bias, epi, tiles_m, tiles_n, pt.m0, pt.n0, vec_c, cg)
     if (bm == 32 && bn == 32) PYC_SMALL(32, 32, 4);
     else if (bm == 64 && bn == 64) PYC_SMALL(64, 64, 2);
+    else if (bm == 128 && bn == 64) PYC_SMALL(128, 64, 1);
     else if (bm == 128 && bn == 128) PYC_SMALL(128, 128, 1);
     else if constexpr (SRC != kAny) {
         if (bm == 128 && bn == 256) PYC_SMALL(128, 256, 1);
@@ -482,7 +489,7 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
 
 }  // namespace pyc
 
-// bm x bn: one of the tiles above. Rows of A (and of [N,K] B) past the end are
+// bm x bn: one of the tiles above; m0 .. n1: the part of C (SmPart). Rows of A (and of [N,K] B) past the end are
 // read as zeros through the buffer descriptors, [K,N] B columns past N read
 // neighbouring data, and only the rows and columns of C inside M x N are
 // written. LDS-DMA takes K a multiple of 8 and, for [K,N] B, N of 4, with A and
@@ -492,9 +499,10 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
 // rows, 0 on launch, -2 on a launch error.
 extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
                                          const void* B, void* C, float alpha, float beta, const float* bias,
-                                         int epi, void* stream) {
+                                         int epi, int m0, int m1, int n0, int n1, void* stream) {
     using namespace pyc;
     if (M <= 0 || N <= 0 || K <= 0) return 1;
+    const SmPart pt{m0, m1, n0, n1};
     const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
     const bool tail = K % kSmBK != 0;
     const bool any = K % 8 || (!b_trans && N % 4) || (((uintptr_t)A | (uintptr_t)B) & 15) ||
@@ -504,21 +512,23 @@ extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int b
     hipStream_t s = (hipStream_t)stream;
     const SmConv cg{};
 #define PYC_GO(TY, BT)                                                                                              \
-    (any    ? launch_small<TY, BT, kAny>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                   \
-     : tail ? launch_small<TY, BT, kTail>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg)                  \
-            : launch_small<TY, BT, kDense>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, s, cg))
+    (any    ? launch_small<TY, BT, kAny>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, pt, s, cg)                   \
+     : tail ? launch_small<TY, BT, kTail>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, pt, s, cg)                  \
+            : launch_small<TY, BT, kDense>(bm, bn, M, N, K, A, B, C, alpha, beta, bias, epi, pt, s, cg))
     if (is_bf16) return b_trans ? PYC_GO(bf16_t, true) : PYC_GO(bf16_t, false);
     return b_trans ? PYC_GO(f16_t, true) : PYC_GO(f16_t, false);
 #undef PYC_GO
 }
 
-// NHWC convolution on the same tiles (bm output pixels x bn output channels).
+// NHWC convolution on the same tiles (bm output pixels x bn output channels),
+// output pixels m0 .. m1 - 1.
 // Returns 1 outside its preconditions (C % 8 == 0, x and w 16-byte aligned and
 // below 4 GiB, reciprocals exact: R*S*C * C < 2^32), 0 on launch, -2 on a
 // launch error.
 extern "C" int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg, int H, int W, int C, int Kout,
                                            int R, int S, int ph, int pw, int sh, int sw, const void* x,
-                                           const void* w, const float* bias, int relu, void* y, void* stream) {
+                                           const void* w, const float* bias, int relu, void* y, int m0, int m1,
+                                           void* stream) {
     using namespace pyc;
     const long long P = (H + 2LL * ph - R) / sh + 1, Q = (W + 2LL * pw - S) / sw + 1;
     const long long M = (long long)Nimg * P * Q, Kg = (long long)R * S * C;
@@ -531,11 +541,14 @@ extern "C" int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg
     const SmConv cg{H, W, C, S, (int)P, (int)Q, ph, pw, sh, sw, (uint32_t)(((1ull << 32) + C - 1) / C),
                     S == 1 ? 0u : (uint32_t)(((1ull << 32) + S - 1) / S),
                     (uint32_t)((size_t)Nimg * H * W * C * 2)};
+    const SmPart pt{m0, m1 > 0 ? m1 : (int)M, 0, Kout};  // m1 <= 0: to the last pixel
     const int epi = (bias ? 1 : 0) | (relu ? 2 : 0);
     hipStream_t st = (hipStream_t)stream;
     if (is_bf16)
-        return launch_small<bf16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, st, cg);
-    return launch_small<f16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, st, cg);
+        return launch_small<bf16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, pt, st,
+                                                 cg);
+    return launch_small<f16_t, true, kConv>(bm, bn, (int)M, Kout, (int)Kg, x, w, y, 1.0f, 0.0f, bias, epi, pt, st,
+                                                 cg);
 }
 
 // Registry figures: the ring allows one 8-wave workgroup per CU.

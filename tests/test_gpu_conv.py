@@ -185,7 +185,7 @@ def test_conv_unaligned_bias_takes_general_kernel(gpu):
     assert d <= 2e-2 * Y2.float().abs().max().item()
 
 
-@pytest.mark.parametrize("bm,bn", [(32, 32), (64, 64), (128, 128), (128, 256)])
+@pytest.mark.parametrize("bm,bn", [(32, 32), (64, 64), (128, 64), (128, 128), (128, 256)])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("N,H,W,C,K,R,S,pad,stride", [
     (2, 9, 7, 8, 33, 3, 3, (1, 1), (1, 1)),     # 8 channels: a stage spans 8 taps, one odd output channel
@@ -208,9 +208,10 @@ def test_conv_lds_tiles(gpu, bm, bn, dt, N, H, W, C, K, R, S, pad, stride):
     Bd = dev_f32(torch, bias)
     Y = torch.full((N * P * Q * K + 512,), 7.0, dtype=tdt, device="cuda")
     launch = pyc_amd.lib().pyc_hip_conv2d_small_launch
-    launch.argtypes = [ctypes.c_int] * 14 + [ctypes.c_void_p] * 3 + [ctypes.c_int] + [ctypes.c_void_p] * 2
+    launch.argtypes = ([ctypes.c_int] * 14 + [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_void_p] +
+                       [ctypes.c_int] * 2 + [ctypes.c_void_p])
     assert launch(int(dt == "bf16"), bm, bn, N, H, W, C, K, R, S, pad[0], pad[1], stride[0], stride[1], X.data_ptr(),
-                  Wd.data_ptr(), Bd.data_ptr(), 1, Y.data_ptr(), None) == 0
+                  Wd.data_ptr(), Bd.data_ptr(), 1, Y.data_ptr(), 0, N * P * Q, None) == 0
     torch.cuda.synchronize()
     assert bool((Y[N * P * Q * K:] == 7.0).all())
     ref = oracle.conv2d_nhwc_f32(X.float().cpu().numpy(), Wd.float().cpu().numpy(), bias, pad, stride, relu=True)

@@ -424,7 +424,7 @@ def test_ragged_persistent_gemm(gpu, m, n, k, epi, layout, dtype):
     assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
 
 
-LDS_TILES = [(32, 32), (64, 64), (128, 128), (128, 256)]
+LDS_TILES = [(32, 32), (64, 64), (128, 64), (128, 128), (128, 256)]
 
 
 @pytest.mark.parametrize("bm,bn", LDS_TILES)
@@ -452,9 +452,9 @@ def test_lds_tiles_ragged(gpu, bm, bn, layout, dtype, k, beta, epi):
     Cd = C0.clone()
     L = pyc_amd.lib()
     launch = L.pyc_hip_gemm_small_launch
-    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p, C.c_int, C.c_void_p]
+    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p] + [C.c_int] * 5 + [C.c_void_p]
     assert launch(int(dtype == "bf16"), int(bt), bm, bn, m, n, k, A.data_ptr(), B.data_ptr(), Cd.data_ptr(), 0.75,
-                  beta, bias.data_ptr(), epi, None) == 0
+                  beta, bias.data_ptr(), epi, 0, m, 0, n, None) == 0
     torch.cuda.synchronize()
     assert torch.equal(Cd[m * n:], C0[m * n:])
     a, b = A.float().cpu().numpy(), B.float().cpu().numpy()
@@ -520,9 +520,9 @@ def test_register_staged_tiles(gpu, bt, layout, dtype, dn, k, off):
     Bd = dev_f32(torch, bias)
     Cd = torch.full((m * n + 256,), 7.0, dtype=t, device="cuda")
     launch = pyc_amd.lib().pyc_hip_gemm_small_launch
-    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p, C.c_int, C.c_void_p]
-    assert launch(int(dtype == "bf16"), int(nt), bt, bt, m, n, k, ap, bp, Cd.data_ptr(), -0.5, 0.0, Bd.data_ptr(), 1,
-                  None) == 0
+    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 3 + [C.c_float] * 2 + [C.c_void_p] + [C.c_int] * 5 + [C.c_void_p]
+    assert launch(int(dtype == "bf16"), int(nt), bt, bt, m, n, k, ap, bp, Cd.data_ptr(), -0.5, 0.0, Bd.data_ptr(), 1, 0,
+                  m, 0, n, None) == 0
     torch.cuda.synchronize()
     assert bool((Cd[m * n:] == 7.0).all())
     ref = -0.5 * (a @ (b.T if nt else b)) + bias
@@ -578,3 +578,28 @@ def test_f32_ragged_tiles(gpu, m, n, k, off, layout):
     bad = ~(np.abs(got - ref) <= 2.0 ** -24 * (k + 4) * 4 * np.sqrt(k))
     bad[1] = False
     assert not bad.any(), f"{bad.sum()} elements off, first at {np.argwhere(bad)[0]}"
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("m,n,k", [(1999, 11008, 64),    # a round of 256 x 256 tiles by columns, the rest smaller
+                                   (8200, 2056, 128),    # more tile rows than columns
+                                   (3000, 3000, 72),     # rounds of 128-row tiles (K no multiple of 64), the rest
+                                   (3001, 3002, 71)])    # the same on the register-staged tiles
+def test_gemm_in_two_parts(gpu, m, n, k, layout):
+    """Products that take whole rounds of one tile and the rest of C on another:
+    every element against fp32, and nothing past C."""
+    torch = gpu
+    bt = layout == "nt"
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    A = (torch.randn((m, k), generator=g, device="cuda") / np.sqrt(k)).bfloat16()
+    B = torch.randn((n, k) if bt else (k, n), generator=g, device="cuda").bfloat16()
+    bias = torch.randn(n, generator=g, device="cuda")
+    Cd = torch.full((m * n + 4096,), 7.0, dtype=torch.bfloat16, device="cuda")
+    pyc_amd.gemm(f"hip_gemm_bf16_{layout}", A, B, Cd, m, n, k, bias=bias, epilogue=1)
+    torch.cuda.synchronize()
+    assert bool((Cd[m * n:] == 7.0).all())
+    ref = A.float() @ (B.float().t() if bt else B.float()) + bias
+    # one rounding of the result (2^-8 relative) plus fp32 summation order
+    bad = ~((Cd[:m * n].view(m, n).float() - ref).abs() <=
+            2.0 ** -8 * ref.abs() + 4e-6 * np.sqrt(k) * ref.abs().max())
+    assert not bool(bad.any()), int(bad.sum())
