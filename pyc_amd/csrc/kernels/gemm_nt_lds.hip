@@ -349,8 +349,6 @@ gemm_nt_persist_kernel(const uint16_t* __restrict__ A, const uint16_t* __restric
     const uint32_t bs_base = (uint32_t)(uintptr_t)&Bs[0];
     const i32x4 a_rsrc = make_buf_rsrc(A, CONV ? cg.x_bytes : (uint32_t)((size_t)M * K * 2));
     const i32x4 b_rsrc = make_buf_rsrc(B, (uint32_t)((size_t)N * K * 2));
-    const __amdgpu_buffer_rsrc_t c_rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(C, 0, RAG ? (uint32_t)((size_t)M * N * 2) : 0u, 0x00020000);
     uint32_t voff[2 * LOADS];
     uint32_t ldso[2 * LOADS];
     // CONV: per A row, the pixel index of tap (0,0) (voff[j]) and the packed
@@ -575,8 +573,8 @@ gemm_nt_persist_kernel(const uint16_t* __restrict__ A, const uint16_t* __restric
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             bv[j] = has_bias ? *reinterpret_cast<const float4*>(
-                                   bias + (RAG ? min(n0 + wn * 128 + 16 * j + 4 * lgrp, N - 4)
-                                               : n0 + wn * 128 + 16 * j + 4 * lgrp))
+                                   RAG ? bias + min(n0 + wn * 128 + 16 * j + 4 * lgrp, N - 4)
+                                       : bias + n0 + wn * 128 + 16 * j + 4 * lgrp)
                              : float4{0.f, 0.f, 0.f, 0.f};
 
         const int cm0 = m0, cn0 = n0;
@@ -621,6 +619,8 @@ gemm_nt_persist_kernel(const uint16_t* __restrict__ A, const uint16_t* __restric
                 const uint4 val = *reinterpret_cast<const uint4*>(stage + r * 128 + ((lrow ^ (r & 15)) << 3));
                 const int gm = cm0 + wm * 128 + pass * STAGE_ROWS + r;
                 if constexpr (RAG) {
+                    const __amdgpu_buffer_rsrc_t c_rsrc =
+                        __builtin_amdgcn_make_buffer_rsrc(C, 0, (uint32_t)((size_t)M * N * 2), 0x00020000);
                     const int gn = cn0 + wn * 128 + lrow * 8;
                     const uint32_t off = gm < M && gn < N ? ((uint32_t)gm * (uint32_t)N + (uint32_t)gn) * 2u : kPastEnd;
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, val), c_rsrc, off, 0, 0);
