@@ -288,6 +288,105 @@ __global__ void __launch_bounds__(256) layernorm_reg_kernel(const store_t<T>* __
         }
 }
 
+// Any D from one chunk up, any alignment: W waves share a row (4 / W rows per
+// workgroup), up to CAP chunks of 16 bytes per lane in registers, loaded and
+// stored unaligned where rows are no whole chunks (the device runs with
+// unaligned access on). A row's last chunk is moved back to end with the row:
+// its first elements are then another chunk's too, so they are left out of
+// the sums, and both lanes write them the same value. Every load of a row is
+// complete before its first store (the sums need them all), so y may be x.
+// gamma and beta are loaded with the row (the row itself in place of an
+// absent one). W > 1 where one wave would need more than 8 chunks per lane,
+// and for few rows, where a row's latency is what counts.
+template <typename T, int CAP>
+__global__ void __launch_bounds__(256) layernorm_row_kernel(const store_t<T>* __restrict__ x,
+                                                            const store_t<T>* __restrict__ gamma,
+                                                            const store_t<T>* __restrict__ beta,
+                                                            store_t<T>* __restrict__ y, int rows, int D, int W,
+                                                            float eps) {
+    using IO = io<T>;
+    constexpr int V = IO::kVec;
+    __shared__ float part[2][4];
+    const int wave = threadIdx.x >> 6;
+    const int per = 4 / W, sub = wave & (W - 1);  // rows per workgroup, this wave's place in its row
+    const int own = (int)blockIdx.x * per + wave / W;
+    const bool live = own < rows;  // surplus waves only keep the barriers company: they read the last row, store nothing
+    const int row = live ? own : rows - 1;
+    const int t = sub * kWave + (threadIdx.x & 63);
+    const int n = (D + V - 1) / V, skip = n * V - D;  // chunks; elements of the last one that are another's
+    const store_t<T>* xr = x + (size_t)row * D;
+    store_t<T>* yr = y + (size_t)row * D;
+    const store_t<T>* gp = gamma ? gamma : xr;
+    const store_t<T>* bp = beta ? beta : xr;
+    auto at = [&](int j) { return min((t + j * W * kWave) * V, D - V); };  // first element of the lane's chunk j
+    auto raw = [&](const store_t<T>* p, int i) {
+        u32x4 c;
+        __builtin_memcpy(&c, p + i, 16);
+        return c;
+    };
+    u32x4 rx[CAP], rg[CAP], rb[CAP];
+#pragma unroll
+    for (int j = 0; j < CAP; ++j) rx[j] = raw(xr, at(j));
+#pragma unroll
+    for (int j = 0; j < CAP; ++j) {
+        rg[j] = raw(gp, at(j));
+        rb[j] = raw(bp, at(j));
+    }
+    // sum of f over the elements that are chunk j's own
+    auto sum = [&](auto&& f) {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < CAP; ++j) {
+            const int c = t + j * W * kWave;
+            if (c < n) {
+                float v[V];
+                IO::unpack(rx[j], v);
+                const int from = c == n - 1 ? skip : 0;
+#pragma unroll
+                for (int e = 0; e < V; ++e) s += e >= from ? f(v[e]) : 0.f;
+            }
+        }
+        return wave_sum(s);
+    };
+    auto row_sum = [&](float s, int k) {
+        if (W == 1) return s;
+        if ((threadIdx.x & 63) == 0) part[k][wave] = s;
+        __syncthreads();
+        float r = 0.f;
+        for (int w = 0; w < W; ++w) r += part[k][(wave & ~(W - 1)) + w];
+        return r;
+    };
+    const float mean = row_sum(sum([](float v) { return v; }), 0) / (float)D;
+    const float var = row_sum(sum([&](float v) { return (v - mean) * (v - mean); }), 1) / (float)D;
+    const float rstd = 1.0f / sqrtf(var + eps);
+#pragma unroll
+    for (int j = 0; j < CAP; ++j) {
+        if (live && t + j * W * kWave < n) {
+            float v[V], g[V], b[V];
+            IO::unpack(rx[j], v);
+            IO::unpack(rg[j], g);
+            IO::unpack(rb[j], b);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                float o = (v[e] - mean) * rstd;
+                if (gamma) o *= g[e];
+                if (beta) o += b[e];
+                v[e] = o;
+            }
+            u32x4 c;
+            if constexpr (V == 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c[e] = __float_as_uint(v[e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    c[e] = (uint32_t)elem<T>::from_f32(v[2 * e]) | ((uint32_t)elem<T>::from_f32(v[2 * e + 1]) << 16);
+            }
+            __builtin_memcpy(yr + at(j), &c, 16);
+        }
+    }
+}
+
 template <typename T>
 static int launch_gelu(const void* x, void* y, size_t n, hipStream_t s) {
     constexpr int V = io<T>::kVec;
@@ -301,6 +400,8 @@ static int launch_gelu(const void* x, void* y, size_t n, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+constexpr int kLnFewRows = 2048;  // fewer rows than this leave SIMDs idle at one wave each
+
 template <typename T>
 static int launch_layernorm(const void* x, const void* g, const void* b, void* y, int rows, int D, float eps,
                             hipStream_t s) {
@@ -309,6 +410,28 @@ static int launch_layernorm(const void* x, const void* g, const void* b, void* y
     const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
     const int nc = (vec && D % (V * kWave) == 0) ? D / (V * kWave) : 0;  // chunks per lane
     constexpr bool kCap16 = !std::is_same<T, f16_t>::value;  // fp16 rows past 8 chunks: three passes
+    // Few rows, or rows that are no whole chunks per lane: W waves per row. In
+    // us, one of the other two kernels / this one: 1 x 3392 bf16 6.3 / 3.5, 64 x 4096
+    // 4.9 / 3.8, 8000 x 5003 127 / 50, 6000 x 8190 187 / 46, 4000 x 6145 fp32 130 /
+    // 45, 5000 x 8192 fp16 59 / 39; 2000 x 4096 bf16 9.9 / 10.0 (so whole rows of
+    // that many stay with one wave each).
+    const int n = (D + V - 1) / V;
+    const bool whole = (nc >= 1 && nc <= 8) || (kCap16 && nc > 8 && nc <= 16);
+    if (D >= V && n <= 4 * kWave * 8 && (!whole || rows < kLnFewRows / 2)) {
+        int W = 1;
+        while (W < 4 && (n > W * kWave * 8 || ((long)rows * W < kLnFewRows && n > W * kWave))) W *= 2;
+        const int cap = (n + W * kWave - 1) / (W * kWave);
+        const dim3 g2((unsigned)(((long)rows * W + 3) / 4));
+#define PYC_LN(C)                                                                                              \
+    hipLaunchKernelGGL((layernorm_row_kernel<T, C>), g2, block, 0, s, (const store_t<T>*)x, (const store_t<T>*)g, \
+                       (const store_t<T>*)b, (store_t<T>*)y, rows, D, W, eps)
+        if (cap <= 1) PYC_LN(1);
+        else if (cap <= 2) PYC_LN(2);
+        else if (cap <= 4) PYC_LN(4);
+        else PYC_LN(8);
+#undef PYC_LN
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    }
     if (nc >= 1 && nc <= 8)
         hipLaunchKernelGGL((layernorm_reg_kernel<T, 8>), grid, block, 0, s, (const store_t<T>*)x,
                            (const store_t<T>*)g, (const store_t<T>*)b, (store_t<T>*)y, rows, D, eps);

@@ -180,3 +180,36 @@ def test_wrappers_follow_the_current_stream(gpu):
         assert seen == [torch.cuda.default_stream().cuda_stream]
     assert pyc_amd._stream(None) == torch.cuda.current_stream().cuda_stream
     assert pyc_amd._stream(side.cuda_stream) == side.cuda_stream
+
+
+@pytest.mark.parametrize("name", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,D,off", [(1, 8, 0), (5, 9, 1),        # one chunk, one element more
+                                        (3, 513, 0), (1500, 520, 3),  # a lane's second chunk; bases off 16 bytes
+                                        (7, 4095, 1), (2, 16383, 0),  # four waves a row, a moved last chunk
+                                        (1023, 1024, 0), (1024, 1024, 0),  # both sides of the few-rows rule
+                                        (3, 16400, 0)])               # more chunks than the row kernel holds (bf16)
+def test_layernorm_rows(gpu, name, rows, D, off):
+    """Rows of any length and alignment, out of place and in place, with and
+    without gamma and beta, against float64; nothing is written outside y."""
+    torch = gpu
+    t = _tdtype(torch, name)
+    g = torch.Generator(device="cuda").manual_seed(rows + D)
+    buf = torch.full((rows * D + 64,), 5.0, dtype=t, device="cuda")
+    x = buf[8 + off:8 + off + rows * D].view(rows, D)
+    x.copy_(torch.randn((rows, D), generator=g, device="cuda") * 3.0 + 5.0)
+    gb = torch.randn(2 * D + 8, generator=g, device="cuda").to(t)
+    gamma, beta = gb[off:off + D], gb[D + 1:2 * D + 1]
+    xin = x.float().cpu().numpy()
+    for ga, be in ((gamma, beta), (None, beta), (None, None)):
+        ref = oracle.layernorm_f64(xin, None if ga is None else ga.float().cpu().numpy(),
+                                   None if be is None else be.float().cpu().numpy(), 1e-5)
+        y = torch.full((rows * D + 64,), 3.0, dtype=t, device="cuda")
+        yv = y[8 + off:8 + off + rows * D].view(rows, D)
+        pyc_amd.layernorm(x, yv, ga, be)
+        torch.cuda.synchronize()
+        assert bool((y[:8 + off] == 3.0).all()) and bool((y[8 + off + rows * D:] == 3.0).all())
+        _check(yv.float().cpu().numpy(), ref, name)
+    pyc_amd.layernorm(x, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x, yv)
+    assert bool((buf[:8 + off] == 5.0).all()) and bool((buf[8 + off + rows * D:] == 5.0).all())
