@@ -518,7 +518,8 @@ w8a16_lds_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ Wq,
 // in LDS as bf16; a lane reads its 16 k of each token once for all R rows, and
 // v_dot2_f32_bf16 multiplies pairs (exact products, fp32 sums). The lanes' sums
 // meet in a butterfly at the end. Two batches of kTokBatch KiB per row are in
-// flight per wave. Bound: the weight stream (HBM).
+// flight per wave. Bound: the weight stream (HBM): [14336,14336], one token, 6.2 TB/s;
+// [4096,11008] 18.9 -> 11.1 us (split-K kernel -> this), [1024,1024] 9 -> 2.7.
 constexpr int kTokBatch = 4;
 constexpr int kTokWaves = 8;
 constexpr size_t kTokLdsMax = 64 * 1024;
@@ -609,6 +610,136 @@ w8a16_token_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W
                 Y[(size_t)m * N + n0 + r] = elem<bf16_t>::from_f32(y);
             }
         }
+}
+
+// ---------------------------------------------------------------------------
+// Up to 32 tokens without split-K: a workgroup owns 16 UB channels over the
+// whole K, so no partial leaves the CU. It reads more of X than the split
+// kernels above (all of it, from L2), but ends in one LDS reduction instead of
+// partial stores, counters and a reduction over memory (about 6 us). UB is
+// chosen so that the units fill the chip once with the fewest bytes per CU.
+// A ring slot is 256 k: 16 UB rows of 256 weight bytes and 16 TH tokens of 512
+// bytes (TH 1 up to 16 tokens), moved by LDS-DMA, 16-byte chunk c of row r at
+// c ^ (r & 15). The 8 waves split the slot's eight 32-k chunks and the token
+// halves: with TH 2 wave w takes chunks w & 3 and (w & 3) + 4 of tokens 16 (w >> 2)
+// .. +15, with TH 1 chunk w; their sums meet in LDS at the end, in wave order.
+// Every wave issues the same number of loads per slot; a surplus one reads an
+// empty buffer into a spare KiB. Rows past N, tokens past M and chunks past K
+// read zeros.
+constexpr int kOwnK = 256;
+template <int UB, int TH> struct W8Own {
+    static constexpr uint32_t W_BYTES = UB * 16 * kOwnK, X_BYTES = TH * 16 * kOwnK * 2;
+    static constexpr uint32_t SLOT = W_BYTES + X_BYTES;
+    static constexpr int FIT = (int)((160 * 1024 - 1024) / SLOT);
+    static constexpr int SLOTS = FIT < 10 ? FIT : 10;
+    static constexpr int NW = (UB * 4 + 7) / 8, NX = TH;  // loads per wave and slot
+};
+
+template <int UB, int TH>
+__global__ void __launch_bounds__(512)
+w8a16_own_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ Wq, const float* __restrict__ scale,
+                 uint16_t* __restrict__ Y, int M, int N, int K, int relu) {
+    using C = W8Own<UB, TH>;
+    constexpr int SLOTS = C::SLOTS, LOADS = C::NW + C::NX;
+    static_assert(SLOTS >= 3 && (SLOTS - 2) * LOADS <= 60, "ring");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[SLOTS * C::SLOT + 1024];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const int n0 = blockIdx.x * 16 * UB;
+    const int KT = (K + kOwnK - 1) / kOwnK;
+    constexpr uint32_t kPast = 0xFFFFFFF0u;
+
+    const i32x4 wrs = make_buf_rsrc(Wq, (uint32_t)((size_t)N * K));
+    const i32x4 xrs = make_buf_rsrc(X, (uint32_t)((size_t)M * K * 2));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    // weight load e of a wave: rows 4q .. 4q+3 (q = NW wave + e), 16 lanes a row;
+    // X load e: tokens 2q, 2q+1 (q = NX wave + e), 32 lanes a token
+    uint32_t wo[C::NW], xo[C::NX];
+    int wk[C::NW], xk[C::NX];  // first k of the lane's chunk within a slot
+#pragma unroll
+    for (int e = 0; e < C::NW; ++e) {
+        const int row = 4 * (C::NW * wave + e) + lane / 16;
+        wk[e] = 16 * ((lane & 15) ^ (row & 15));
+        wo[e] = (uint32_t)(n0 + row) * (uint32_t)K + (uint32_t)wk[e];
+    }
+#pragma unroll
+    for (int e = 0; e < C::NX; ++e) {
+        const int tok = 2 * (C::NX * wave + e) + lane / 32;
+        xk[e] = 8 * ((lane & 31) ^ (tok & 15));
+        xo[e] = ((uint32_t)tok * (uint32_t)K + (uint32_t)xk[e]) * 2u;
+    }
+    auto issue = [&](int kt, int slot) {
+        const uint32_t base = lds0 + (uint32_t)slot * C::SLOT;
+        const int k0 = kt * kOwnK;
+#pragma unroll
+        for (int e = 0; e < C::NW; ++e) {
+            const int q = C::NW * wave + e;
+            const bool spare = q >= UB * 4;  // uniform
+            const uint32_t off = k0 + wk[e] < K && !spare ? wo[e] + (uint32_t)k0 : kPast;
+            lds_dma_buf_b128_nt_u(wrs, off, 0u, spare ? lds0 + SLOTS * C::SLOT : base + (uint32_t)q * 1024u);
+        }
+#pragma unroll
+        for (int e = 0; e < C::NX; ++e)
+            lds_dma_buf_b128_u(xrs, k0 + xk[e] < K ? xo[e] + (uint32_t)k0 * 2u : kPast, 0u,
+                               base + C::W_BYTES + (uint32_t)(C::NX * wave + e) * 1024u);
+    };
+
+    f32x4 acc[UB];
+#pragma unroll
+    for (int u = 0; u < UB; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int th = TH == 2 ? wave >> 2 : 0;
+    const int c0 = TH == 2 ? wave & 3 : wave;
+#pragma unroll 1
+    for (int p = 0; p < SLOTS - 1; ++p) issue(p, p);
+    int cur = 0, nxt = SLOTS - 1;
+#pragma unroll 1
+    for (int kt = 0; kt < KT; ++kt) {
+        wait_vmem_le<(SLOTS - 2) * LOADS>();  // own loads of slot kt landed
+        __syncthreads();                       // every wave's; slot kt-1 is consumed
+        issue(kt + SLOTS - 1, nxt);
+        const uint8_t* ws = smem + (uint32_t)cur * C::SLOT;
+        const uint8_t* xs = ws + C::W_BYTES;
+#pragma unroll
+        for (int i = 0; i < TH; ++i) {
+            const int c = c0 + 4 * i;  // 32-k chunk: 16-byte chunks 2c, 2c+1 of a weight row, 4c .. 4c+3 of a token
+            const int t = 16 * th + lr;
+            const u32x4 xf = *reinterpret_cast<const u32x4*>(xs + t * (kOwnK * 2) + (((4 * c + lg) ^ (t & 15)) * 16));
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int r = 16 * u + lr;
+                const u32x2 w = *reinterpret_cast<const u32x2*>(ws + r * kOwnK + (((2 * c + (lg >> 1)) ^ (r & 15)) * 16) +
+                                                                8 * (lg & 1));
+                acc[u] = mfma16x16x32(fp8x8_to_bf16x8(w[0], w[1]), xf, acc[u], bf16_t{});
+            }
+        }
+        nxt = cur;
+        cur = cur + 1 == SLOTS ? 0 : cur + 1;
+    }
+    wait_vmem_le<0>();
+    __syncthreads();  // the ring takes the sums
+    f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int u = 0; u < UB; ++u) red[(wave * UB + u) * kWave + lane] = acc[u];
+    __syncthreads();
+    // thread: channels 16 u + 4 lg .. +3 of the unit, token 16 h + lr
+    if (tid < TH * UB * kWave) {
+        const int u = (tid >> 6) % UB, h = (tid >> 6) / UB;
+        constexpr int NP = 8 / TH;
+        f32x4 v = red[(h * NP * UB + u) * kWave + lane];
+#pragma unroll
+        for (int p = 1; p < NP; ++p) v += red[((h * NP + p) * UB + u) * kWave + lane];
+        const int t = 16 * h + lr, n = n0 + 16 * u + 4 * lg;
+        if (t < M) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) {
+                    float y = v[r] * scale[n + r];
+                    if (relu) y = y > 0.f ? y : 0.f;
+                    Y[(size_t)t * N + n + r] = elem<bf16_t>::from_f32(y);
+                }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1139,27 +1270,73 @@ extern "C" int pyc_hip_w8a16_reserve(int N, int K) {
     return w8_reserve(w8_plan(N, K, cu_count())) ? 0 : -2;
 }
 
-extern "C" int pyc_hip_w8a16_launch(int M, int N, int K, const void* X, const void* Wq, const float* scale,
-                                    int relu, void* Y, void* stream) {
+namespace {
+
+// Estimated microseconds of one layer on the MI355X, fitted to back-to-back runs.
+// Token kernel [N,K]: 4096 x 11008 11.1 (1 token), 12.7 (2); 4096 x 8192 10.5 (3),
+// 11.8 (4; whole-K 10.5); 11008 x 4096 9.7 (1; whole-K 10.7), 16.5 (4; whole-K
+// 11.2). Whole-K kernel with UB 1 / 2 / 3 / 4 (split-K kernel), 32 tokens:
+// 4096 x 11008 18.4 / 22 / 26 / 28 (22.7), 11008 x 4096 24.5 / 20.6 / 14.0 / 14.7 (21.6),
+// 14336 x 14336 82 / 56 / 66 / 42 (57), 6144 x 6144 21 / 14.6 / 17 / 18 (20), 12160 x
+// 1664 16 / 13 / 8.6 / 8.7 (16), 1024 x 1024 4.7 / 5.2 / 6.0 / 5.9 (9.2); the split
+// keeps few units over a deep K: 1024 x 14336 20.6 / 25 / 30 / 33 (19.8).
+// 16 tokens of 4096 x 11008 14.5 (20.5), 5 13.3 (19.6); 8 of 4096 x 4096 7.2 (11.7).
+size_t w8_token_lds(int M, int K) { return (size_t)M * ((K / 16 + pyc::kWave - 1) / pyc::kWave) * pyc::kWave * 32; }
+
+bool w8_token_fits(int M, int K) { return M <= 4 && w8_token_lds(M, K) <= pyc::kTokLdsMax; }
+
+// 32-bit byte offsets, also of the rows a last unit has past N
+bool w8_own_fits(int N, int K) {
+    return ((size_t)N + 64) * K < 0xFFFFFFF0ull && (size_t)32 * K * 2 < 0xFFFFFFF0ull;
+}
+
+double w8_token_cost(int M, int N, int K) { return 2.6 + (double)N * K / 5.9e6 * (1.0 + 0.15 * (M - 1)); }
+
+double w8_own_cost(int ub, int M, int N, int K) {
+    const int units = (N + 16 * ub - 1) / (16 * ub);
+    const double rounds = (double)((units + 255) / 256);
+    // us per KB of W: more channels a workgroup, more of W in flight
+    constexpr double kPerKb[5] = {0.0, 0.055, 0.045, 0.037, 0.033};
+    return 1.2 + rounds * (1.8 + (kPerKb[ub] * 16 * ub + 0.008 * 2 * M) * K / 1000.0);
+}
+
+double w8_split_cost(int N, int K) { return 11.0 + 0.058 * ((double)N * K / 256.0 / 1000.0); }
+
+// The cheapest kernel that splits no row over workgroups: 0 = token, 1..4 = own
+// with that UB; -1 where neither can (offsets past 32 bits). *cost: its estimate.
+int w8_whole_form(int M, int N, int K, double* cost) {
+    int form = -1;
+    if (w8_token_fits(M, K)) {
+        form = 0;
+        *cost = w8_token_cost(M, N, K);
+    }
+    if (w8_own_fits(N, K)) {
+        for (int ub = 1; ub <= 4; ++ub) {
+            const double c = w8_own_cost(ub, M, N, K);
+            if (form < 0 || c < *cost) {
+                form = ub;
+                *cost = c;
+            }
+        }
+    }
+    return form;
+}
+
+int w8_whole_launch(int form, int M, int N, int K, const void* X, const void* Wq, const float* scale, int relu,
+                    void* Y, hipStream_t s) {
     using namespace pyc;
-    hipStream_t s = (hipStream_t)stream;
-    // Up to four tokens whose X fits the token kernel's LDS: two rows per wave
-    // where that still gives every CU a workgroup, else one. In us, split-K
-    // kernel / token kernel, [N,K] 4096 x 11008: 19.4 / 11.1 (one token), 19.5 /
-    // 12.7 (two); 8192 deep 14.9 / 11.9 (four); 11008 x 4096: 18.3 / 9.7 (one),
-    // 18.6 / 16.7 (four); 14336 x 14336: 53 / 33 (6.2 TB/s); 1024 x 1024: 7.9 / 2.7.
-    const size_t xbytes = (size_t)M * ((K / 16 + kWave - 1) / kWave) * kWave * 32;
-    if (M <= 4 && xbytes <= kTokLdsMax) {
+    const uint16_t* x = (const uint16_t*)X;
+    const uint8_t* w = (const uint8_t*)Wq;
+    uint16_t* y = (uint16_t*)Y;
+    if (form == 0) {
+        // two rows per wave where that still gives every CU a workgroup, else one
         const int r = N >= 2 * kTokWaves * 256 ? 2 : 1;
         const dim3 grid((N + r * kTokWaves - 1) / (r * kTokWaves)), block(kTokWaves * kWave);
-#define PYC_TOK(MM)                                                                                             \
-    do {                                                                                                        \
-        if (r == 2)                                                                                             \
-            hipLaunchKernelGGL((w8a16_token_kernel<MM, 2>), grid, block, xbytes, s, (const uint16_t*)X,         \
-                               (const uint8_t*)Wq, scale, (uint16_t*)Y, N, K, relu);                            \
-        else                                                                                                    \
-            hipLaunchKernelGGL((w8a16_token_kernel<MM, 1>), grid, block, xbytes, s, (const uint16_t*)X,         \
-                               (const uint8_t*)Wq, scale, (uint16_t*)Y, N, K, relu);                            \
+        const size_t lds = w8_token_lds(M, K);
+#define PYC_TOK(MM)                                                                                                 \
+    do {                                                                                                            \
+        if (r == 2) hipLaunchKernelGGL((w8a16_token_kernel<MM, 2>), grid, block, lds, s, x, w, scale, y, N, K, relu); \
+        else hipLaunchKernelGGL((w8a16_token_kernel<MM, 1>), grid, block, lds, s, x, w, scale, y, N, K, relu);        \
     } while (0)
         switch (M) {
             case 1: PYC_TOK(1); break;
@@ -1168,8 +1345,40 @@ extern "C" int pyc_hip_w8a16_launch(int M, int N, int K, const void* X, const vo
             default: PYC_TOK(4); break;
         }
 #undef PYC_TOK
-        return hipGetLastError() == hipSuccess ? 0 : -2;
+    } else {
+        const dim3 grid((N + 16 * form - 1) / (16 * form)), block(512);
+#define PYC_OWN(UB)                                                                                                \
+    do {                                                                                                           \
+        if (M <= 16) hipLaunchKernelGGL((w8a16_own_kernel<UB, 1>), grid, block, 0, s, x, w, scale, y, M, N, K, relu); \
+        else hipLaunchKernelGGL((w8a16_own_kernel<UB, 2>), grid, block, 0, s, x, w, scale, y, M, N, K, relu);         \
+    } while (0)
+        switch (form) {
+            case 1: PYC_OWN(1); break;
+            case 2: PYC_OWN(2); break;
+            case 3: PYC_OWN(3); break;
+            default: PYC_OWN(4); break;
+        }
+#undef PYC_OWN
     }
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+}  // namespace
+
+// form: -1 = the cheapest by estimate, 0 = token kernel, 1 .. 4 = whole-K kernel
+// with that UB, 5 = split-K kernel; -1 is returned where the form cannot run.
+extern "C" int pyc_hip_w8a16_launch_form(int form, int M, int N, int K, const void* X, const void* Wq,
+                                         const float* scale, int relu, void* Y, void* stream) {
+    using namespace pyc;
+    hipStream_t s = (hipStream_t)stream;
+    if (form < 0) {
+        double whole = 0.0;
+        form = w8_whole_form(M, N, K, &whole);
+        if (form < 0 || whole >= w8_split_cost(N, K)) form = 5;
+    } else if (form == 0 ? !w8_token_fits(M, K) : form < 5 ? !w8_own_fits(N, K) : form > 5) {
+        return -1;
+    }
+    if (form < 5) return w8_whole_launch(form, M, N, K, X, Wq, scale, relu, Y, s);
     W8Plan p = w8_plan(N, K, cu_count());
     float* part = nullptr;
     int* cnt = nullptr;
@@ -1202,6 +1411,11 @@ extern "C" int pyc_hip_w8a16_launch(int M, int N, int K, const void* X, const vo
                            (const uint8_t*)Wq, scale, (uint16_t*)Y, M, N, K, relu, p.base, p.rem, part, cnt,
                            p.max_slots);
     return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+extern "C" int pyc_hip_w8a16_launch(int M, int N, int K, const void* X, const void* Wq, const float* scale,
+                                    int relu, void* Y, void* stream) {
+    return pyc_hip_w8a16_launch_form(-1, M, N, K, X, Wq, scale, relu, Y, stream);
 }
 
 namespace {

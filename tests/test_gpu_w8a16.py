@@ -2,6 +2,8 @@
 
 Tolerance: max|got-ref| <= 2e-2 * max|ref|, and each bf16
 output within two bf16 roundings of the oracle's bf16 output."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -113,22 +115,32 @@ def test_w8a16_chain_graph_replay(gpu):
     assert rel_max_err(got, y_ref) <= 2e-2
 
 
-@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
-@pytest.mark.parametrize("N,K", [(1, 16), (9, 1024), (17, 1040), (4103, 2064), (70, 8192), (70, 8208)])
-def test_w8a16_few_tokens(gpu, M, N, K):
-    """One to four tokens on the row-per-wave kernel (one and two rows per wave,
-    rows of one piece, of whole KiB and one piece over, N no multiple of a
-    workgroup's rows, X at and past its LDS limit), five on the split-K one."""
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(1, 16), (9, 1024), (17, 1040), (49, 256), (4103, 2064), (70, 8192), (70, 8208)])
+def test_w8a16_forms(gpu, M, N, K):
+    """Every kernel a layer can take, each at its edges: row per wave (0: one and
+    two rows per wave, rows of one piece, of whole KiB and one piece over, N no
+    multiple of a workgroup's rows, X at and past its LDS limit), whole K per
+    workgroup (1 .. 4: channels short of and past one unit, one token half and
+    two, fewer k steps than the ring has slots, and a partial last one), split K
+    (5), and the one chosen (-1)."""
     torch = gpu
     x, wq, scale = _layer(M, N, K, M * 7 + N + K)
-    Y = torch.full((M * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
     L = pyc_amd.lib()
+    f = L.pyc_hip_w8a16_launch_form
+    f.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.c_int] + [C.c_void_p] * 2
     X, Wq, S = dev_bits16(torch, x), dev_u8(torch, wq), dev_f32(torch, scale)
-    assert L.pyc_hip_w8a16_gemm_dispatch(b"hip_gemm_w8a16_e4m3", M, N, K, X.data_ptr(), Wq.data_ptr(), S.data_ptr(), 0,
-                                         Y.data_ptr(), None) == 0
-    torch.cuda.synchronize()
-    assert bool((Y[M * N:] == 7.0).all())
     ref = oracle.bf16_to_f32(oracle.w8a16_layer(x, wq, scale, False))
-    got = Y[:M * N].float().cpu().numpy().reshape(M, N)
-    # two roundings to bf16 of nearby sums, plus fp32 summation order
-    assert (np.abs(got - ref) <= 2.0 ** -7 * np.abs(ref) + 4e-6 * np.sqrt(K) * np.abs(ref).max()).all()
+    for form in (-1, 0, 1, 2, 3, 4, 5):
+        Y = torch.full((M * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+        rc = f(form, M, N, K, X.data_ptr(), Wq.data_ptr(), S.data_ptr(), 0, Y.data_ptr(), None)
+        if form == 0 and (M > 4 or M * -(-K // 1024) * 2048 > 65536):
+            assert rc == -1
+            continue
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert bool((Y[M * N:] == 7.0).all())
+        got = Y[:M * N].float().cpu().numpy().reshape(M, N)
+        # two roundings to bf16 of nearby sums, plus fp32 summation order
+        bound = 2.0 ** -7 * np.abs(ref) + 4e-6 * np.sqrt(K) * np.abs(ref).max()
+        assert (np.abs(got - ref) <= bound).all(), form
