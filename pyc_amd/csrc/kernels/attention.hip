@@ -894,43 +894,60 @@ static hipError_t launch_attn_small(int BH, int S, int causal, const void* q, co
     return hipGetLastError();
 }
 
-// Estimated microseconds of each form, from measurements on the MI355X (warm, back
-// to back; [B,H,S,D], persistent / QW = 2 / QW = 4): [2,16,1000,64] 22.8 / 17.1 /
-// 16.7, [1,8,1917,128] causal 57.5 / 24.2 / 37, [1,8,1917,64] causal 44 / 15.8 /
-// 25, [4,16,954,64] causal 29.6 / 21 / 18.6, [3,32,473,128] 21.5 / 32 / 29,
-// [8,32,300,128] causal 29.4 / 42 / 35, [8,32,2048,64] causal 190 / 312 / 207,
-// [1,12,64,64] 5.8 / 4.9 / 4.7. The persistent form takes a fixed part, then
-// one time per 64-key block of its longest workgroup; the others one per step
-// of the longest workgroup or of the average CU, and a start and end per round
-// of workgroups.
+// Estimated microseconds of each form, fitted to 400 shapes on the MI355X (warm, back
+// to back; mean error 3 to 6 %, S from 64 to 4096, B H from 8 to 256). Persistent /
+// QW = 2 / QW = 4 of [B,H,S,D]: [2,16,1000,64] 22.8 / 17.1 / 16.7, [1,32,1196,128]
+// causal 43 / 33 / 26.7, [1,8,1260,64] causal 32 / 11.8 / 18.4, [8,16,583,128]
+// causal 33.7 / 47 / 36.9, [1,32,2551,128] 121 / 157 / 149, [7,32,539,128] causal
+// 60 / 80 / 66, [8,32,2048,64] causal 190 / 312 / 207, [1,12,64,64] 5.8 / 4.9 / 4.7.
+// The persistent form takes a fixed part and, per round of its grid, a start and
+// one time per 64-key block of its longest workgroup, more with more CUs busy.
+// A workgroup of the small forms takes a start and one time per step; at d = 128
+// one fits a CU, at d = 64 two share it (the terms in both kinds of rounds).
 static double attn_cost_persist(int BH, int S, int D, int causal) {
     const int nqb = (S + 255) / 256;
     const bool pair = causal && nqb > 1;
     const long units = (long)BH * (pair ? (nqb + 1) / 2 : nqb);
-    const double rounds = (double)((units + 255) / 256), busy = units < 256 ? (double)units / 256.0 : 1.0;
+    const double rounds = (double)((units + 255) / 256), busy = (double)units / (256.0 * rounds);
     // a pair's blocks: its first q-block (ragged) and q-block 0, or any other pair's 4 (nqb + 1)
     const double top = (double)((S + 63) / 64), rest = nqb >= 4 ? 4.0 * (nqb + 1) : nqb == 3 ? 8.0 : 0.0;
     const double blocks = !pair ? top : top + 4.0 > rest ? top + 4.0 : rest;
-    const double block = D == 128 ? 1.45 + 0.65 * busy : 1.1 + 0.2 * busy;
-    return 4.5 + rounds * blocks * block + (pair ? 3.0 : 0.0) * rounds;
+    if (D == 128)
+        return causal ? 0.2 + (pair ? 4.1 : 0.0) + rounds * (6.9 + blocks * (1.22 + 0.35 * busy))
+                      : 3.8 + rounds * (3.7 + blocks * (1.12 + 0.58 * busy));
+    return causal ? 2.8 + (pair ? 3.1 : 0.0) + rounds * (3.05 + blocks * (0.96 + 0.13 * busy))
+                  : 3.0 + rounds * (3.1 + blocks * (0.94 + 0.2 * busy));
 }
 
 static double attn_cost_small(int BH, int S, int D, int causal, int qw) {
-    const int bq = 32 * qw, rows = 256 / qw, nqb = (S + bq - 1) / bq;
-    const double wgs = (double)BH * nqb, n = (double)((S + rows - 1) / rows);
-    const double step = D == 128 ? (qw == 2 ? 1.28 : 1.1) : (qw == 2 ? 0.77 : 0.74);
-    const double at_once = D == 128 ? 256.0 : 512.0;
-    const double rounds = (double)(long)((wgs + at_once - 1.0) / at_once);
-    double steps;
-    if (causal) {
-        // block q of nqb walks (q + 1) bq keys; the long ones start first
-        const double mean = 0.5 * ((double)bq / rows) * (nqb + 1) + 0.5 * (1.0 - 1.0 / qw);
-        const double avg = wgs * (mean < n ? mean : n) / 256.0;
-        steps = n > avg ? n : avg;
-    } else {
-        steps = rounds * n * (D == 64 && wgs > 256.0 ? 2.0 : 1.0);
+    const int bq = 32 * qw, rows = 256 / qw, nqb = (S + bq - 1) / bq, nmax = (S + rows - 1) / rows;
+    const long wgs = (long)BH * nqb;
+    const double n = nmax, per_cu = (double)wgs / 256.0, r1 = (double)((wgs + 255) / 256);
+    if (!causal) {
+        if (D == 128) return qw == 2 ? 1.5 + r1 * (5.2 + n * 1.19) : 1.1 + r1 * (5.7 + n * 1.04);
+        const double r2 = (double)((wgs + 511) / 512);
+        return qw == 2 ? 2.65 + 2.1 * r1 + n * (0.236 * r1 + 0.37 * r2 + 0.18 * per_cu)
+                       : 1.85 + 2.9 * r1 + n * (0.237 * r1 + 0.4 * r2 + 0.086 * per_cu);
     }
-    return (D == 128 ? 0.0 : 2.5) + (D == 128 ? (qw == 2 ? 4.5 : 5.0) : 2.0) * rounds + steps * step;
+    // q-block q walks (q + 1) bq keys; the steps of all of them
+    const double m = nqb, sum = qw == 2 ? (double)((long)(nqb + 1) * (nqb + 1) / 4) : m * (m + 1.0) - (2.0 * m - n);
+    const double avg = BH * sum / 256.0, longest = n > avg ? n : avg;
+    if (D == 64)
+        return qw == 2 ? 1.9 + 2.65 * (per_cu > 1.0 ? per_cu : 1.0) + 0.134 * avg + 0.38 * n + 0.305 * longest
+                       : 0.3 + 4.15 * (per_cu > 1.0 ? per_cu : 1.0) + 0.056 * avg + 0.49 * n + 0.17 * longest;
+    // the long ones start first: one alone, the 256th and 257th in line, or an even share
+    const double start = qw == 2 ? 6.1 : 9.7, step = qw == 2 ? 1.22 : 1.03;
+    double t = start + n * step;
+    if (wgs > 256) {
+        const int q0 = nqb - 1 - 255 / BH, q1 = nqb - 1 - 256 / BH;
+        const double s0 = qw == 2 ? (q0 + 2) / 2 : (2 * q0 + 2 < nmax ? 2 * q0 + 2 : nmax);
+        const double s1 = qw == 2 ? (q1 + 2) / 2 : (2 * q1 + 2 < nmax ? 2 * q1 + 2 : nmax);
+        const double two = 2.0 * start + (s0 + s1) * step;
+        const double even = per_cu * start + avg * step + (qw == 2 ? 1.7 : 0.8);
+        t = t > two ? t : two;
+        t = t > even ? t : even;
+    }
+    return t + (qw == 2 ? 0.1 : -3.4);
 }
 
 // form: 0 = the cheapest by estimate, 1 = persistent, 2 / 4 = small with that QW
@@ -946,7 +963,8 @@ static hipError_t launch_attn(int form, int B, int H, int S, int causal, const v
     if (form == 0) {
         const double c1 = attn_cost_persist(BH, S, D, causal), c2 = attn_cost_small(BH, S, D, causal, 2),
                      c4 = attn_cost_small(BH, S, D, causal, 4);
-        form = c1 <= c2 && c1 <= c4 ? 1 : c2 <= c4 ? 2 : 4;
+        // the estimates' error: a small form has to be 5 % ahead
+        form = c1 <= 1.05 * c2 && c1 <= 1.05 * c4 ? 1 : c2 <= c4 ? 2 : 4;
     }
     if (form == 2) return launch_attn_small<T, D, 2>(BH, S, causal, q, k, v, o, scale_log2, s);
     if (form == 4) return launch_attn_small<T, D, 4>(BH, S, causal, q, k, v, o, scale_log2, s);
