@@ -19,6 +19,11 @@
 // same k permutation {4*(lane/16)+e}. B is staged in LDS as [n][k] for both
 // layouts ([K,N] tiles are transposed on the LDS store). Waves 0-3 stage B,
 // waves 4-7 stage A.
+//
+// gemm_f32_dma_kernel takes nearly all shapes (whole tiles, and ragged ones on
+// 64x64 or 32x32 tiles) with both operands moved to LDS by LDS-DMA; the
+// register-staged gemm_f32_kernel takes operands past 32-bit offsets and
+// many ragged tiles of a short k (see pyc_hip_gemm_f32_launch).
 #include "common.hpp"
 #include "lds_dma.hpp"
 
@@ -482,14 +487,26 @@ extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const v
                      (whole ? (size_t)M * K * 4 < (1ull << 32) && (size_t)N * K * 4 < (1ull << 32)
                             : ((size_t)M + pad) * ((size_t)K + pad) * 4 < kF32PastEnd &&
                                   ((size_t)N + pad) * ((size_t)K + pad) * 4 < kF32PastEnd);
-    if (dma) {
-        const int tile = tile_f32(M, N, K, whole);
+    const int tile = tile_f32(M, N, K, whole);
+    // More ragged 64 x 64 tiles than CUs and a short k: starts and ends count,
+    // and two register-staged workgroups share a CU where one ring takes it. us,
+    // ring / register-staged, [K,N] B: 1728 x 2568 x 64 26.8 / 20.3, 1015 x 2944 x 128
+    // 21.1 / 19.1, 2805 x 1600 x 140 38 / 36, 2676 x 560 x 448 25.7 / 27.6; rows off 16
+    // bytes 1472 x 1980 x 194 28.8 / 36; [N,K] B 2916 x 448 x 192 16.2 / 14.2, 512 x
+    // 2440 x 512 27.3 / 26.6.
+    const bool wide = K % 4 == 0 && (b_trans || N % 4 == 0);
+    const bool staged = !whole && tile == 64 && (long)((M + 63) / 64) * ((N + 63) / 64) > 256 &&
+                        K <= (!wide ? 128 : b_trans ? 512 : 256);
+    if (dma && !staged) {
         const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
         const dim3 tiles((unsigned)(tiles_m * tiles_n));
         const int gm = tiles_m < 4 ? tiles_m : 4;
         RunSignal sg{nullptr, nullptr, 0u};
-        // when this launch ends the run, it stores the completion word itself
-        const bool sig = run_signal_claim(&sg);
+        // when this launch ends the run, it stores the completion word itself; ragged
+        // rows reach the coherent level more slowly than the run's own signal
+        // takes (us, one run: 693 x 3008 x 720 74 / 67, 300 x 3008 x 72 22 / 20.6,
+        // 232 x 448 x 71 17.4 / 17.2)
+        const bool sig = whole && run_signal_claim(&sg);
 #define PYC_F32(BT, SIG, TILE, RAG)                                                                                \
     hipLaunchKernelGGL((gemm_f32_dma_kernel<BT, SIG, TILE, RAG>), tiles, block, 0, s, a, b, c, M, N, K, alpha, beta, \
                        bias, epi, gm, sg.word, sg.count, sg.seq)
@@ -497,7 +514,7 @@ extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const v
     do {                                                   \
         if (tile == 32) PYC_F32(BT, SIG, 32, true);        \
         else if (whole) PYC_F32(BT, SIG, 64, false);       \
-        else PYC_F32(BT, SIG, 64, true);                   \
+        else PYC_F32(BT, false, 64, true);                 \
     } while (0)
         if (sig) {
             if (b_trans) PYC_F32_TILE(true, true);

@@ -541,6 +541,7 @@ def test_register_staged_tiles(gpu, bt, layout, dtype, dn, k, off):
     (700, 1000, 66, 0),  # 64 x 64 tiles, crossing chunks
     (961, 1021, 129, 3), # 64 x 64 tiles, one element into the third k-tile
     (64, 64, 257, 0),    # whole M and N
+    (1030, 1090, 100, 0),  # more 64 x 64 tiles than CUs, short k: register-staged
 ])
 def test_f32_ragged_tiles(gpu, m, n, k, off, layout):
     """fp32 shapes that are no whole 64 x 64 x 64 tiles, on both tiles, against
