@@ -31,6 +31,10 @@
 // scale/ReLU, writes Y and resets the counter to zero for the next launch (so
 // graph replays need no memset).
 // Without a workspace every workgroup owns whole units instead.
+//
+// That split pays for few channels over a deep K. Elsewhere, and for up to four
+// tokens, the two kernels that split no row (token, own) are faster; the
+// launch estimates all of them (w8_whole_form, w8_split_cost).
 #include <stdlib.h>
 
 #include <mutex>
@@ -1564,6 +1568,39 @@ int chain_stages() {
     return stages;
 }
 
+// A chain layer by layer (the kernels that split no row, one launch each, the
+// activations in the same workspace) instead of in one launch: a step of the
+// chain kernel costs about 8.5 us besides what its weight stream adds (partials,
+// counters and the wait for all other workgroups), a layer's launch 3, but with
+// 24 to 32 tokens and long rows the layers read more of X. In us, chain kernel /
+// layers (tokens x width x inner width, pairs of layers): 1 x 4096 x 11008, 8
+// 235 / 206; 16: 243 / 222; 24: 251 / 250; 32: 258 / 266; 1 x 3584 x 3200, 4 83 /
+// 37; 10 x 1536 x 4224, 8 140 / 100; 31 x 3328 x 4608, 5 113 / 100; 31 x 2560 x 8960,
+// 6 150 / 153. `form`: 0 = by estimate, 1 = one launch, 2 = layers.
+bool chain_by_layers(int form, const pyc::W8ChainArgs& a) {
+    if (form != 0) return form == 2;
+    double chain = 0.0, layers = 0.0;
+    for (int s = 0; s < a.nsteps; ++s) {
+        double c = 0.0;
+        if (w8_whole_form(a.M, a.st[s].N, a.st[s].K, &c) < 0) return false;
+        layers += c;
+        chain += 8.5 + 0.036 * ((double)a.st[s].N * a.st[s].K / 256.0 / 1000.0) + 0.04 * a.M;
+    }
+    return layers < 0.9 * chain;
+}
+
+int chain_layers_launch(const pyc::W8ChainArgs& a, hipStream_t st) {
+    for (int s = 0; s < a.nsteps; ++s) {
+        const pyc::W8ChainStep& P = a.st[s];
+        double c = 0.0;
+        const int form = w8_whole_form(a.M, P.N, P.K, &c);
+        if (form < 0) return -1;
+        const int rc = w8_whole_launch(form, a.M, P.N, P.K, P.X, P.W, P.scale, P.relu, P.Y, st);
+        if (rc != 0) return rc;
+    }
+    return 0;
+}
+
 int chain_kernel_launch(const pyc::W8ChainArgs& a, hipStream_t st) {
     using namespace pyc;
     const int stages = chain_stages();
@@ -1585,9 +1622,10 @@ extern "C" int pyc_hip_w8a16_chain_reserve(int M, int nsteps, const int* N, cons
     return chain_reserve(L.total) ? 0 : -2;
 }
 
-extern "C" int pyc_hip_w8a16_chain_launch(int M, int nsteps, const void* X, const void* const* Wq,
-                                          const float* const* scale, const int* N, const int* K, const int* relu,
-                                          void* Y, void* stream) {
+// form: see chain_by_layers
+extern "C" int pyc_hip_w8a16_chain_launch_form(int form, int M, int nsteps, const void* X, const void* const* Wq,
+                                               const float* const* scale, const int* N, const int* K,
+                                               const int* relu, void* Y, void* stream) {
     using namespace pyc;
     ChainLayout L;
     if (!N || !K || !Wq || !scale || !relu || !X || !Y || chain_layout(M, nsteps, N, K, L) != 0) return -1;
@@ -1602,7 +1640,13 @@ extern "C" int pyc_hip_w8a16_chain_launch(int M, int nsteps, const void* X, cons
     }
     W8ChainArgs a;
     if (chain_args(a, L, g_chainws[dev].buf, M, nsteps, X, Wq, scale, N, K, relu, Y) != 0) return -1;
-    return chain_kernel_launch(a, st);
+    return chain_by_layers(form, a) ? chain_layers_launch(a, st) : chain_kernel_launch(a, st);
+}
+
+extern "C" int pyc_hip_w8a16_chain_launch(int M, int nsteps, const void* X, const void* const* Wq,
+                                          const float* const* scale, const int* N, const int* K, const int* relu,
+                                          void* Y, void* stream) {
+    return pyc_hip_w8a16_chain_launch_form(0, M, nsteps, X, Wq, scale, N, K, relu, Y, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1655,6 +1699,7 @@ extern "C" int pyc_hip_w8a16_chain_launch_noalloc(int M, int nsteps, const void*
     W8ChainArgs a;
     if (chain_args(a, L, base, M, nsteps, X, Wq, scale, N, K, relu, Y) != 0) return -1;
     hipStream_t st = (hipStream_t)stream;
+    if (chain_by_layers(0, a)) return chain_layers_launch(a, st);  // needs no counters
     const int words = (int)((L.zero_hi - L.zero_lo) / sizeof(uint32_t));
     hipLaunchKernelGGL(zero_words_kernel, dim3((words + 255) / 256 < 256 ? (words + 255) / 256 : 256), dim3(256), 0,
                        st, (uint32_t*)(base + L.zero_lo), words);

@@ -199,3 +199,29 @@ def test_chain_rejects_bad_shapes(gpu):
     assert call(b"hip_w8a16_chain_e4m3", 4, [256, 128], [256, 128]) == -1  # K[1] != N[0]
     torch.cuda.synchronize()
     assert pyc_amd.w8a16_chain_error() == 0
+
+
+@pytest.mark.parametrize("form", [1, 2, 0])
+@pytest.mark.parametrize("M,dims", [(32, [128, 64]), (17, [1152, 2176, 1152]), (4, [1024, 128, 128, 2816]),
+                                    (1, [384, 4096, 512])])
+def test_chain_forms(gpu, form, M, dims):
+    """One launch for the chain and one per layer, each against the oracle."""
+    torch = gpu
+    relus = [i % 2 == 0 for i in range(len(dims) - 1)]
+    ws = _weights(dims, M)
+    layers = _dev_layers(torch, ws, relus)
+    x = oracle.f32_to_bf16(np.random.default_rng(M).standard_normal((M, dims[0])).astype(np.float32))
+    X = dev_bits16(torch, x)
+    f = pyc_amd.lib().pyc_hip_w8a16_chain_launch_form
+    f.argtypes = [C.c_int] * 3 + [C.c_void_p] * 8
+    n, wq, sc, N, K, relu = pyc_amd._chain_arrays(layers)
+    v = lambda a: C.cast(a, C.c_void_p)
+    cur = x
+    for (w, s), r in zip(ws, relus):
+        cur = oracle.w8a16_layer(cur, w, s, r)
+    for _ in range(2):
+        Y = torch.full((M, dims[-1]), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert f(form, M, n, X.data_ptr(), v(wq), v(sc), v(N), v(K), v(relu), Y.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        assert pyc_amd.w8a16_chain_error() == 0
+        assert rel_max_err(oracle.bf16_to_f32(host_bits16(Y)), oracle.bf16_to_f32(cur)) <= 2e-2
