@@ -13,7 +13,9 @@
 // gathered on the fly: with C % 8 == 0 every 16-byte k-chunk of a row is 8
 // consecutive channels of one input pixel, so each A load is one coalesced
 // 16-byte NHWC read (zero for taps in the padding). The mainloop, LDS layout and
-// epilogue are those of gemm_core.hpp.
+// epilogue are those of gemm_core.hpp. The automatic route takes the LDS-DMA
+// kernels (persistent or ring tiles) where their 32-bit offsets reach; these
+// tiles serve the tiled symbols and what is left.
 #include "gemm_core.hpp"
 
 namespace pyc {

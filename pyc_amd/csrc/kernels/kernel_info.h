@@ -39,7 +39,7 @@ enum {
 int pyc_hip_kinfo_nt_lds(int kid, int is_bf16, pyc_hip_kinfo* out);
 /* gemm_mfma.hip: register-staged tiles (tile 64, 128 or 256) */
 int pyc_hip_kinfo_half(int tile, int b_trans, int is_bf16, pyc_hip_kinfo* out);
-/* gemm_small.hip: LDS-DMA ring tiles (tile 64 or 128) */
+/* gemm_small.hip: LDS-DMA ring tiles (the registry's tile is 64 or 128; the launch may take others) */
 int pyc_hip_kinfo_small(int tile, int b_trans, int is_bf16, pyc_hip_kinfo* out);
 /* gemm_f32.hip: the LDS-DMA fp32 kernel */
 int pyc_hip_kinfo_f32(int b_trans, pyc_hip_kinfo* out);
