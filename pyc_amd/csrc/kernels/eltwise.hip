@@ -32,6 +32,9 @@ template <> struct io<float> {
     __device__ static inline void put16(float* p, size_t i, const float (&v)[4]) {
         *reinterpret_cast<f32x4*>(p + i) = f32x4{v[0], v[1], v[2], v[3]};
     }
+    __device__ static inline u32x4 pack(const float (&v)[4]) {
+        return u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    }
     __device__ static inline u32x4 raw16(const float* p, size_t i) { return *reinterpret_cast<const u32x4*>(p + i); }
     __device__ static inline void unpack(const u32x4& c, float (&v)[4]) {
 #pragma unroll
@@ -51,12 +54,15 @@ template <typename H> struct io_half {
     }
     __device__ static inline u32x4 raw16(const uint16_t* p, size_t i) { return *reinterpret_cast<const u32x4*>(p + i); }
     __device__ static inline void get16(const uint16_t* p, size_t i, float (&v)[8]) { unpack(raw16(p, i), v); }
-    __device__ static inline void put16(uint16_t* p, size_t i, const float (&v)[8]) {
+    __device__ static inline u32x4 pack(const float (&v)[8]) {
         u32x4 c;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             c[e] = (uint32_t)elem<H>::from_f32(v[2 * e]) | ((uint32_t)elem<H>::from_f32(v[2 * e + 1]) << 16);
-        *reinterpret_cast<u32x4*>(p + i) = c;
+        return c;
+    }
+    __device__ static inline void put16(uint16_t* p, size_t i, const float (&v)[8]) {
+        *reinterpret_cast<u32x4*>(p + i) = pack(v);
     }
 };
 template <> struct io<bf16_t> : io_half<bf16_t> {};
@@ -93,34 +99,32 @@ __device__ inline float gelu_f(float x) {
     return x * (x >= 0.0f ? 1.0f - half_erfc : half_erfc);
 }
 
-// Grid-stride over 16-byte chunks; the n % kVec tail (and unaligned tensors)
-// by elements.
+// One 16-byte chunk per thread, at any alignment (the device runs with unaligned
+// access on; by elements, as unaligned tensors went before, 22.0e6 bf16 took 40 us);
+// the n % kVec tail by elements. Bound: the copy rate. The loads in flight come from the wavefronts
+// (all of a CU's slots), which start and end on their own; more chunks per
+// thread start fewer of them, and a wavefront's chunks then wait for each other.
+// In us, over buffers beyond the caches: one chunk / two / four / the capped grid
+// of 8192 workgroups striding over up to four chunks each that this replaced, bf16:
+// 4 Mi elements 5.3 / 6.0 / 6.4 / 5.8, 22.0e6 17.7 / 19.7 / 21.7 / 19.2, 64 Mi 44.8 /
+// 50.4 / 49.4 / 55.8; fp32 16 Mi 23.5 / 23.5 / 24.1 / 25.8, 64 Mi 87 / 91 / 91 / 103.
 template <typename T>
 __global__ void __launch_bounds__(256) gelu_kernel(const store_t<T>* __restrict__ x, store_t<T>* __restrict__ y,
-                                                   size_t n, int vec_ok) {
+                                                   size_t n) {
     using IO = io<T>;
     constexpr int V = IO::kVec;
     const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    const size_t nchunks = vec_ok ? n / V : 0;
-    // four chunks per thread and iteration: all four loads are issued, as raw
-    // 16-byte words, before any is unpacked (unpacking as each arrives would
-    // wait for the loads one at a time)
-    for (size_t c0 = tid; c0 < nchunks; c0 += 4 * stride) {
-        u32x4 raw[4];
+    const size_t nchunks = n / V;
+    for (size_t c = tid; c < nchunks; c += stride) {
+        u32x4 raw;
+        __builtin_memcpy(&raw, x + c * V, 16);
+        float v[V];
+        IO::unpack(raw, v);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (c0 + u * stride < nchunks) raw[u] = IO::raw16(x, (c0 + u * stride) * V);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (c0 + u * stride < nchunks) {
-                float v[V];
-                IO::unpack(raw[u], v);
-#pragma unroll
-                for (int e = 0; e < V; ++e) v[e] = gelu_f(v[e]);
-                IO::put16(y, (c0 + u * stride) * V, v);
-            }
-        }
+        for (int e = 0; e < V; ++e) v[e] = gelu_f(v[e]);
+        raw = IO::pack(v);
+        __builtin_memcpy(y + c * V, &raw, 16);
     }
     for (size_t i = nchunks * V + tid; i < n; i += stride) IO::put(y, i, gelu_f(IO::get(x, i)));
 }
@@ -390,13 +394,11 @@ __global__ void __launch_bounds__(256) layernorm_row_kernel(const store_t<T>* __
 template <typename T>
 static int launch_gelu(const void* x, void* y, size_t n, hipStream_t s) {
     constexpr int V = io<T>::kVec;
-    const int vec_ok = ((((uintptr_t)x | (uintptr_t)y) & 15) == 0) ? 1 : 0;
-    const size_t work = vec_ok ? (n + V - 1) / V : n;
-    size_t blocks = (work + 255) / 256;
-    if (blocks > 256 * 32) blocks = 256 * 32;  // 32 workgroups per CU, grid-stride beyond
+    size_t blocks = ((n + V - 1) / V + 255) / 256;
+    if (blocks > (1u << 23)) blocks = 1u << 23;  // a launch holds fewer than 2^32 threads; grid-stride beyond
     if (blocks == 0) blocks = 1;
     hipLaunchKernelGGL(gelu_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, s, (const store_t<T>*)x,
-                       (store_t<T>*)y, n, vec_ok);
+                       (store_t<T>*)y, n);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

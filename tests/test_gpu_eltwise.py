@@ -49,8 +49,33 @@ def test_gelu(gpu, name, n):
     assert y[0].item() == 0.0
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("name", ["f32", "bf16", "f16"])
+def test_gelu_chunk_edges(gpu, name, off):
+    """Around one 16-byte chunk, one wavefront's and one workgroup's worth of
+    them, and past 8192 workgroups, on and off 16-byte boundaries; what lies
+    around the output stays as it was. 4096 values, tiled: one oracle result
+    serves every size."""
+    torch = gpu
+    v = 4 if name == "f32" else 8
+    g = torch.Generator(device="cuda").manual_seed(7)
+    tile = (torch.randn(4096, generator=g, device="cuda") * 4.0).to(_tdtype(torch, name))
+    ref = oracle.gelu_f64(tile.float().cpu().numpy())
+    for n in (v - 1, v, v + 1, 64 * v - 1, 64 * v + 1, 256 * v, 256 * v + 1, 8192 * 256 * v + v + 1):
+        x = torch.empty(n + off, dtype=tile.dtype, device="cuda")[off:]
+        x.copy_(tile.repeat((n + 4095) // 4096)[:n])
+        buf = torch.full((n + off + 16,), 7.0, dtype=x.dtype, device="cuda")
+        y = buf[off:off + n]
+        pyc_amd.gelu(x, y)
+        torch.cuda.synchronize()
+        head = min(n, 4096)
+        _check(y[:head].float().cpu().numpy(), ref[:head], name)
+        assert torch.equal(y, y[:head].repeat((n + head - 1) // head)[:n]), n
+        assert bool((buf[:off] == 7.0).all()) and bool((buf[off + n:] == 7.0).all()), n
+
+
 def test_gelu_unaligned(gpu):
-    """A view starting one element into its storage takes the element path."""
+    """A view starting one element into its storage."""
     torch = gpu
     base = torch.randn(4097, device="cuda")
     x = base[1:]
