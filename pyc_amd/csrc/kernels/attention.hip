@@ -617,10 +617,12 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp,
 // other wave of the SIMD (at head dim 64 the other three: two workgroups fit a
 // CU) fills the softmax with its MFMAs. Halves past the last are issued from an
 // empty buffer, so the count of outstanding loads is the same every step.
-// A query's softmax reference m is the maximum of the first block with an
-// unmasked key (m = -inf, l = 0 until then); later blocks exponentiate against
-// it without a maximum, and only when a lane's sum passes 2^14 is m raised where
-// the block's maximum is more than 2^8 above it.
+// A query's softmax reference m is the one of the kernel above, the maximum
+// over its first 64 keys (the blocks of key groups 0 and 1 in step 0, joined
+// through LDS; 0 where none of them has a score above -inf), so that P rounds to
+// 16 bits at the same points in every form. Later blocks exponentiate against it
+// without a maximum, and only when a lane's sum passes 2^14 does the wave raise
+// its own m where the block's maximum is more than 2^8 above it.
 template <int D, int QW> struct AttnSmall {
     static constexpr int KW = 8 / QW;
     static constexpr int ROWS = 32 * KW;                  // keys of a step
@@ -724,7 +726,7 @@ attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K
     for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
+    float m_run = 0.f, l_run = 0.f;
     u32x4 pf[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
 
 #pragma unroll 1
@@ -760,20 +762,21 @@ attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K
                     acc[t] = mfma32x32x16(u32x4{a0[0], a0[1], a1[0], a1[1]}, pf[ks], acc[t], T{});
                 }
         }
-        if (i < n && key0 <= k_last) {
-            const uint16_t* ks = smem + (uint32_t)sk * (Cfg::HALF / 2);
-            f32x16 sc;
+        const bool work = i < n && key0 <= k_last;    // wave-uniform
+        f32x16 sc;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+        // maximum of the block's exponents over all its keys
+        auto block_max = [&]() {
+            float mb = vmax(sc[0], sc[1]);
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk)
-                sc = mfma32x32x16(*reinterpret_cast<const u32x4*>(ks + k_off[kk]), qf[kk], sc, T{});
-            // exponents against m (0 while every key so far was masked); lane
-            // holds keys key0 + 8 (r / 4) + 4 h + r % 4 of query qi
-            const bool fresh = m_run == -INFINITY;
-            const float mref = fresh ? 0.f : m_run;
+            for (int r = 2; r < 16; r += 2) mb = vmax(vmax(mb, sc[r]), sc[r + 1]);
+            return vmax(mb, other_half(mb, xaddr));
+        };
+        // exponents against m; lane holds keys key0 + 8 (r / 4) + 4 h + r % 4 of query qi
+        auto exponents = [&](float mul) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = fmaf(sc[r], scale_log2, -mref);
+            for (int r = 0; r < 16; ++r) sc[r] = fmaf(sc[r], mul, -m_run);
             if ((causal && key0 + 31 > q0) || key0 + 32 > S) {
                 const int thr = (causal ? min(qi, S - 1) : S - 1) - key0 - 4 * h;
 #pragma unroll
@@ -783,25 +786,30 @@ attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K
                     sc[r] = x;
                 }
             }
-            // raises m to the block's maximum where that is far above it, or
-            // where m is not set yet and the block has an unmasked key
-            auto raise = [&](bool unset) {
-                float mb = vmax(sc[0], sc[1]);
+        };
+        if (work) {
+            const uint16_t* ks = smem + (uint32_t)sk * (Cfg::HALF / 2);
 #pragma unroll
-                for (int r = 2; r < 16; r += 2) mb = vmax(vmax(mb, sc[r]), sc[r + 1]);
-                mb = vmax(mb, other_half(mb, xaddr));
-                const bool up = unset ? mb > -INFINITY : mb > kRaise;
-                const float shift = up ? mb : 0.f;
-                const float alpha = unset ? 0.f : __builtin_amdgcn_exp2f(-shift);
-                m_run = up ? mref + mb : m_run;
-                l_run *= alpha;
-#pragma unroll
-                for (int t = 0; t < DT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sc[r] -= shift;
-            };
+            for (int kk = 0; kk < KK; ++kk)
+                sc = mfma32x32x16(*reinterpret_cast<const u32x4*>(ks + k_off[kk]), qf[kk], sc, T{});
+        }
+        float mul = scale_log2;
+        if (i == 0) {
+            // the reference, through the ring slot that step 1 fills (after its barrier)
+            float(*const s_m)[QW][32] =
+                reinterpret_cast<float(*)[QW][32]>(smem + (uint32_t)(SLOTS - 1) * (Cfg::HALF / 2));
+            if (kg < 2) {
+                if (work) exponents(scale_log2);      // m = 0
+                const float mb = work ? block_max() : -INFINITY;
+                if (h == 0) s_m[kg][qg][l32] = mb;
+                mul = 1.f;                            // scaled already
+            }
+            __syncthreads();
+            const float m = vmax(s_m[0][qg][l32], s_m[1][qg][l32]);
+            m_run = m == -INFINITY ? 0.f : m;
+        }
+        if (work) {
+            exponents(mul);
             auto exponentiate = [&]() {
                 float ls[2] = {0.f, 0.f};
 #pragma unroll
@@ -814,11 +822,19 @@ attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K
                 }
                 return ls[0] + ls[1];
             };
-            const bool any_fresh = __any(fresh);
-            if (any_fresh) raise(fresh);
             float lsum = exponentiate();
-            if (!any_fresh && __any(!(lsum <= kAttnFastSumMax))) {
-                raise(false);
+            if (__any(!(lsum <= kAttnFastSumMax))) {
+                const float mb = block_max();
+                const float shift = mb > kRaise ? mb : 0.f;
+                const float alpha = __builtin_amdgcn_exp2f(-shift);
+                m_run += shift;
+                l_run *= alpha;
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] -= shift;
                 lsum = exponentiate();
             }
             l_run += lsum;
@@ -834,18 +850,19 @@ attn_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K
     __syncthreads();
 
     // Join the KW key groups of a query: factor exp2(m_kg - max) / sum
-    float mmax = -INFINITY;
+    float mmax = s_ml[qg][l32].x;
 #pragma unroll
-    for (int g = 0; g < KW; ++g) mmax = fmaxf(mmax, s_ml[g * QW + qg][l32].x);
-    const float mz = mmax == -INFINITY ? 0.f : mmax;
+    for (int g = 1; g < KW; ++g) mmax = fmaxf(mmax, s_ml[g * QW + qg][l32].x);
     float lsum = 0.f;
 #pragma unroll
     for (int g = 0; g < KW; ++g) {
         const float2 ml = s_ml[g * QW + qg][l32];
-        lsum += ml.y * __builtin_amdgcn_exp2f(ml.x - mz);
+        lsum += ml.y * __builtin_amdgcn_exp2f(ml.x - mmax);
     }
-    // m and l of a query with a NaN score are NaN in some group; the sum carries it
-    const float f = __builtin_amdgcn_exp2f(m_run - mz) * (lsum > 0.f || lsum != lsum ? 1.f / lsum : 0.f);
+    // l of a query with a NaN score is NaN in some group and the sum carries it;
+    // a query whose scores are all -inf has lsum = 0 and every partial O 0: NaN,
+    // as the softmax of such a row
+    const float f = __builtin_amdgcn_exp2f(m_run - mmax) * (1.f / lsum);
     // partial O of wave w: 32 rows (queries) of D floats, 16-byte chunk c of row q at c ^ (q & 15)
     f32x4* part = reinterpret_cast<f32x4*>(smem);
     constexpr int CW = D / 4;  // chunks per row

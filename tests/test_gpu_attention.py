@@ -232,3 +232,64 @@ def test_attention_forms(gpu, form, D, causal, case, S):
         assert bool((O[B * H * S * D:] == 3.0).all())
         ref = oracle.attention_f32(*(x.float().cpu().numpy() for x in (Q, K, V)), causal, scale)
         _check(O[:B * H * S * D].float().cpu().numpy().reshape(ref.shape), ref)
+
+
+def _launch_form(form, q, k, v, causal, scale):
+    import ctypes as C
+    torch = __import__("torch")
+    B, H, S, D = q.shape
+    o = torch.empty_like(q)
+    launch = pyc_amd.lib().pyc_hip_attention_launch_form
+    launch.argtypes = [C.c_int] * 7 + [C.c_void_p] * 4 + [C.c_float, C.c_void_p]
+    assert launch(form, int(q.dtype == torch.bfloat16), B, H, S, D, int(causal), q.data_ptr(), k.data_ptr(),
+                  v.data_ptr(), o.data_ptr(), scale, None) == 0
+    torch.cuda.synchronize()
+    return o
+
+
+@pytest.mark.parametrize("form", [2, 4])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("S", [20, 64, 70, 1000])
+def test_attention_forms_round_alike(gpu, form, D, causal, S):
+    """The small forms round the probabilities at the same points as the
+    persistent one (the same reference per query), so their outputs differ only
+    where the order of the fp32 sums moves a result across a rounding boundary: a
+    sum of S terms is off by about 2^-24 sqrt(S) relative to its largest terms,
+    2e-6 at S = 1000, which crosses a boundary of 16-bit results (2^-8 / 2^-11
+    apart) for about one in 1000 / 100 of them. Bounds: four times that share."""
+    torch = gpu
+    for t, share in ((torch.bfloat16, 0.004), (torch.float16, 0.04)):
+        g = torch.Generator(device="cuda").manual_seed(S + D)
+        q, k, v = (torch.randn((2, 5, S, D), generator=g, device="cuda").to(t) for _ in range(3))
+        a, b = (_launch_form(f, q, k, v, causal, D ** -0.5) for f in (1, form))
+        assert float((a != b).float().mean()) <= share
+        eps = 2.0 ** (-7 if t == torch.bfloat16 else -10)
+        af, bf = a.float(), b.float()
+        assert bool(((af - bf).abs() <= eps * af.abs() + 1e-5 * af.abs().max()).all())
+
+
+@pytest.mark.parametrize("form", [2, 4])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S", [40, 300])
+def test_attention_small_forms_not_finite(gpu, form, D, S):
+    """Scores of -inf (keys with an infinite component): they count as no key; a
+    query all of whose scores are -inf is NaN, as the softmax of that row. A NaN or
+    +inf score makes its query NaN and no other; against float64."""
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    for t, tol in ((torch.bfloat16, 2e-2), (torch.float16, 2e-3)):
+        q, k, v = (torch.randn((1, 4, S, D), generator=g, device="cuda").to(t) for _ in range(3))
+        q[..., 0] = 1.0
+        k[0, 0, :min(S, 64), 0] = -float("inf")    # the keys that set the reference (all of them at S = 40)
+        k[0, 1, 33:, 0] = -float("inf")            # keys after it
+        q[0, 2, 5, 3] = float("nan")
+        k[0, 2, S - 1, 1] = float("inf")           # +-inf by the sign of the query's component
+        q[0, 3, 7, 0] = float("inf")               # inf, -inf or NaN scores for one query
+        s = D ** -0.5
+        p = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * s
+        ref = torch.matmul(torch.softmax(p, -1), v.double())
+        o = _launch_form(form, q, k, v, False, s).double()
+        assert torch.equal(torch.isnan(o), torch.isnan(ref))
+        ok = ~torch.isnan(ref)
+        assert float((o - ref)[ok].abs().max()) <= tol * float(ref[ok].abs().max())
