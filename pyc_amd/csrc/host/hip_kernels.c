@@ -28,6 +28,11 @@ int pyc_hip_gemm_half_launch(int is_bf16, int b_trans, int tile, int M, int N, i
 int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
                               const void* B, void* C, float alpha, float beta, const float* bias, int epi, int m0,
                               int m1, int n0, int n1, void* stream);
+int pyc_hip_gemm_small_takes(int b_trans, int M, int N, int K, const void* A, const void* B);
+int pyc_hip_gemm_nt_lds_takes(int M, int N, int K, const void* A, const void* B, const void* C, float beta,
+                              const float* bias, int epi);
+int pyc_hip_gemm_nn_lds_takes(int ragged, int M, int N, int K, const void* A, const void* B, const void* C, float beta,
+                              const float* bias, int epi);
 int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B, void* C,
                                float alpha, float beta, const float* bias, int epi, int m_end, int n_end,
                                void* stream);
@@ -332,6 +337,51 @@ static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_on
     return p;
 }
 
+/* The plan of a half GEMM on LDS-DMA tiles, made before anything is launched
+ * from what each kernel says it takes: both parts run once the first has. 0 when
+ * none of them takes the product (the general register-staged tiles do).
+ *  - Operands that LDS-DMA can move in whole chunks: every tile.
+ *  - Others (bases off a 16-byte boundary, odd rows): the 256 x 256 kernels for
+ *    all of C where they give every CU a tile, else tiles up to 128 x 128. */
+static int plan_gemm(int b_trans, int M, int N, int K, const void* A, const void* B, const void* C, float beta,
+                     const float* bias, int epi, dma_plan* p) {
+    const int small = pyc_hip_gemm_small_takes(b_trans, M, N, K, A, B);
+    const int big = b_trans ? pyc_hip_gemm_nt_lds_takes(M, N, K, A, B, C, beta, bias, epi)
+                            : 2 * pyc_hip_gemm_nn_lds_takes(1, M, N, K, A, B, C, beta, bias, epi);
+    const int fills = pick_half_tile(M, N) == 256;
+    if (small < 2 && big > 0 && fills) {
+        p->t = DT_256;
+        p->rest = -1;
+        p->m_end = M;
+        p->n_end = N;
+        return 1;
+    }
+    if (small == 0) {
+        return 0;
+    }
+    const int last = small < 2 ? DT_128 : big > 0 ? DT_256 : DT_128X256;
+    *p = plan_dma(M, N, K, !b_trans, 0, 0, last, last);
+    return 1;
+}
+
+/* plan_gemm for the shape-chosen symbols, as tile edges: out = {rows and columns of
+ * the first part's tile, of the second's (0, 0: one launch), m_end, n_end}. Returns
+ * what plan_gemm does. Host only; the pointers are looked at for their alignment. */
+int pyc_hip_gemm_plan(int b_trans, int M, int N, int K, const void* A, const void* B, const void* C, float beta,
+                      const float* bias, int epi, int* out) {
+    dma_plan p;
+    if (M <= 0 || N <= 0 || K <= 0 || !out || !plan_gemm(b_trans, M, N, K, A, B, C, beta, bias, epi, &p)) {
+        return 0;
+    }
+    out[0] = k_dma_tiles[p.t].bm;
+    out[1] = k_dma_tiles[p.t].bn;
+    out[2] = p.rest < 0 ? 0 : k_dma_tiles[p.rest].bm;
+    out[3] = p.rest < 0 ? 0 : k_dma_tiles[p.rest].bn;
+    out[4] = p.m_end;
+    out[5] = p.n_end;
+    return 1;
+}
+
 static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, const void* B,
                     void* C, float alpha, float beta, const float* bias, int epilogue, void* stream) {
     if (!v || M <= 0 || N <= 0 || K <= 0 || !A || !B || !C) {
@@ -363,18 +413,11 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
             return -1;
         }
     }
-    /* The shape-chosen symbols: the LDS-DMA tile that the table above makes the
-     * cheapest. A launcher answers 1 when the shape is outside its kernel's
-     * preconditions (K % 64 and beta == 0 for the persistent 256 x 256 tile,
-     * operands that LDS-DMA can move for 128 x 256); then the next smaller kind
-     * is asked. Operands off a 16-byte boundary go to the persistent tile only
-     * where they always did, with a tile for every CU. */
+    /* The shape-chosen symbols: the tiles that the table above makes the cheapest. */
     if (v->tile == 0) {
         const int bf = v->dtype == VT_BF16;
-        const int off16 = (int)(((uintptr_t)A | (uintptr_t)B) & 15) != 0;
-        int last = off16 && pick_half_tile(M, N) != 256 ? DT_128X256 : DT_256;
-        for (; last >= DT_128; --last) {
-            const dma_plan p = plan_dma(M, N, K, !v->b_trans, 0, 0, last, last);
+        dma_plan p;
+        if (plan_gemm(v->b_trans, M, N, K, A, B, C, beta, bias, epilogue, &p)) {
             const dma_tile* d = &k_dma_tiles[p.t];
             int rc;
             if (p.t == DT_256) {
@@ -391,14 +434,13 @@ static int gemm_run(const hip_variant* v, int M, int N, int K, const void* A, co
                 rc = pyc_hip_gemm_small_launch(bf, v->b_trans, d->bm, d->bn, M, N, K, A, B, C, alpha, beta, bias,
                                                epilogue, p.m_end < M ? p.m_end : 0, M, p.n_end < N ? p.n_end : 0, N,
                                                stream);
+                if (rc == 1) {
+                    return -2; /* the first part has run: starting again would add beta * C to it twice */
+                }
             }
             if (rc != 1) {
                 return rc;
             }
-            if (p.t < DT_128X256) {
-                break;
-            }
-            last = p.t;
         }
     }
     return pyc_hip_gemm_half_launch(v->dtype == VT_BF16, v->b_trans, v->tile > 0 ? v->tile : pick_half_tile(M, N),

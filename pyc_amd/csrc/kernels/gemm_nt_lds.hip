@@ -895,25 +895,41 @@ static int launch_ragged(int is_bf16, int M, int N, int K, const void* A, const 
 
 }  // namespace pyc
 
-// Rows 0 .. m_end - 1 and columns 0 .. n_end - 1 of C (each whole tiles, or all).
-// Returns 1 when the shape is outside these kernels' preconditions (the caller
-// uses another variant), 0 on launch, -2 on a launch error. Full-tile shapes
-// with beta == 0 take the persistent kernel; PYC_GEMM_NT_PERSIST=0 forces the
-// one-shot kernel (for comparisons).
-extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B,
-                                          void* C, float alpha, float beta, const float* bias, int epi, int m_end,
-                                          int n_end, void* stream) {
+// What runs a product with B stored [N,K] here (host only, no launch): 0 = none
+// (K no multiple of 64, operands past 32-bit byte counts), 1 = the one-shot
+// kernel, 2 = the persistent kernel, in its ragged form where M or N is no
+// multiple of 256. beta == 0, with C and bias on 16-byte boundaries, is the
+// persistent kernel's; PYC_GEMM_NT_PERSIST=0 forces the one-shot kernel (for
+// comparisons).
+extern "C" int pyc_hip_gemm_nt_lds_takes(int M, int N, int K, const void* A, const void* B, const void* C, float beta,
+                                         const float* bias, int epi) {
     using namespace pyc;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 1;
-    if (m_end <= 0 || m_end > M || n_end <= 0 || n_end > N) return 1;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
     // buffer descriptors hold 32-bit byte counts
-    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
+    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 0;
     static int persist_env = -1;
-    static int n_cu = 0;
     if (persist_env < 0) {
         const char* e = getenv("PYC_GEMM_NT_PERSIST");
         persist_env = (e && e[0] == '0') ? 0 : 1;
     }
+    if (!persist_env) return 1;
+    if (M % kD_BM || N % kD_BN) return ragged_ok(M, N, K, A, B, C, beta, bias, epi) ? 2 : 1;
+    return beta == 0.f && ((uintptr_t)C & 15) == 0 &&
+                   ((epi & 1) == 0 || bias == nullptr || ((uintptr_t)bias & 15) == 0)
+               ? 2
+               : 1;
+}
+
+// Rows 0 .. m_end - 1 and columns 0 .. n_end - 1 of C (each whole tiles, or all).
+// Returns 1 when the shape is outside these kernels' preconditions (the caller
+// uses another variant), 0 on launch, -2 on a launch error.
+extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, const void* A, const void* B,
+                                          void* C, float alpha, float beta, const float* bias, int epi, int m_end,
+                                          int n_end, void* stream) {
+    using namespace pyc;
+    const int form = pyc_hip_gemm_nt_lds_takes(M, N, K, A, B, C, beta, bias, epi);
+    if (form == 0 || m_end <= 0 || m_end > M || n_end <= 0 || n_end > N) return 1;
+    static int n_cu = 0;
     if (n_cu == 0) {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
@@ -925,17 +941,15 @@ extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, cons
     const int tiles_m = (m_end + kD_BM - 1) / kD_BM;
     const int tiles_n = (n_end + kD_BN - 1) / kD_BN;
     const int ntiles = tiles_m * tiles_n;
-    if (persist_env && (M % kD_BM || N % kD_BN) && ragged_ok(M, N, K, A, B, C, beta, bias, epi))
+    if (form == 2 && (M % kD_BM || N % kD_BN))
         return launch_ragged<false>(is_bf16, M, N, K, A, B, C, alpha, bias, epi, m_end, n_end, n_cu,
                                     (hipStream_t)stream);
-    const bool persist = persist_env && M % kD_BM == 0 && N % kD_BN == 0 && beta == 0.f &&
-                         ((uintptr_t)C & 15) == 0 && ((epi & 1) == 0 || bias == nullptr || ((uintptr_t)bias & 15) == 0);
     hipStream_t s = (hipStream_t)stream;
     const dim3 block(4 * kWave);
     const uint16_t* a = (const uint16_t*)A;
     const uint16_t* b = (const uint16_t*)B;
     uint16_t* c = (uint16_t*)C;
-    if (persist) {
+    if (form == 2) {
         const int pepi = (((epi & 1) && bias != nullptr) ? 1 : 0) | (epi & 2);
         const dim3 grid(ntiles < n_cu ? ntiles : n_cu);
 #define PYC_PERSIST(TY, E) \
@@ -965,21 +979,30 @@ extern "C" int pyc_hip_gemm_nt_lds_launch(int is_bf16, int M, int N, int K, cons
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// NN form (B stored [K,N]) of the persistent kernel: returns 1 when the shape
-// is outside its preconditions (M, N multiples of 256, K of 64, beta == 0,
-// 16-byte aligned C and bias, M*K*2 and K*N*2 below 2^32, at least as many
-// 256 x 256 tiles as CUs; with `ragged` those of ragged_ok instead of the
-// first, and any number of tiles), 0 on launch, -2 on a launch error.
+// 1 when the NN form (B stored [K,N]) of the persistent kernel runs a product
+// (host only, no launch): M, N multiples of 256, K of 64, beta == 0, 16-byte
+// aligned C and bias, M*K*2 and K*N*2 below 2^32; with `ragged` the ones of
+// ragged_ok instead of the first two.
+extern "C" int pyc_hip_gemm_nn_lds_takes(int ragged, int M, int N, int K, const void* A, const void* B, const void* C,
+                                         float beta, const float* bias, int epi) {
+    using namespace pyc;
+    if (M <= 0 || N <= 0 || K <= 0 || beta != 0.f) return 0;
+    const bool whole = M % kD_BM == 0 && N % kD_BN == 0 && K % 64 == 0;
+    if (!whole && !(ragged && ragged_ok(M, N, K, A, B, C, beta, bias, epi))) return 0;
+    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 0;
+    return ((uintptr_t)C & 15) == 0 && ((epi & 1) == 0 || bias == nullptr || ((uintptr_t)bias & 15) == 0);
+}
+
+// Returns 1 when the shape is outside the kernel's preconditions (above; without
+// `ragged` also at least as many 256 x 256 tiles as CUs), 0 on launch, -2 on a
+// launch error.
 extern "C" int pyc_hip_gemm_nn_lds_launch(int is_bf16, int ragged, int M, int N, int K, const void* A,
                                           const void* B, void* C, float alpha, float beta, const float* bias,
                                           int epi, int m_end, int n_end, void* stream) {
     using namespace pyc;
-    if (M <= 0 || N <= 0 || K <= 0 || beta != 0.f) return 1;
+    if (!pyc_hip_gemm_nn_lds_takes(ragged, M, N, K, A, B, C, beta, bias, epi)) return 1;
     if (m_end <= 0 || m_end > M || n_end <= 0 || n_end > N) return 1;
-    const bool whole = M % kD_BM == 0 && N % kD_BN == 0 && K % 64 == 0;
-    if (!whole && !(ragged && ragged_ok(M, N, K, A, B, C, beta, bias, epi))) return 1;
-    if ((size_t)M * K * 2 > 0xFFFFFFFFull || (size_t)N * K * 2 > 0xFFFFFFFFull) return 1;
-    if (((uintptr_t)C & 15) != 0 || ((epi & 1) && bias != nullptr && ((uintptr_t)bias & 15) != 0)) return 1;
+    const bool whole = M % kD_BM == 0 && N % kD_BN == 0;  // (K is a multiple of 64 in both forms)
     static int n_cu = 0;
     if (n_cu == 0) {
         int dev = 0, cus = 0;

@@ -489,26 +489,33 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
 
 }  // namespace pyc
 
+// Which of these tiles run a product (host only, no launch): 2 = all of them, by
+// LDS-DMA (K a multiple of 8 and, for [K,N] B, N of 4, with A and B 16-byte
+// aligned and below 4 GiB), 1 = those up to 128 x 128, staged through registers
+// (rows of at least 8 elements), 0 = none.
+extern "C" int pyc_hip_gemm_small_takes(int b_trans, int M, int N, int K, const void* A, const void* B) {
+    using namespace pyc;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
+    if (K % 8 || (!b_trans && N % 4) || (((uintptr_t)A | (uintptr_t)B) & 15) || (size_t)M * K * 2 > kSmPastEnd ||
+        (size_t)N * K * 2 > kSmPastEnd || ((K % kSmBK || !b_trans) && (size_t)N * kpad * 2 > kSmPastEnd))
+        return K < 8 || (!b_trans && N < 8) ? 0 : 1;
+    return 2;
+}
+
 // bm x bn: one of the tiles above; m0 .. n1: the part of C (SmPart). Rows of A (and of [N,K] B) past the end are
 // read as zeros through the buffer descriptors, [K,N] B columns past N read
 // neighbouring data, and only the rows and columns of C inside M x N are
-// written. LDS-DMA takes K a multiple of 8 and, for [K,N] B, N of 4, with A and
-// B 16-byte aligned and below 4 GiB; other shapes are staged through registers,
-// up to 128 x 128 tiles, with rows of at least 8 elements. Returns 1 for an
-// unknown tile (128 x 256 for a shape that is register-staged) and for shorter
-// rows, 0 on launch, -2 on a launch error.
+// written. Returns 1 for an unknown tile and for one that does not take the
+// product (pyc_hip_gemm_small_takes), 0 on launch, -2 on a launch error.
 extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int bn, int M, int N, int K, const void* A,
                                          const void* B, void* C, float alpha, float beta, const float* bias,
                                          int epi, int m0, int m1, int n0, int n1, void* stream) {
     using namespace pyc;
-    if (M <= 0 || N <= 0 || K <= 0) return 1;
+    const int takes = pyc_hip_gemm_small_takes(b_trans, M, N, K, A, B);
+    if (takes == 0) return 1;
     const SmPart pt{m0, m1, n0, n1};
-    const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
-    const bool tail = K % kSmBK != 0;
-    const bool any = K % 8 || (!b_trans && N % 4) || (((uintptr_t)A | (uintptr_t)B) & 15) ||
-                     (size_t)M * K * 2 > kSmPastEnd || (size_t)N * K * 2 > kSmPastEnd ||
-                     ((tail || !b_trans) && (size_t)N * kpad * 2 > kSmPastEnd);
-    if (any && (K < 8 || (!b_trans && N < 8))) return 1;
+    const bool any = takes == 1, tail = K % kSmBK != 0;
     hipStream_t s = (hipStream_t)stream;
     const SmConv cg{};
 #define PYC_GO(TY, BT)                                                                                              \

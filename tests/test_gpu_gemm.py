@@ -604,3 +604,52 @@ def test_gemm_in_two_parts(gpu, m, n, k, layout):
     bad = ~((Cd[:m * n].view(m, n).float() - ref).abs() <=
             2.0 ** -8 * ref.abs() + 4e-6 * np.sqrt(k) * ref.abs().max())
     assert not bool(bad.any()), int(bad.sum())
+
+
+def _plan(bt, m, n, k, A, B, C_, beta, bias):
+    out = (C.c_int * 6)()
+    f = pyc_amd.lib().pyc_hip_gemm_plan
+    f.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.c_float, C.c_void_p, C.c_int, C.c_void_p]
+    assert f(int(bt), m, n, k, A, B, C_, beta, bias, 1, out) == 1
+    return tuple(out)
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("m,n,k,beta,off_a,off_c,plan", [
+    (1999, 11008, 4096, 0.0, 0, 0, (256, 256, 128, 256, 1999, 8192)),  # by columns
+    (1999, 11008, 4096, 0.5, 0, 0, None),    # [N,K]: the one-shot kernel on part of C
+    (1999, 11008, 4096, -1.0, 0, 3, None),   # and C off an 8-byte boundary
+    (5000, 8192, 4096, 0.0, 0, 0, (256, 256, 128, 256, 4096, 8192)),   # by rows
+    (5000, 8192, 4096, 0.5, 0, 0, None),
+    (4608, 4608, 1024, 1.0, 4, 0, None),     # A off a 16-byte boundary: one launch
+    (2500, 2200, 136, 0.5, 1, 0, None),      # register-staged tiles
+])
+def test_gemm_parts_as_planned(gpu, m, n, k, beta, off_a, off_c, plan, layout):
+    """Products whose plan has two parts (asserted where one is given; with beta or
+    operands off a 16-byte boundary it may have one): every element once, with beta * C
+    added once, and nothing past C."""
+    torch = gpu
+    bt = layout == "nt"
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    Ab = torch.zeros(m * k + 8, dtype=torch.bfloat16, device="cuda")
+    A = Ab[off_a:off_a + m * k].view(m, k)
+    A.copy_(torch.randn((m, k), generator=g, device="cuda") / np.sqrt(k))
+    B = torch.randn((n, k) if bt else (k, n), generator=g, device="cuda").bfloat16()
+    bias = torch.randn(n, generator=g, device="cuda")
+    Cb = torch.randn(m * n + 4096, generator=g, device="cuda").bfloat16()
+    C0 = Cb.clone()
+    Cd = Cb[off_c:]
+    got_plan = _plan(bt, m, n, k, A.data_ptr(), B.data_ptr(), Cd.data_ptr(), beta, bias.data_ptr())
+    if plan:
+        assert got_plan == plan
+    else:
+        assert not (off_a and got_plan[0] == 256 and got_plan[2])
+    pyc_amd.gemm(f"hip_gemm_bf16_{layout}", A, B, Cd, m, n, k, beta=beta, bias=bias, epilogue=1)
+    torch.cuda.synchronize()
+    end = off_c + m * n
+    assert torch.equal(Cb[:off_c], C0[:off_c]) and torch.equal(Cb[end:], C0[end:])
+    ref = A.float() @ (B.float().t() if bt else B.float()) + bias + beta * C0[off_c:end].view(m, n).float()
+    # one rounding of the result (2^-8 relative) plus fp32 summation order
+    bad = ~((Cb[off_c:end].view(m, n).float() - ref).abs() <=
+            2.0 ** -8 * ref.abs() + 4e-6 * np.sqrt(k) * ref.abs().max())
+    assert not bool(bad.any()), int(bad.sum())
