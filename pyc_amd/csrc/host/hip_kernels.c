@@ -340,7 +340,12 @@ static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_on
 /* The plan of a half GEMM on LDS-DMA tiles, made before anything is launched
  * from what each kernel says it takes: both parts run once the first has. 0 when
  * none of them takes the product (the general register-staged tiles do).
- *  - Operands that LDS-DMA can move in whole chunks: every tile.
+ *  - Operands that LDS-DMA can move in whole chunks: every tile, and 256 x 256
+ *    where the table describes it: the persistent kernel, or the one-shot kernel
+ *    ([N,K] only) with plain whole-chunk stores. With beta or a C that takes
+ *    narrow stores the one-shot kernel ends far later and stays where it gives
+ *    every CU a tile (us, one-shot / the smaller tiles: 3072 x 4096 x 2048 with beta
+ *    89 / 69, 3001 x 4096 x 1024 67 / 46, C off 16 bytes 56 / 35).
  *  - Others (bases off a 16-byte boundary, odd rows): the 256 x 256 kernels for
  *    all of C where they give every CU a tile, else tiles up to 128 x 128. */
 static int plan_gemm(int b_trans, int M, int N, int K, const void* A, const void* B, const void* C, float beta,
@@ -359,7 +364,8 @@ static int plan_gemm(int b_trans, int M, int N, int K, const void* A, const void
     if (small == 0) {
         return 0;
     }
-    const int last = small < 2 ? DT_128 : big > 0 ? DT_256 : DT_128X256;
+    const int plain = beta == 0.0f && ((uintptr_t)C & 15) == 0 && N % 8 == 0;
+    const int last = small < 2 ? DT_128 : big == 2 || (big == 1 && (fills || plain)) ? DT_256 : DT_128X256;
     *p = plan_dma(M, N, K, !b_trans, 0, 0, last, last);
     return 1;
 }

@@ -121,3 +121,15 @@ def test_every_call_computes_each_element_once(dispatch):
         _once(parts, m, n)
         split += len(parts) == 2
     assert split > 50
+
+
+@pytest.mark.parametrize("m,n,k", [(3072, 4096, 2048), (3001, 4096, 1024), (1024, 4096, 4096)])
+def test_one_shot_kernel_only_with_a_tile_per_cu(dispatch, m, n, k):
+    """[N,K] products with beta, or with C off a 16-byte boundary, cannot take the
+    persistent kernel; the one-shot kernel is slower than smaller tiles for them unless
+    the 256 x 256 tiles fill the chip."""
+    for kw in (dict(beta=0.5), dict(c_off=8), dict(c_off=8, bias_off=4)):
+        rc, parts = _run(dispatch, True, m, n, k, **kw)
+        assert rc == 0 and all(p[0] == 1 for p in parts), (kw, parts)
+    rc, parts = _run(dispatch, True, 4096, 4096, k, beta=0.5)
+    assert rc == 0 and parts[0][:2] == (2, 1)
