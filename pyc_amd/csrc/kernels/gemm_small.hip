@@ -527,10 +527,25 @@ extern "C" int pyc_hip_gemm_small_launch(int is_bf16, int b_trans, int bm, int b
 #undef PYC_GO
 }
 
+// Reciprocals of a filter's tap split: k / C and t / S by a multiplication with the
+// rounded-up rc = ceil(2^32 / C) and rs = ceil(2^32 / S) (*rs 0 for S == 1: no
+// division). x * ceil(2^32 / d) is x * e / 2^32 above x / d * 2^32, with e =
+// d * ceil(2^32 / d) - 2^32, so floor is exact while x * e < 2^32. Returns 1 where
+// that holds for every k < R*S*C and every tap t < R*S, else 0. Host only.
+extern "C" int pyc_hip_conv2d_tap_split(int R, int S, int C, uint32_t* rc, uint32_t* rs) {
+    const uint64_t two32 = 1ull << 32;
+    if (R <= 0 || S <= 0 || C <= 1 || (uint64_t)R * S > 0x7FFFFFFFull / C) return 0;
+    const uint64_t taps = (uint64_t)R * S, c = (uint64_t)C, s = (uint64_t)S;
+    const uint64_t qc = (two32 + c - 1) / c, qs = (two32 + s - 1) / s;
+    *rc = (uint32_t)qc;
+    *rs = S == 1 ? 0u : (uint32_t)qs;
+    return taps * c * c < two32 && (taps - 1) * (qs * s - two32) < two32;  // (e < C)
+}
+
 // NHWC convolution on the same tiles (bm output pixels x bn output channels),
 // output pixels m0 .. m1 - 1.
 // Returns 1 outside its preconditions (C % 8 == 0, x and w 16-byte aligned and
-// below 4 GiB, reciprocals exact: R*S*C * C < 2^32), 0 on launch, -2 on a
+// below 4 GiB, exact reciprocals: pyc_hip_conv2d_tap_split), 0 on launch, -2 on a
 // launch error.
 extern "C" int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg, int H, int W, int C, int Kout,
                                            int R, int S, int ph, int pw, int sh, int sw, const void* x,
@@ -541,13 +556,12 @@ extern "C" int pyc_hip_conv2d_small_launch(int is_bf16, int bm, int bn, int Nimg
     const long long M = (long long)Nimg * P * Q, Kg = (long long)R * S * C;
     const unsigned long long lim = kSmPastEnd;
     if (C % 8 || P <= 0 || Q <= 0 || M > 0x7FFFFF00LL || Kg > 0x7FFFFF00LL) return 1;
-    if ((unsigned long long)Kg * C >= (1ull << 32)) return 1;
+    uint32_t rc = 0, rs = 0;
+    if (!pyc_hip_conv2d_tap_split(R, S, C, &rc, &rs)) return 1;
     if ((unsigned long long)Nimg * H * W * C * 2 > lim || (unsigned long long)Kout * Kg * 2 > lim) return 1;
     if (H >= (1 << 28) || W >= (1 << 28) || ph >= (1 << 28) || pw >= (1 << 28)) return 1;
     if (((uintptr_t)x | (uintptr_t)w) & 15) return 1;
-    const SmConv cg{H, W, C, S, (int)P, (int)Q, ph, pw, sh, sw, (uint32_t)(((1ull << 32) + C - 1) / C),
-                    S == 1 ? 0u : (uint32_t)(((1ull << 32) + S - 1) / S),
-                    (uint32_t)((size_t)Nimg * H * W * C * 2)};
+    const SmConv cg{H, W, C, S, (int)P, (int)Q, ph, pw, sh, sw, rc, rs, (uint32_t)((size_t)Nimg * H * W * C * 2)};
     const SmPart pt{m0, m1 > 0 ? m1 : (int)M, 0, Kout};  // m1 <= 0: to the last pixel
     const int epi = (bias ? 1 : 0) | (relu ? 2 : 0);
     hipStream_t st = (hipStream_t)stream;
