@@ -1203,6 +1203,10 @@ struct W8Plan {
 // register-direct one (items of 64 k).
 bool w8_use_lds(int K) { return K % pyc::kQK == 0; }
 
+// LDS-DMA moves 16-byte chunks of X and W from 16-byte boundaries (rows keep them:
+// K % 16 == 0). A layer whose operands lie elsewhere is loaded through registers.
+bool w8_aligned(const void* X, const void* Wq) { return (((uintptr_t)X | (uintptr_t)Wq) & 15) == 0; }
+
 W8Plan w8_split(int units, int ksteps, int n_wg) {
     W8Plan p;
     p.units = units;
@@ -1219,9 +1223,9 @@ W8Plan w8_split(int units, int ksteps, int n_wg) {
     return p;
 }
 
-W8Plan w8_plan(int N, int K, int n_wg) {
+W8Plan w8_plan(int N, int K, int n_wg, bool lds) {
     const int units = (N + pyc::kW8Rows - 1) / pyc::kW8Rows;
-    if (!w8_use_lds(K)) return w8_split(units, (K + pyc::kW8K - 1) / pyc::kW8K, n_wg);
+    if (!lds) return w8_split(units, (K + pyc::kW8K - 1) / pyc::kW8K, n_wg);
     // the LDS kernel reduces at most 8 partial slots per unit: use fewer
     // workgroups (longer runs) when K is so deep that more would share a unit
     W8Plan p = w8_split(units, K / pyc::kQK, n_wg);
@@ -1271,7 +1275,7 @@ bool w8_reserve(const W8Plan& p) {
 // outside any stream capture (callers that capture launches call this first).
 extern "C" int pyc_hip_w8a16_reserve(int N, int K) {
     if (N <= 0 || K <= 0) return -1;
-    return w8_reserve(w8_plan(N, K, cu_count())) ? 0 : -2;
+    return w8_reserve(w8_plan(N, K, cu_count(), w8_use_lds(K))) ? 0 : -2;
 }
 
 namespace {
@@ -1289,9 +1293,9 @@ size_t w8_token_lds(int M, int K) { return (size_t)M * ((K / 16 + pyc::kWave - 1
 
 bool w8_token_fits(int M, int K) { return M <= 4 && w8_token_lds(M, K) <= pyc::kTokLdsMax; }
 
-// 32-bit byte offsets, also of the rows a last unit has past N
-bool w8_own_fits(int N, int K) {
-    return ((size_t)N + 64) * K < 0xFFFFFFF0ull && (size_t)32 * K * 2 < 0xFFFFFFF0ull;
+// LDS-DMA, with 32-bit byte offsets, also of the rows a last unit has past N
+bool w8_own_fits(int N, int K, const void* X, const void* Wq) {
+    return ((size_t)N + 64) * K < 0xFFFFFFF0ull && (size_t)32 * K * 2 < 0xFFFFFFF0ull && w8_aligned(X, Wq);
 }
 
 double w8_token_cost(int M, int N, int K) { return 2.6 + (double)N * K / 5.9e6 * (1.0 + 0.15 * (M - 1)); }
@@ -1307,14 +1311,15 @@ double w8_own_cost(int ub, int M, int N, int K) {
 double w8_split_cost(int N, int K) { return 11.0 + 0.058 * ((double)N * K / 256.0 / 1000.0); }
 
 // The cheapest kernel that splits no row over workgroups: 0 = token, 1..4 = own
-// with that UB; -1 where neither can (offsets past 32 bits). *cost: its estimate.
-int w8_whole_form(int M, int N, int K, double* cost) {
+// with that UB; -1 where neither can (for own: offsets past 32 bits, operands off a
+// 16-byte boundary). *cost: its estimate.
+int w8_whole_form(int M, int N, int K, const void* X, const void* Wq, double* cost) {
     int form = -1;
     if (w8_token_fits(M, K)) {
         form = 0;
         *cost = w8_token_cost(M, N, K);
     }
-    if (w8_own_fits(N, K)) {
+    if (w8_own_fits(N, K, X, Wq)) {
         for (int ub = 1; ub <= 4; ++ub) {
             const double c = w8_own_cost(ub, M, N, K);
             if (form < 0 || c < *cost) {
@@ -1369,21 +1374,27 @@ int w8_whole_launch(int form, int M, int N, int K, const void* X, const void* Wq
 
 }  // namespace
 
-// form: -1 = the cheapest by estimate, 0 = token kernel, 1 .. 4 = whole-K kernel
-// with that UB, 5 = split-K kernel; -1 is returned where the form cannot run.
+// The kernel a layer takes: 0 = token kernel, 1 .. 4 = whole-K kernel with that UB,
+// 5 = split-K kernel through LDS, 6 = split-K kernel through registers. Host only;
+// the pointers are looked at for their alignment.
+extern "C" int pyc_hip_w8a16_form(int M, int N, int K, const void* X, const void* Wq) {
+    double whole = 0.0;
+    const int form = w8_whole_form(M, N, K, X, Wq, &whole);
+    if (form >= 0 && whole < w8_split_cost(N, K)) return form;
+    return w8_use_lds(K) && w8_aligned(X, Wq) ? 5 : 6;
+}
+
+// form: -1 = pyc_hip_w8a16_form's, or one of its forms (5 is 6 where LDS-DMA cannot
+// load the operands); -1 is returned where the form cannot run.
 extern "C" int pyc_hip_w8a16_launch_form(int form, int M, int N, int K, const void* X, const void* Wq,
                                          const float* scale, int relu, void* Y, void* stream) {
     using namespace pyc;
     hipStream_t s = (hipStream_t)stream;
-    if (form < 0) {
-        double whole = 0.0;
-        form = w8_whole_form(M, N, K, &whole);
-        if (form < 0 || whole >= w8_split_cost(N, K)) form = 5;
-    } else if (form == 0 ? !w8_token_fits(M, K) : form < 5 ? !w8_own_fits(N, K) : form > 5) {
-        return -1;
-    }
+    if (form < 0) form = pyc_hip_w8a16_form(M, N, K, X, Wq);
+    else if (form == 0 ? !w8_token_fits(M, K) : form < 5 ? !w8_own_fits(N, K, X, Wq) : form > 6) return -1;
     if (form < 5) return w8_whole_launch(form, M, N, K, X, Wq, scale, relu, Y, s);
-    W8Plan p = w8_plan(N, K, cu_count());
+    const bool lds = form == 5 && w8_use_lds(K) && w8_aligned(X, Wq);
+    W8Plan p = w8_plan(N, K, cu_count(), lds);
     float* part = nullptr;
     int* cnt = nullptr;
     if (p.max_slots > 1) {
@@ -1399,14 +1410,14 @@ extern "C" int pyc_hip_w8a16_launch_form(int form, int M, int N, int K, const vo
             cnt = g_w8ws[dev].cnt;
         } else {
             // no workspace: whole units per workgroup
-            const int ksteps = (K + (w8_use_lds(K) ? kQK : kW8K) - 1) / (w8_use_lds(K) ? kQK : kW8K);
+            const int ksteps = (K + (lds ? kQK : kW8K) - 1) / (lds ? kQK : kW8K);
             p.G = p.units;
             p.base = ksteps;
             p.rem = 0;
             p.max_slots = 1;
         }
     }
-    if (w8_use_lds(K))
+    if (lds)
         hipLaunchKernelGGL(w8a16_lds_kernel, dim3(p.G), dim3(kQWaves * kWave), 0, s, (const uint16_t*)X,
                            (const uint8_t*)Wq, scale, (uint16_t*)Y, M, N, K, relu, p.base, p.rem, part, cnt,
                            p.max_slots);
@@ -1470,7 +1481,7 @@ int chain_layout(int M, int nsteps, const int* N, const int* K, ChainLayout& L, 
         if (N[s] / pyc::kW8Rows > kChainMaxUnits) return -1;
         if (s > 0 && K[s] != N[s - 1]) return -1;
         if ((size_t)N[s] * K[s] >= 0xFFFFFFFFull || (size_t)M * K[s] * 2 >= 0xFFFFFFFFull) return -1;
-        L.plan[s] = w8_plan(N[s], K[s], cu_count());
+        L.plan[s] = w8_plan(N[s], K[s], cu_count(), true);
         if (L.plan[s].max_slots > 8) return -1;
     }
     size_t off;
@@ -1576,13 +1587,14 @@ int chain_stages() {
 // layers (tokens x width x inner width, pairs of layers): 1 x 4096 x 11008, 8
 // 235 / 206; 16: 243 / 222; 24: 251 / 250; 32: 258 / 266; 1 x 3584 x 3200, 4 83 /
 // 37; 10 x 1536 x 4224, 8 140 / 100; 31 x 3328 x 4608, 5 113 / 100; 31 x 2560 x 8960,
-// 6 150 / 153. `form`: 0 = by estimate, 1 = one launch, 2 = layers.
+// 6 150 / 153. With operands off a 16-byte boundary only the token kernel can take
+// a layer. `form`: 0 = by estimate, 1 = one launch, 2 = layers.
 bool chain_by_layers(int form, const pyc::W8ChainArgs& a) {
     if (form != 0) return form == 2;
     double chain = 0.0, layers = 0.0;
     for (int s = 0; s < a.nsteps; ++s) {
         double c = 0.0;
-        if (w8_whole_form(a.M, a.st[s].N, a.st[s].K, &c) < 0) return false;
+        if (w8_whole_form(a.M, a.st[s].N, a.st[s].K, a.st[s].X, a.st[s].W, &c) < 0) return false;
         layers += c;
         chain += 8.5 + 0.036 * ((double)a.st[s].N * a.st[s].K / 256.0 / 1000.0) + 0.04 * a.M;
     }
@@ -1590,12 +1602,15 @@ bool chain_by_layers(int form, const pyc::W8ChainArgs& a) {
 }
 
 int chain_layers_launch(const pyc::W8ChainArgs& a, hipStream_t st) {
+    int form[pyc::kChainMaxSteps];
+    for (int s = 0; s < a.nsteps; ++s) {  // all of them before the first launch
+        double c = 0.0;
+        form[s] = w8_whole_form(a.M, a.st[s].N, a.st[s].K, a.st[s].X, a.st[s].W, &c);
+        if (form[s] < 0) return -1;
+    }
     for (int s = 0; s < a.nsteps; ++s) {
         const pyc::W8ChainStep& P = a.st[s];
-        double c = 0.0;
-        const int form = w8_whole_form(a.M, P.N, P.K, &c);
-        if (form < 0) return -1;
-        const int rc = w8_whole_launch(form, a.M, P.N, P.K, P.X, P.W, P.scale, P.relu, P.Y, st);
+        const int rc = w8_whole_launch(form[s], a.M, P.N, P.K, P.X, P.W, P.scale, P.relu, P.Y, st);
         if (rc != 0) return rc;
     }
     return 0;

@@ -144,3 +144,32 @@ def test_w8a16_forms(gpu, M, N, K):
         # two roundings to bf16 of nearby sums, plus fp32 summation order
         bound = 2.0 ** -7 * np.abs(ref) + 4e-6 * np.sqrt(K) * np.abs(ref).max()
         assert (np.abs(got - ref) <= bound).all(), form
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 200, 1040), (5, 1000, 1040), (17, 96, 2064), (32, 2048, 2048), (32, 130, 4096)])
+@pytest.mark.parametrize("x_off,w_off", [(1, 0), (2, 0), (0, 1), (0, 4), (3, 8)])
+def test_w8a16_unaligned_operands(gpu, M, N, K, x_off, w_off):
+    """X that starts x_off elements and weights that start w_off bytes past a 16-byte
+    boundary, among NaNs: through the public entry against the oracle, and the kernels
+    that load by LDS-DMA refuse them."""
+    torch = gpu
+    x, wq, scale = _layer(M, N, K, M + N + K)
+    Xb = torch.full((M * K + 32,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    Wb = torch.full((N * K + 64,), 0x7F, dtype=torch.uint8, device="cuda")
+    X = Xb[8 + x_off:8 + x_off + M * K].view(M, K)
+    Wq = Wb[16 + w_off:16 + w_off + N * K].view(N, K)
+    X.copy_(dev_bits16(torch, x))
+    Wq.copy_(dev_u8(torch, wq))
+    S = dev_f32(torch, scale)
+    Y = torch.full((M * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    pyc_amd.w8a16_gemm(X, Wq, S, Y[:M * N].view(M, N), True)
+    torch.cuda.synchronize()
+    assert bool((Y[M * N:] == 7.0).all())
+    got = Y[:M * N].float().cpu().numpy().reshape(M, N)
+    ref = oracle.bf16_to_f32(oracle.w8a16_layer(x, wq, scale, True))
+    # two roundings to bf16 of nearby sums, plus fp32 summation order
+    assert (np.abs(got - ref) <= 2.0 ** -7 * np.abs(ref) + 4e-6 * np.sqrt(K) * np.abs(ref).max()).all()
+    f = pyc_amd.lib().pyc_hip_w8a16_launch_form
+    f.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.c_int] + [C.c_void_p] * 2
+    for form in (1, 2, 3, 4):
+        assert f(form, M, N, K, X.data_ptr(), Wq.data_ptr(), S.data_ptr(), 0, Y.data_ptr(), None) == -1
