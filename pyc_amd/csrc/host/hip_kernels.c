@@ -292,10 +292,11 @@ static int pick_dma_tile(long M, long N, long K, int k_rows, int tail, int last,
 typedef struct {
     int t, rest; /* tiles; rest < 0: one launch */
     int m_end, n_end;
+    double cost; /* estimate for operands that LDS-DMA moves */
 } dma_plan;
 
 static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_only, int first_split, int last) {
-    dma_plan p = {0, -1, M, N};
+    dma_plan p = {0, -1, M, N, 0.0};
     double best;
     int t;
     p.t = pick_dma_tile(M, N, K, k_rows, tail, last, &best);
@@ -334,12 +335,44 @@ static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_on
             }
         }
     }
+    p.cost = best;
     return p;
+}
+
+/* What the general tiles cost (pick_half_tile), in microseconds: a launch, then for
+ * each K / 64 stage a time and, per 256 tiles, another, a time for every further
+ * round of 256 tiles, and what reading C for beta adds. By the rows of the
+ * operands: whole tiles, ragged in whole 16-byte chunks (at any base), by elements.
+ * Fitted to 4900 products of operands that LDS-DMA cannot move whole, M and N up to
+ * 9000, K 8 to 9000; mean error 12 %. 256 x 256 whole tiles: as ragged ones. */
+typedef struct {
+    double launch, stage, busy, round, beta;
+} half_cost;
+
+static double general_cost(int b_trans, int M, int N, int K, float beta) {
+    static const half_cost k_half[3][5] = {
+        /* 64 x 64 and 128 x 128, each with B [K,N] and [N,K]; 256 x 256 */
+        {{3.1, 0.49, 0.26, 0.1, 1.8}, {2.7, 0.39, 0.22, 0.4, 1.8}, {5.0, 0.79, 1.18, 2.4, 12.5},
+         {5.0, 0.48, 0.65, 1.8, 8.9}, {30.0, 5.1, 5.3, 44.0, 58.0}},
+        {{3.7, 1.40, 0.18, 1.2, 1.4}, {3.6, 1.13, 0.14, 1.8, 1.2}, {10.7, 2.04, 1.19, 4.3, 8.4},
+         {10.9, 1.33, 0.67, 4.2, 7.1}, {30.0, 5.1, 5.3, 44.0, 58.0}},
+        {{3.5, 1.72, 0.90, 0.5, 1.7}, {3.4, 1.63, 1.19, 0.6, 1.6}, {9.8, 3.10, 2.84, 4.3, 10.3},
+         {10.2, 2.45, 2.86, 4.4, 10.3}, {23.0, 13.0, 8.4, 42.0, 84.0}},
+    };
+    const int t = pick_half_tile(M, N);
+    const int chunks = K % 8 == 0 && (b_trans || N % 8 == 0);
+    const int rows = !chunks ? 2 : M % t == 0 && N % t == 0 && K % 64 == 0 ? 0 : 1;
+    const half_cost* h = &k_half[rows][t == 256 ? 4 : (t == 128 ? 2 : 0) + (b_trans ? 1 : 0)];
+    const double tiles = (double)((M + t - 1) / t) * (double)((N + t - 1) / t);
+    const double rounds = (double)(long)((tiles + 255.0) / 256.0), kt = (double)((K + 63) / 64);
+    const double c = h->launch + kt * (h->stage + h->busy * tiles / 256.0) + h->round * (rounds - 1.0) +
+                     (beta != 0.0f ? h->beta : 0.0);
+    return c < 3.4 ? 3.4 : c;
 }
 
 /* The plan of a half GEMM on LDS-DMA tiles, made before anything is launched
  * from what each kernel says it takes: both parts run once the first has. 0 when
- * none of them takes the product (the general register-staged tiles do).
+ * the general register-staged tiles do the product.
  *  - Operands that LDS-DMA can move in whole chunks: every tile, and 256 x 256
  *    where the table describes it: the persistent kernel, or the one-shot kernel
  *    ([N,K] only) with plain whole-chunk stores. With beta or a C that takes
@@ -347,7 +380,12 @@ static dma_plan plan_dma(int M, int N, long K, int k_rows, int tail, int rows_on
  *    every CU a tile (us, one-shot / the smaller tiles: 3072 x 4096 x 2048 with beta
  *    89 / 69, 3001 x 4096 x 1024 67 / 46, C off 16 bytes 56 / 35).
  *  - Others (bases off a 16-byte boundary, odd rows): the 256 x 256 kernels for
- *    all of C where they give every CU a tile, else tiles up to 128 x 128. */
+ *    all of C where they give every CU a tile, else tiles up to 128 x 128 staged
+ *    through registers (1.7 times what the table says), or the general tiles
+ *    where those take less by estimate: short K, above all in whole chunks, which
+ *    they load directly. us, general / register-staged: [K,N] 832 x 768 x 64 off 2
+ *    bytes 3.6 / 8.8, [N,K] 3840 x 3840 x 64 off 8 bytes 12.6 / 27.8, 1792 x 4096 x
+ *    832 22 / 30, 4050 x 359 x 31 7.8 / 11.5; 5888 x 1856 x 320 47 / 29. */
 static int plan_gemm(int b_trans, int M, int N, int K, const void* A, const void* B, const void* C, float beta,
                      const float* bias, int epi, dma_plan* p) {
     const int small = pyc_hip_gemm_small_takes(b_trans, M, N, K, A, B);
@@ -367,7 +405,7 @@ static int plan_gemm(int b_trans, int M, int N, int K, const void* A, const void
     const int plain = beta == 0.0f && ((uintptr_t)C & 15) == 0 && N % 8 == 0;
     const int last = small < 2 ? DT_128 : big == 2 || (big == 1 && (fills || plain)) ? DT_256 : DT_128X256;
     *p = plan_dma(M, N, K, !b_trans, 0, 0, last, last);
-    return 1;
+    return small == 2 || 0.3 + 1.7 * p->cost < 0.95 * general_cost(b_trans, M, N, K, beta);
 }
 
 /* plan_gemm for the shape-chosen symbols, as tile edges: out = {rows and columns of

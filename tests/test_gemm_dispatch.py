@@ -133,3 +133,18 @@ def test_one_shot_kernel_only_with_a_tile_per_cu(dispatch, m, n, k):
         assert rc == 0 and all(p[0] == 1 for p in parts), (kw, parts)
     rc, parts = _run(dispatch, True, 4096, 4096, k, beta=0.5)
     assert rc == 0 and parts[0][:2] == (2, 1)
+
+
+@pytest.mark.parametrize("bt,m,n,k,off,general", [
+    (False, 832, 768, 64, 2, True), (True, 3840, 3840, 64, 8, True), (True, 2048, 2048, 128, 8, True),
+    (False, 64, 64, 64, 2, True), (True, 1, 330, 17, 0, True),
+    (False, 5888, 1856, 320, 8, False), (False, 1280, 3072, 1600, 8, False), (True, 839, 7424, 2347, 0, False),
+    (False, 3218, 922, 7424, 0, False)])
+def test_short_k_off_16_bytes_takes_the_general_tiles(dispatch, bt, m, n, k, off, general):
+    """Operands that LDS-DMA cannot move in whole chunks: the general tiles, which load
+    them directly, are up to twice as fast as the register-staged ring at a short K,
+    and far slower at a long one."""
+    rc, parts = _run(dispatch, bt, m, n, k, off, off)
+    assert rc == 0 and (parts[0][0] == 4) == general, parts
+    rc, parts = _run(dispatch, bt, m, n, k)  # on 16-byte boundaries: as ever
+    assert rc == 0 and (k % 8 != 0 or parts[0][0] != 4)
