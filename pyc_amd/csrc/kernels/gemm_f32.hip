@@ -468,16 +468,12 @@ static int tile_f32(long M, long N, long K, bool whole) {
     return c32 < c64 ? 32 : 64;
 }
 
-extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A,
-                                       const void* B, void* C, float alpha, float beta,
-                                       const float* bias, int epi, void* stream) {
+// What runs an fp32 product (host only, no launch): 64 or 32 = the LDS-DMA kernel
+// with that tile, 0 = the register-staged kernel. The pointers are looked at for
+// their alignment.
+extern "C" int pyc_hip_gemm_f32_form(int b_trans, int M, int N, int K, const void* A, const void* B) {
     using namespace pyc;
-    dim3 grid((N + kF32BN - 1) / kF32BN, (M + kF32BM - 1) / kF32BM), block(512);
     const bool even = (M % kF32BM == 0) && (N % kF32BN == 0) && (K % kF32BK == 0);
-    hipStream_t s = (hipStream_t)stream;
-    const float* a = (const float*)A;
-    const float* b = (const float*)B;
-    float* c = (float*)C;
     // the LDS-DMA kernel addresses each operand through a buffer descriptor
     // (32-bit byte offsets, rows and k padded to whole tiles and ring stages)
     // and moves 16-byte chunks, of whole tiles on 16-byte boundaries
@@ -488,16 +484,41 @@ extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const v
                             : ((size_t)M + pad) * ((size_t)K + pad) * 4 < kF32PastEnd &&
                                   ((size_t)N + pad) * ((size_t)K + pad) * 4 < kF32PastEnd);
     const int tile = tile_f32(M, N, K, whole);
-    // More ragged 64 x 64 tiles than CUs and a short k: starts and ends count,
-    // and two register-staged workgroups share a CU where one ring takes it. us,
-    // ring / register-staged, [K,N] B: 1728 x 2568 x 64 26.8 / 20.3, 1015 x 2944 x 128
-    // 21.1 / 19.1, 2805 x 1600 x 140 38 / 36, 2676 x 560 x 448 25.7 / 27.6; rows off 16
-    // bytes 1472 x 1980 x 194 28.8 / 36; [N,K] B 2916 x 448 x 192 16.2 / 14.2, 512 x
-    // 2440 x 512 27.3 / 26.6.
-    const bool wide = K % 4 == 0 && (b_trans || N % 4 == 0);
-    const bool staged = !whole && tile == 64 && (long)((M + 63) / 64) * ((N + 63) / 64) > 256 &&
-                        K <= (!wide ? 128 : b_trans ? 512 : 256);
-    if (dma && !staged) {
+    if (!dma || whole) return dma ? tile : 0;
+    // A short k on the register-staged kernel: starts and ends count, and two of its
+    // workgroups share a CU where one ring takes it. More ragged 64 x 64 tiles than CUs,
+    // us, ring / register-staged, [K,N] B: 1728 x 2568 x 64 26.8 / 20.3, 1015 x 2944 x 128
+    // 21.1 / 19.1, 2805 x 1600 x 140 38 / 36, 1465 x 3792 x 404 91 / 82, 2676 x 560 x 448
+    // 25.7 / 27.6; odd rows 910 x 1651 x 144 23 / 20, 1472 x 1980 x 194 28.8 / 36; [N,K] B
+    // 2916 x 448 x 192 16.2 / 14.2, 512 x 2440 x 512 27.3 / 26.6, 3435 x 2968 x 664 195 /
+    // 173. Whole tiles whose operands start off a 16-byte boundary, which that kernel
+    // takes without guards: 3520 x 7424 x 320 346 / 224, 1664 x 7936 x 576 220 / 178, 1280 x
+    // 1088 x 320 20.3 / 16.8; [N,K] 8320 x 2176 x 832 363 / 300, 5504 x 2112 x 1664 432 /
+    // 386, 384 x 1536 x 192 8.3 / 6.9; from k = 2000 on the ring is level or ahead.
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+    int k_staged = 0;
+    if (even)
+        k_staged = t64 > 1024 ? 1792 : t64 > 512 ? 1280 : t64 > 256 ? 1024 : b_trans ? 448 : 320;
+    else if (tile == 64 && t64 > 256) {
+        const bool wide = K % 4 == 0 && (b_trans || N % 4 == 0);
+        k_staged = !wide ? (b_trans ? 128 : 160) : !b_trans ? 416 : t64 > 1024 ? 768 : 512;
+    }
+    return K <= k_staged ? 0 : tile;
+}
+
+extern "C" int pyc_hip_gemm_f32_launch(int b_trans, int M, int N, int K, const void* A,
+                                       const void* B, void* C, float alpha, float beta,
+                                       const float* bias, int epi, void* stream) {
+    using namespace pyc;
+    dim3 grid((N + kF32BN - 1) / kF32BN, (M + kF32BM - 1) / kF32BM), block(512);
+    const bool even = (M % kF32BM == 0) && (N % kF32BN == 0) && (K % kF32BK == 0);
+    hipStream_t s = (hipStream_t)stream;
+    const float* a = (const float*)A;
+    const float* b = (const float*)B;
+    float* c = (float*)C;
+    const bool whole = even && ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0);
+    const int tile = pyc_hip_gemm_f32_form(b_trans, M, N, K, A, B);
+    if (tile) {
         const int tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
         const dim3 tiles((unsigned)(tiles_m * tiles_n));
         const int gm = tiles_m < 4 ? tiles_m : 4;

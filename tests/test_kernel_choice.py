@@ -1,0 +1,39 @@
+"""Which kernel fp32 GEMM calls take, on the CPU (the choice looks at
+sizes and at the operands' alignment only)."""
+import ctypes as C
+
+import pytest
+
+import pyc_amd
+
+BASE = 1 << 40
+
+
+def _f32(bt, m, n, k, a_off=0, b_off=0):
+    f = pyc_amd.lib().pyc_hip_gemm_f32_form
+    f.argtypes = [C.c_int] * 4 + [C.c_void_p] * 2
+    return f(int(bt), m, n, k, BASE + a_off, BASE + b_off)
+
+
+@pytest.mark.parametrize("bt,m,n,k,staged", [
+    (False, 3520, 7424, 320, True), (False, 1280, 1088, 320, True), (True, 384, 1536, 192, True),
+    (True, 8320, 2176, 832, True), (True, 5504, 2112, 1664, True),
+    (True, 1024, 1024, 2048, False), (False, 1024, 1024, 1024, False), (False, 4096, 4096, 4096, False)])
+def test_f32_whole_tiles_off_16_bytes(bt, m, n, k, staged):
+    """Whole tiles off a 16-byte boundary: the register-staged kernel where k is short,
+    which takes them without guards; on 16-byte boundaries always the ring."""
+    assert (_f32(bt, m, n, k, 4) == 0) == (_f32(bt, m, n, k, 0, 8) == 0) == staged
+    assert _f32(bt, m, n, k) in (32, 64)
+
+
+@pytest.mark.parametrize("bt,m,n,k,form", [
+    (False, 1728, 2568, 64, 0), (False, 1465, 3792, 404, 0), (False, 2676, 560, 448, 64),
+    (True, 3435, 2968, 664, 0), (True, 2805, 1600, 1400, 64), (False, 910, 1651, 144, 0),
+    (False, 1472, 1980, 194, 64), (False, 700, 701, 702, 32), (True, 440, 440, 440, 32)])
+def test_f32_ragged(bt, m, n, k, form):
+    assert _f32(bt, m, n, k) == form
+
+
+def test_f32_unusual_operands():
+    assert _f32(True, 512, 512, 512, 1) == 0 and _f32(False, 512, 512, 512, 0, 2) == 0  # off 4 bytes
+    assert _f32(True, 1 << 16, 64, 1 << 15) == 0                                        # 8 GiB of A
