@@ -404,6 +404,25 @@ static int launch_gelu(const void* x, void* y, size_t n, hipStream_t s) {
 
 constexpr int kLnFewRows = 2048;  // fewer rows than this leave SIMDs idle at one wave each
 
+// Whether layernorm_row_kernel takes rows of D elements of 16 / V bytes; `vec`: whole
+// 16-byte chunks on 16-byte boundaries, nc: chunks per lane where those are even.
+// Few rows, or rows that are no whole chunks per lane. In us, one of the other kernels /
+// the row kernel: 1 x 3392 bf16 6.3 / 3.5, 64 x 4096 4.9 / 3.8, 8000 x 5003 127 / 50, 6000 x
+// 8190 187 / 46, 4000 x 6145 fp32 130 / 45, 5000 x 8192 fp16 59 / 39; 2000 x 4096 bf16 9.9
+// / 10.0 (so whole rows of that many stay with one wave each). Not rows that
+// layernorm_kernel reads with one load per lane (a chunk, or up to three elements): it
+// has less to do per row there. Graph replays: fp16 14495 x 61 5.8 / 9.5, bf16 27475 x 91
+// 11.0 / 14.1. The row kernel's time over the other's: by elements 1.2 to 1.8 up to D =
+// 64 (fp32 1.0 to 1.2), in 16 bits with 2048 rows or more 1.1 to 1.4 up to 128 and 1.0 to
+// 1.15 up to 192, below 1 past that; in chunks with 1024 rows or more 1.0 to 1.13 in 16
+// bits, fp32 1.0 to 1.05 up to D = 64 and 0.8 to 1.0 past it.
+static bool ln_row_form(int rows, int D, int V, bool vec, int nc, bool cap16) {
+    const bool whole = (nc >= 1 && nc <= 8) || (cap16 && nc > 8 && nc <= 16);
+    if (D < V || (D + V - 1) / V > 4 * kWave * 8 || (whole && rows >= kLnFewRows / 2)) return false;
+    if (vec) return rows < kLnFewRows / 2 || D > (V == 8 ? kWave * V : kWave);
+    return D > (V == 8 && rows >= kLnFewRows ? 3 * kWave : kWave);
+}
+
 template <typename T>
 static int launch_layernorm(const void* x, const void* g, const void* b, void* y, int rows, int D, float eps,
                             hipStream_t s) {
@@ -412,15 +431,9 @@ static int launch_layernorm(const void* x, const void* g, const void* b, void* y
     const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
     const int nc = (vec && D % (V * kWave) == 0) ? D / (V * kWave) : 0;  // chunks per lane
     constexpr bool kCap16 = !std::is_same<T, f16_t>::value;  // fp16 rows past 8 chunks: three passes
-    // Few rows, or rows that are no whole chunks per lane: W waves per row. In
-    // us, one of the other two kernels / this one: 1 x 3392 bf16 6.3 / 3.5, 64 x 4096
-    // 4.9 / 3.8, 8000 x 5003 127 / 50, 6000 x 8190 187 / 46, 4000 x 6145 fp32 130 /
-    // 45, 5000 x 8192 fp16 59 / 39; 2000 x 4096 bf16 9.9 / 10.0 (so whole rows of
-    // that many stay with one wave each).
     const int n = (D + V - 1) / V;
-    const bool whole = (nc >= 1 && nc <= 8) || (kCap16 && nc > 8 && nc <= 16);
-    if (D >= V && n <= 4 * kWave * 8 && (!whole || rows < kLnFewRows / 2)) {
-        int W = 1;
+    if (ln_row_form(rows, D, V, vec, nc, kCap16)) {
+        int W = 1;  // waves per row
         while (W < 4 && (n > W * kWave * 8 || ((long)rows * W < kLnFewRows && n > W * kWave))) W *= 2;
         const int cap = (n + W * kWave - 1) / (W * kWave);
         const dim3 g2((unsigned)(((long)rows * W + 3) / 4));
@@ -463,6 +476,17 @@ extern "C" int pyc_hip_gelu_launch(int dtype, size_t n, const void* x, void* y, 
         case 2: return launch_gelu<f16_t>(x, y, n, s);
         default: return -1;
     }
+}
+
+// 1 where layernorm_row_kernel takes the call, else 0 (host only; the pointers are
+// looked at for their alignment).
+extern "C" int pyc_hip_layernorm_row_form(int dtype, int rows, int D, const void* x, const void* gamma,
+                                          const void* beta, const void* y) {
+    using namespace pyc;
+    const int V = dtype == 0 ? 4 : 8;
+    const bool vec = D % V == 0 && ((((uintptr_t)x | (uintptr_t)y | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0);
+    const int nc = (vec && D % (V * kWave) == 0) ? D / (V * kWave) : 0;
+    return ln_row_form(rows, D, V, vec, nc, dtype != 2);
 }
 
 extern "C" int pyc_hip_layernorm_launch(int dtype, int rows, int D, float eps, const void* x, const void* gamma,

@@ -238,3 +238,30 @@ def test_layernorm_rows(gpu, name, rows, D, off):
     torch.cuda.synchronize()
     assert torch.equal(x, yv)
     assert bool((buf[:8 + off] == 5.0).all()) and bool((buf[8 + off + rows * D:] == 5.0).all())
+
+
+@pytest.mark.parametrize("name", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,D,off", [(1024, 4096, 0), (1025, 8192, 0), (1024, 512, 0),  # 8 and 16 chunks a lane, 1
+                                        (1025, 504, 0), (2050, 192, 1), (2048, 193, 1),    # one pass and past it
+                                        (2047, 130, 1), (70, 64, 1), (70, 65, 1)])
+def test_layernorm_choice_edges(gpu, name, rows, D, off):
+    """Both sides of the rules that choose between the kernels, with enough rows that
+    whole rows stay with one wave each; against float64, nothing outside y."""
+    torch = gpu
+    t = _tdtype(torch, name)
+    g = torch.Generator(device="cuda").manual_seed(rows + D)
+    x = torch.empty(rows * D + 8, dtype=t, device="cuda")[off:off + rows * D].view(rows, D)
+    x.copy_(torch.randn((rows, D), generator=g, device="cuda") * 3.0 + 5.0)
+    gamma, beta = (torch.randn(D, generator=g, device="cuda").to(t) for _ in range(2))
+    y = torch.full((rows * D + 16,), 3.0, dtype=t, device="cuda")
+    yv = y[off:off + rows * D].view(rows, D)
+    pyc_amd.layernorm(x, yv, gamma, beta)
+    torch.cuda.synchronize()
+    assert bool((y[:off] == 3.0).all()) and bool((y[off + rows * D:] == 3.0).all())
+    pick = torch.unique(torch.cat([torch.arange(40), torch.arange(rows - 40, rows)])).tolist()
+    ref = oracle.layernorm_f64(x[pick].float().cpu().numpy(), gamma.float().cpu().numpy(),
+                               beta.float().cpu().numpy(), 1e-5)
+    _check(yv[pick].float().cpu().numpy(), ref, name)
+    pyc_amd.layernorm(x, x, gamma, beta)
+    torch.cuda.synchronize()
+    assert torch.equal(x, yv)

@@ -1,4 +1,4 @@
-"""Which kernel fp32 GEMM calls take, on the CPU (the choice looks at
+"""Which kernel fp32 GEMM and LayerNorm calls take, on the CPU (the choice looks at
 sizes and at the operands' alignment only)."""
 import ctypes as C
 
@@ -37,3 +37,17 @@ def test_f32_ragged(bt, m, n, k, form):
 def test_f32_unusual_operands():
     assert _f32(True, 512, 512, 512, 1) == 0 and _f32(False, 512, 512, 512, 0, 2) == 0  # off 4 bytes
     assert _f32(True, 1 << 16, 64, 1 << 15) == 0                                        # 8 GiB of A
+
+
+@pytest.mark.parametrize("dtype,rows,d,off,row", [
+    (2, 14495, 61, 0, 0), (1, 27475, 91, 0, 0), (1, 100, 64, 2, 0), (1, 100, 65, 2, 1), (2, 2047, 192, 2, 1),
+    (2, 2048, 192, 2, 0), (2, 2048, 193, 2, 1), (1, 1024, 504, 0, 0), (1, 1023, 504, 0, 1), (1, 5000, 520, 0, 1),
+    (0, 5000, 64, 0, 0), (0, 5000, 68, 0, 1), (0, 5000, 63, 0, 0), (0, 50, 64, 0, 1),
+    (1, 1, 3392, 0, 1), (1, 8000, 5003, 0, 1), (1, 1023, 4096, 0, 1), (1, 1024, 4096, 0, 0), (0, 3, 2, 0, 0),
+    (1, 5, 7, 0, 0), (2, 3, 16400, 0, 0)])
+def test_layernorm_row_kernel(dtype, rows, d, off, row):
+    """Short rows, which the plain kernel reads with one to three loads per lane, stay
+    with it (the row kernel took 1.1 to 1.8 times as long); long and few ones do not."""
+    f = pyc_amd.lib().pyc_hip_layernorm_row_form
+    f.argtypes = [C.c_int] * 3 + [C.c_void_p] * 4
+    assert f(dtype, rows, d, BASE + off, BASE, BASE, BASE) == row
