@@ -133,6 +133,15 @@ def _ptr(t) -> int:
 _current_raw_stream = None  # resolved at the first call
 
 
+def _forget_raw_stream() -> None:
+    global _current_raw_stream
+    _current_raw_stream = None
+
+
+# A forked child asks torch again, which refuses a device that its parent has initialised.
+os.register_at_fork(after_in_child=_forget_raw_stream)
+
+
 def _find_current_raw_stream():
     """A function that returns torch's current stream of the current device as
     an integer. torch.cuda.current_stream() builds a Stream object, 2.8 us a
