@@ -143,8 +143,11 @@ static const hip_variant k_variants[] = {
 /* The kernel an entry launches at the large shapes its descriptor is for:
  * the persistent LDS-DMA kernel for the shape-chosen and _lds half GEMMs,
  * the named tile otherwise; the persistent conv for the automatic and
- * persistent conv paths; the head-dim-128 attention; the K % 128 fp8 kernel;
- * the chain kernel; the register-resident LayerNorm. */
+ * persistent conv paths; the persistent head-dim-128 attention; the K % 128
+ * split-K fp8 kernel; the chain kernel; the register-resident LayerNorm. An entry
+ * that chooses by shape launches other kernels at other shapes (ring tiles, the
+ * attention's small forms, the fp8 token and whole-K kernels, the LayerNorm row
+ * kernel), whose LDS and occupancy these figures do not describe. */
 static int variant_kinfo(const hip_variant* v, pyc_hip_kinfo* ki) {
     const int bf = v->dtype == VT_BF16;
     memset(ki, 0, sizeof(*ki));
@@ -227,8 +230,8 @@ static int pick_half_tile(int M, int N) {
 }
 
 /* The LDS-DMA tiles and what a product costs on each, in microseconds: a
- * launch, then for every round of one tile per CU a start and end and K / 64
- * stages. A stage takes longer the more CUs fetch at once (stage[0] with few of
+ * launch, then for every round of one tile per CU (256 of them; with another count
+ * the choice is only less good) a start and end and K / 64 stages. A stage takes longer the more CUs fetch at once (stage[0] with few of
  * them busy, stage[1] with all 256), and `many` times as long when there is more
  * than one round (the operands of the small tiles then come from beyond L2 more
  * often; the persistent 256 x 256 tile hides its next tile's start). Measured on
@@ -529,6 +532,29 @@ int pyc_cutlass_attention_dispatch(const char* symbol, int seq_len, int d_head, 
 
 /* ---------------------------------------------------------------- conv2d */
 
+/* The implicit GEMM [N*P*Q, R*S*C] x [K, R*S*C] of a convolution: the persistent
+ * 256 x 256 tiles (and their tail kernel) where they are the cheapest and `big`, else the
+ * best of the smaller tiles, in one part or two by output pixels. */
+static dma_plan plan_conv(long Mg, int K, long Kg, int big) {
+    return plan_dma((int)Mg, K, Kg, 0, big, 1, DT_128X256, big ? DT_256 : DT_128X256);
+}
+
+/* plan_conv as tile edges: out = {rows and columns of the first part's tile, of the
+ * second's (0, 0: one launch), output pixels of the first part}. Host only. */
+int pyc_hip_conv2d_plan(int Mg, int K, int Kg, int big, int* out) {
+    dma_plan p;
+    if (Mg <= 0 || K <= 0 || Kg <= 0 || !out) {
+        return 0;
+    }
+    p = plan_conv(Mg, K, Kg, big);
+    out[0] = k_dma_tiles[p.t].bm;
+    out[1] = k_dma_tiles[p.t].bn;
+    out[2] = p.rest < 0 ? 0 : k_dma_tiles[p.rest].bm;
+    out[3] = p.rest < 0 ? 0 : k_dma_tiles[p.rest].bn;
+    out[4] = p.m_end;
+    return 1;
+}
+
 int pyc_hip_conv2d_dispatch(const char* symbol, int N, int H, int W, int C_in, int K, int R, int S,
                             int pad_h, int pad_w, int stride_h, int stride_w, const void* x,
                             const void* w, const float* bias, int relu, void* y, void* stream) {
@@ -543,20 +569,17 @@ int pyc_hip_conv2d_dispatch(const char* symbol, int N, int H, int W, int C_in, i
         return -1;
     }
     if (v->tile == CONV_AUTO) {
-        /* The implicit GEMM [N*P*Q, R*S*C] x [K, R*S*C]: the persistent 256 x 256
-         * tiles (and their tail kernel) for shapes inside their preconditions
-         * where they are the cheapest, else the best of the smaller tiles. */
         const int bf = v->dtype == VT_BF16;
         const long P = (H + 2L * pad_h - R) / stride_h + 1, Q = (W + 2L * pad_w - S) / stride_w + 1;
         const long Mg = (long)N * P * Q, Kg = (long)R * S * C_in;
         if (Mg <= 0x7FFFFF00L && Kg <= 0x7FFFFF00L) {
-            dma_plan p = plan_dma((int)Mg, K, Kg, 0, 1, 1, DT_128X256, DT_256);
+            dma_plan p = plan_conv(Mg, K, Kg, 1);
             int rc = 1;
             if (p.t == DT_256) {
                 rc = pyc_hip_conv2d_persist_launch(bf, 1, N, H, W, C_in, K, R, S, pad_h, pad_w, stride_h, stride_w, x,
                                                    w, bias, relu ? 1 : 0, y, stream);
                 if (rc == 1) {
-                    p = plan_dma((int)Mg, K, Kg, 0, 0, 1, DT_128X256, DT_128X256);
+                    p = plan_conv(Mg, K, Kg, 0);
                 }
             }
             if (rc == 1) {

@@ -1280,7 +1280,7 @@ extern "C" int pyc_hip_w8a16_reserve(int N, int K) {
 
 namespace {
 
-// Estimated microseconds of one layer on the MI355X, fitted to back-to-back runs.
+// Estimated microseconds of one layer on the MI355X's 256 CUs, fitted to back-to-back runs.
 // Token kernel [N,K]: 4096 x 11008 11.1 (1 token), 12.7 (2); 4096 x 8192 10.5 (3),
 // 11.8 (4; whole-K 10.5); 11008 x 4096 9.7 (1; whole-K 10.7), 16.5 (4; whole-K
 // 11.2). Whole-K kernel with UB 1 / 2 / 3 / 4 (split-K kernel), 32 tokens:
@@ -1601,6 +1601,29 @@ bool chain_by_layers(int form, const pyc::W8ChainArgs& a) {
     return layers < 0.9 * chain;
 }
 
+}  // namespace
+
+// 1 = the chain runs in one launch, 2 = layer by layer (chain_by_layers' estimate); -1
+// for a chain outside the preconditions. Host only; X and Wq are looked at for their
+// alignment.
+extern "C" int pyc_hip_w8a16_chain_form(int M, int nsteps, const int* N, const int* K, const void* X,
+                                        const void* const* Wq) {
+    ChainLayout L;
+    if (!N || !K || !Wq || chain_layout(M, nsteps, N, K, L) != 0) return -1;
+    pyc::W8ChainArgs a{};
+    a.M = M;
+    a.nsteps = nsteps;
+    for (int s = 0; s < nsteps; ++s) {
+        a.st[s].N = N[s];
+        a.st[s].K = K[s];
+        a.st[s].X = s == 0 ? (decltype(a.st[s].X))X : nullptr;  // the workspace's activations are aligned
+        a.st[s].W = (decltype(a.st[s].W))Wq[s];
+    }
+    return chain_by_layers(0, a) ? 2 : 1;
+}
+
+namespace {
+
 int chain_layers_launch(const pyc::W8ChainArgs& a, hipStream_t st) {
     int form[pyc::kChainMaxSteps];
     for (int s = 0; s < a.nsteps; ++s) {  // all of them before the first launch
@@ -1669,10 +1692,10 @@ extern "C" int pyc_hip_w8a16_chain_launch(int M, int nsteps, const void* X, cons
 // device array of kNoAllocScratchBytes that every GPU the library runs on
 // holds until the process ends. Its device address is looked up once per
 // device (hipGetSymbolAddress, with that device current) and kept per device:
-// on the host the array's name stands for no device address. Each launch
-// first clears the step, exit and arrival counters of its layout with a fill
-// kernel (no memset node, so it can be captured), then runs the same chain
-// kernel as pyc_hip_w8a16_chain_launch. The timeout word sits outside the
+// on the host the array's name stands for no device address. A launch runs what
+// pyc_hip_w8a16_chain_launch does: layer by layer, or the chain kernel, whose step,
+// exit and arrival counters are then cleared first by a fill kernel (no memset
+// node, so it can be captured). The timeout word sits outside the
 // cleared range and is read by pyc_hip_w8a16_chain_error. Calls that overlap
 // on one GPU share the array and race.
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;

@@ -114,8 +114,11 @@ TILE_CASES = [
 ]
 
 
-@pytest.mark.parametrize("N,H,W,C,K,dt", TILE_CASES)
-def test_conv_persistent_tile_rounds(gpu, N, H, W, C, K, dt):
+# below one round the automatic symbol takes smaller tiles (its results are checked all
+# the same), so those cases also name the persistent kernel
+@pytest.mark.parametrize("N,H,W,C,K,dt,symbol", [c + ("",) for c in TILE_CASES] +
+                         [c + ("_persist",) for c in (TILE_CASES[0], TILE_CASES[2])])
+def test_conv_persistent_tile_rounds(gpu, N, H, W, C, K, dt, symbol):
     """The persistent implicit-GEMM conv across tile counts below, at and above
     one round of the grid (so workgroups move on to a second tile, through the
     next-tile prologue, or the remainder goes to the tail kernel). Every output
@@ -132,8 +135,8 @@ def test_conv_persistent_tile_rounds(gpu, N, H, W, C, K, dt):
     Bv = 0.01 * torch.randn(K, generator=gb, device="cuda")
     Y = torch.empty((N, H, W, K), dtype=tdt, device="cuda")
     Y2 = torch.empty_like(Y)
-    pyc_amd.conv2d(f"hip_conv2d_{dt}", X, Wd, Y, pad=(1, 1), stride=(1, 1), bias=Bv, relu=True)
-    pyc_amd.conv2d(f"hip_conv2d_{dt}", X, Wd, Y2, pad=(1, 1), stride=(1, 1), bias=Bv, relu=True)
+    for y in (Y, Y2):
+        pyc_amd.conv2d(f"hip_conv2d_{dt}{symbol}", X, Wd, y, pad=(1, 1), stride=(1, 1), bias=Bv, relu=True)
     torch.cuda.synchronize()
     assert torch.equal(Y.view(torch.int16), Y2.view(torch.int16))
     kred = 9 * C
@@ -220,3 +223,64 @@ def test_conv_lds_tiles(gpu, bm, bn, dt, N, H, W, C, K, R, S, pad, stride):
     eps = 2.0 ** (-8 if dt == "bf16" else -11)
     bad = ~(np.abs(got - ref) <= eps * np.abs(ref) + 4e-6 * np.sqrt(R * S * C) * np.abs(ref).max())
     assert not bad.any(), f"{bad.sum()} off, first at {np.argwhere(bad)[0]}"
+
+
+def _check_parts(torch, X, Wd, bias, Y, end, pad, stride):
+    """Y (flat, 7.0 past `end`) against the oracle."""
+    assert bool((Y[end:] == 7.0).all())
+    ref = oracle.conv2d_nhwc_f32(X.float().cpu().numpy(), Wd.float().cpu().numpy(), bias, pad, stride, relu=True)
+    got = Y[:end].float().cpu().numpy().reshape(ref.shape)
+    kred = int(np.prod(Wd.shape[1:]))
+    # one rounding of the result (2^-8 or 2^-11 relative) plus fp32 summation order
+    eps = 2.0 ** (-8 if Y.dtype == torch.bfloat16 else -11)
+    bad = ~(np.abs(got - ref) <= eps * np.abs(ref) + 4e-6 * np.sqrt(kred) * np.abs(ref).max())
+    assert not bad.any(), f"{bad.sum()} off, first at {np.argwhere(bad)[0]}"
+
+
+@pytest.mark.parametrize("first,rest", [((128, 256), (32, 32)), ((128, 128), (64, 64)), ((64, 64), (128, 64)),
+                                        ((32, 32), (128, 128))])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("N,H,W,C,K,R,S,pad,stride", [(3, 9, 11, 24, 70, 3, 3, (1, 1), (1, 1)),
+                                                      (2, 13, 14, 8, 33, 3, 2, (1, 0), (2, 1))])
+def test_conv_lds_tiles_in_two_parts(gpu, first, rest, dt, N, H, W, C, K, R, S, pad, stride):
+    """Two launches on different tiles that meet inside an image and a row of pixels."""
+    import ctypes
+    torch = gpu
+    r = np.random.default_rng(N + H + C + K)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float16
+    X = torch.from_numpy(r.uniform(0, 1, (N, H, W, C)).astype(np.float32)).cuda().to(tdt)
+    Wd = torch.from_numpy(r.normal(0, np.sqrt(2.0 / (R * S * C)), (K, R, S, C)).astype(np.float32)).cuda().to(tdt)
+    bias = r.normal(0, 0.1, K).astype(np.float32)
+    Bd = dev_f32(torch, bias)
+    m = N * ((H + 2 * pad[0] - R) // stride[0] + 1) * ((W + 2 * pad[1] - S) // stride[1] + 1)
+    launch = pyc_amd.lib().pyc_hip_conv2d_small_launch
+    launch.argtypes = ([ctypes.c_int] * 14 + [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_void_p] +
+                       [ctypes.c_int] * 2 + [ctypes.c_void_p])
+    for cut in (m // 2 + 3, 1, m - 1):
+        Y = torch.full((m * K + 512,), 7.0, dtype=tdt, device="cuda")
+        for (bm, bn), m0, m1 in ((first, 0, cut), (rest, cut, m)):
+            assert launch(int(dt == "bf16"), bm, bn, N, H, W, C, K, R, S, pad[0], pad[1], stride[0], stride[1],
+                          X.data_ptr(), Wd.data_ptr(), Bd.data_ptr(), 1, Y.data_ptr(), m0, m1, None) == 0
+        torch.cuda.synchronize()
+        _check_parts(torch, X, Wd, bias, Y, m * K, pad, stride)
+
+
+def test_conv_planned_in_two_parts(gpu):
+    """An automatic call whose plan has two parts (asserted)."""
+    import ctypes
+    torch = gpu
+    N, H, W, C, K = 19, 44, 41, 16, 80
+    plan = (ctypes.c_int * 5)()
+    f = pyc_amd.lib().pyc_hip_conv2d_plan
+    f.argtypes = [ctypes.c_int] * 4 + [ctypes.c_void_p]
+    assert f(N * H * W, K, 9 * C, 1, plan) == 1 and plan[2] > 0 and 0 < plan[4] < N * H * W and plan[0] < 256
+    r = np.random.default_rng(4)
+    X = torch.from_numpy(r.uniform(0, 1, (N, H, W, C)).astype(np.float32)).cuda().bfloat16()
+    Wd = torch.from_numpy(r.normal(0, np.sqrt(2.0 / (9 * C)), (K, 3, 3, C)).astype(np.float32)).cuda().bfloat16()
+    bias = r.normal(0, 0.1, K).astype(np.float32)
+    Bd = dev_f32(torch, bias)
+    m = N * H * W
+    Y = torch.full((m * K + 512,), 7.0, dtype=torch.bfloat16, device="cuda")
+    pyc_amd.conv2d("hip_conv2d_bf16", X, Wd, Y[:m * K].view(N, H, W, K), pad=(1, 1), stride=(1, 1), bias=Bd, relu=True)
+    torch.cuda.synchronize()
+    _check_parts(torch, X, Wd, bias, Y, m * K, (1, 1), (1, 1))

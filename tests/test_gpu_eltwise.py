@@ -91,9 +91,9 @@ def test_gelu_unaligned(gpu):
                                                (33, 8192, True, 1e-5), (20, 6144, False, 1e-5)])
 def test_layernorm(gpu, name, rows, D, affine, eps):
     """Rows of mean far from 0 (two-pass variance), D not a multiple of the
-    16-byte chunk (element path), with and without gamma/beta, several eps;
-    D = 4096, 6144 and 8192 reach the register-resident kernel's 8- and
-    16-chunk forms (bf16: 8, 12 and 16 chunks per lane)."""
+    16-byte chunk (element path), with and without gamma/beta, several eps.
+    So few rows of D = 4096 and more share waves; the register-resident kernel's
+    8- and 16-chunk forms are in test_layernorm_choice_edges."""
     torch = gpu
     t = _tdtype(torch, name)
     g = torch.Generator(device="cuda").manual_seed(rows * D)

@@ -582,12 +582,13 @@ def test_f32_ragged_tiles(gpu, m, n, k, off, layout):
 
 
 @pytest.mark.parametrize("layout", ["nt", "nn"])
-@pytest.mark.parametrize("m,n,k", [(1999, 11008, 64),    # a round of 256 x 256 tiles by columns, the rest smaller
-                                   (8200, 2056, 128),    # more tile rows than columns
+@pytest.mark.parametrize("m,n,k", [(1999, 11008, 64),    # one launch of ragged 256 x 256 tiles, a short K
+                                   (8200, 2056, 128),    # the same, more tile rows than columns
                                    (3000, 3000, 72),     # rounds of 128-row tiles (K no multiple of 64), the rest
                                    (3001, 3002, 71)])    # the same on the register-staged tiles
 def test_gemm_in_two_parts(gpu, m, n, k, layout):
-    """Products that take whole rounds of one tile and the rest of C on another:
+    """Products of more tiles than CUs, in one launch or as whole rounds of one tile
+    and the rest of C on another (plans are asserted in test_gemm_parts_as_planned):
     every element against fp32, and nothing past C."""
     torch = gpu
     bt = layout == "nt"

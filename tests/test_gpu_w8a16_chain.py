@@ -225,3 +225,49 @@ def test_chain_forms(gpu, form, M, dims):
         torch.cuda.synchronize()
         assert pyc_amd.w8a16_chain_error() == 0
         assert rel_max_err(oracle.bf16_to_f32(host_bits16(Y)), oracle.bf16_to_f32(cur)) <= 2e-2
+
+
+@pytest.mark.parametrize("M,dims", [(32, [2048, 3072, 2048, 3072, 2048]), (5, [256, 512, 384, 128]), (1, [128, 64])])
+def test_chain_kernel_graph_replay(gpu, M, dims):
+    """The one-launch chain kernel (these shapes would go layer by layer otherwise),
+    captured and replayed with new inputs, with eager launches of this and of another
+    chain in between: its counters re-arm, so every replay equals the eager launch bit
+    for bit, and both the layers one by one within the chain's tolerance."""
+    torch = gpu
+    relus = [i % 2 == 0 for i in range(len(dims) - 1)]
+    layers = _dev_layers(torch, _weights(dims, 7), relus)
+    other = _dev_layers(torch, _weights([512, 1024, 256], 8), [True, False])
+    f = pyc_amd.lib().pyc_hip_w8a16_chain_launch_form
+    f.argtypes = [C.c_int] * 3 + [C.c_void_p] * 8
+    v = lambda a: C.cast(a, C.c_void_p)
+
+    def run(x, ls, y, stream):
+        n, wq, sc, N, K, relu = pyc_amd._chain_arrays(ls)
+        assert f(1, int(x.shape[0]), n, x.data_ptr(), v(wq), v(sc), v(N), v(K), v(relu), y.data_ptr(), stream) == 0
+
+    X = torch.empty((M, dims[0]), dtype=torch.bfloat16, device="cuda")
+    Yg = torch.empty((M, dims[-1]), dtype=torch.bfloat16, device="cuda")
+    Ye, Xo = torch.empty_like(Yg), torch.randn((M, 512), device="cuda").to(torch.bfloat16)
+    Yo = torch.empty((M, 256), dtype=torch.bfloat16, device="cuda")
+    pyc_amd.w8a16_chain_reserve(M, layers)
+    pyc_amd.w8a16_chain_reserve(M, other)
+    torch.cuda.synchronize()
+    graph, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        graph.capture_begin()
+        run(X, layers, Yg, s.cuda_stream)
+        graph.capture_end()
+    torch.cuda.synchronize()
+    st = torch.cuda.current_stream().cuda_stream
+    for rep in range(4):
+        X.copy_(torch.randn((M, dims[0]), device="cuda").to(torch.bfloat16))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        run(X, layers, Ye, st)
+        run(Xo, other, Yo, st)
+        torch.cuda.synchronize()
+        assert torch.equal(Yg, Ye), f"replay {rep} differs from the eager chain"
+        assert rel_max_err(Ye.float().cpu().numpy(), _sequential(torch, X, layers).float().cpu().numpy()) <= 2e-2
+        assert rel_max_err(Yo.float().cpu().numpy(), _sequential(torch, Xo, other).float().cpu().numpy()) <= 2e-2
+    assert pyc_amd.w8a16_chain_error() == 0

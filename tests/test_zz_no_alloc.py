@@ -120,3 +120,51 @@ def test_noalloc_graph_capture_without_reserve(gpu):
     torch.cuda.synchronize()
     assert torch.equal(Yo, Yo_ref)
     assert pyc_amd.w8a16_chain_error() == 0
+
+
+def test_noalloc_chain_kernel_capture_without_reserve(gpu):
+    """The same with a chain that the estimate leaves with the one-launch chain kernel
+    (asserted), whose counters the captured launch clears itself: replays with new inputs
+    between eager launches of this and of a shorter chain."""
+    torch = gpu
+    M, dims = 32, [2560, 8960, 2560, 8960, 2560]
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def dev_layers(d):
+        out = []
+        for i, (K, N) in enumerate(zip(d[:-1], d[1:])):
+            w = torch.randn((N, K), generator=g, device="cuda") * np.sqrt(2.0 / K)
+            s = (w.abs().amax(1) / 448.0).float().contiguous()
+            out.append(((w / s[:, None]).to(torch.float8_e4m3fn).view(torch.uint8), s, i % 2 == 0))
+        return out
+
+    layers = dev_layers(dims)
+    X = torch.empty((M, dims[0]), dtype=torch.bfloat16, device="cuda")
+    f = pyc_amd.lib().pyc_hip_w8a16_chain_form
+    f.argtypes = [C.c_int] * 2 + [C.c_void_p] * 4
+    for ls in (layers, layers[:2]):
+        n, wq, _, N, K, _ = pyc_amd._chain_arrays(ls)
+        assert f(M, n, C.cast(N, C.c_void_p), C.cast(K, C.c_void_p), X.data_ptr(), C.cast(wq, C.c_void_p)) == 1
+    Yg = torch.empty((M, dims[-1]), dtype=torch.bfloat16, device="cuda")
+    Ye, Ys, Yr = torch.empty_like(Yg), torch.empty_like(Yg), torch.empty_like(Yg)
+    torch.cuda.synchronize()
+    graph, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        graph.capture_begin()
+        rc = _noalloc(torch, X, layers, Yg, stream=s.cuda_stream)
+        graph.capture_end()
+    assert rc == 0
+    torch.cuda.synchronize()
+    for rep in range(4):
+        X.copy_(torch.randn((M, dims[0]), device="cuda").to(torch.bfloat16))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        pyc_amd.w8a16_chain(X, layers, Ye)
+        assert _noalloc(torch, X, layers[:2], Ys) == 0
+        pyc_amd.w8a16_chain(X, layers[:2], Yr)
+        torch.cuda.synchronize()
+        assert torch.equal(Yg, Ye), f"replay {rep} differs from the eager chain"
+        assert torch.equal(Ys, Yr)
+        assert bool(torch.isfinite(Ye.float()).all()) and float(Ye.float().abs().max()) > 0
+    assert pyc_amd.w8a16_chain_error() == 0
