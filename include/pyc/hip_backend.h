@@ -96,15 +96,17 @@ int pyc_hip_w8a16_gemm_dispatch(
     const void* X, const void* Wq, const float* scale, int relu,
     void* Y, void* stream);
 
-/* The decode MLP chain in one launch (no reference counterpart; see
+/* The decode MLP chain in one call (no reference counterpart; see
  * pyc_hip_w8a16_gemm_dispatch): for s = 0..nsteps-1,
  *   X_{s+1} = relu_s?( (X_s * dequant(Wq[s])^T) * scale[s] ),  Y = X_nsteps,
  * X_0 = X bf16 [M, K[0]], Wq[s] e4m3fn [N[s], K[s]], scale[s] fp32 [N[s]],
  * Y bf16 [M, N[nsteps-1]]. 1 <= M <= 32, 1 <= nsteps <= 32, K[s] % 128 == 0,
- * N[s] % 64 == 0, K[s+1] == N[s]. Intermediate activations live in a
- * library-owned device workspace. Returns -1 on bad arguments, and also when
- * the stream is being captured and pyc_hip_w8a16_chain_reserve was not called
- * for this shape first; -2 on a HIP error.
+ * N[s] % 64 == 0, K[s+1] == N[s]. It runs in one persistent launch, or as one launch
+ * per layer where that is estimated to be faster (few tokens, small layers).
+ * Intermediate activations live in a library-owned device workspace. Returns -1 on
+ * bad arguments, and also when the stream is being captured and
+ * pyc_hip_w8a16_chain_reserve was not called for this shape first; -2 on a HIP
+ * error.
  * Symbol "hip_w8a16_chain_e4m3". */
 int pyc_hip_w8a16_chain_dispatch(
     const char* symbol,
@@ -120,8 +122,8 @@ int pyc_hip_w8a16_chain_dispatch(
  * activations, split-K slots) lives in a static device array of
  * PYC_HIP_CHAIN_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds
  * until the process ends, so no reserve call is needed before capturing it.
- * Every call clears its counters with a small kernel on `stream` before the
- * chain kernel (no memset node). Calls on one GPU share the array: calls
+ * A call that takes the one-launch chain kernel clears its counters with a small
+ * kernel on `stream` first (no memset node); layer launches have none. Calls on one GPU share the array: calls
  * whose executions overlap race. The timeout flag is read by
  * pyc_hip_w8a16_chain_error. Returns 0, -1 on bad arguments, -2 on a HIP
  * error, -3 when the chain's workspace exceeds the scratch size (config 5,

@@ -211,7 +211,8 @@ def _chain_arrays(layers):
 
 
 def w8a16_chain(x, layers, y, stream=None, symbol: str = "hip_w8a16_chain_e4m3") -> None:
-    """The whole chain x -> layers -> y in one launch. layers: [(wq [N,K] uint8
+    """The whole chain x -> layers -> y in one call (one launch, or one per layer
+    where that is estimated to be faster). layers: [(wq [N,K] uint8
     e4m3, scale [N] fp32, relu bool), ...], each K equal to the previous N."""
     n, wq, sc, N, K, relu = _chain_arrays(layers)
     _check(lib().pyc_hip_w8a16_chain_dispatch(_b(symbol), int(x.shape[0]), n, _ptr(x), C.cast(wq, C.c_void_p),

@@ -911,7 +911,7 @@ static hipError_t launch_attn_small(int BH, int S, int causal, const void* q, co
     return hipGetLastError();
 }
 
-// Estimated microseconds of each form, fitted to 400 shapes on the MI355X (warm, back
+// Estimated microseconds of each form on 256 CUs, fitted to 400 shapes on the MI355X (warm, back
 // to back; mean error 3 to 6 %, S from 64 to 4096, B H from 8 to 256). Persistent /
 // QW = 2 / QW = 4 of [B,H,S,D]: [2,16,1000,64] 22.8 / 17.1 / 16.7, [1,32,1196,128]
 // causal 43 / 33 / 26.7, [1,8,1260,64] causal 32 / 11.8 / 18.4, [8,16,583,128]

@@ -100,14 +100,15 @@ __device__ inline float gelu_f(float x) {
 }
 
 // One 16-byte chunk per thread, at any alignment (the device runs with unaligned
-// access on; by elements, as unaligned tensors went before, 22.0e6 bf16 took 40 us);
-// the n % kVec tail by elements. Bound: the copy rate. The loads in flight come from the wavefronts
-// (all of a CU's slots), which start and end on their own; more chunks per
-// thread start fewer of them, and a wavefront's chunks then wait for each other.
-// In us, over buffers beyond the caches: one chunk / two / four / the capped grid
-// of 8192 workgroups striding over up to four chunks each that this replaced, bf16:
+// access on); the n % kVec tail by elements. Bound: the copy rate. The loads in flight
+// come from the wavefronts (all of a CU's slots), which start and end on their own;
+// more chunks per thread start fewer of them, and a wavefront's chunks then wait for
+// each other. In us, over buffers beyond the caches: one chunk / two / four / the capped
+// grid of 8192 workgroups striding over up to four chunks each that this replaced, bf16:
 // 4 Mi elements 5.3 / 6.0 / 6.4 / 5.8, 22.0e6 17.7 / 19.7 / 21.7 / 19.2, 64 Mi 44.8 /
-// 50.4 / 49.4 / 55.8; fp32 16 Mi 23.5 / 23.5 / 24.1 / 25.8, 64 Mi 87 / 91 / 91 / 103.
+// 50.4 / 49.4 / 55.8; fp32 16 Mi 23.5 / 23.5 / 24.1 / 25.8, 64 Mi 87 / 91 / 91 / 103. One
+// element off the boundary, where that form went by elements, the same buffers again
+// and again: bf16 22.0e6 16.5 / 23.3 (on it 15.3 / 18.0), fp32 16 Mi 20.4 / 23.1.
 template <typename T>
 __global__ void __launch_bounds__(256) gelu_kernel(const store_t<T>* __restrict__ x, store_t<T>* __restrict__ y,
                                                    size_t n) {
@@ -377,15 +378,7 @@ __global__ void __launch_bounds__(256) layernorm_row_kernel(const store_t<T>* __
                 if (beta) o += b[e];
                 v[e] = o;
             }
-            u32x4 c;
-            if constexpr (V == 4) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) c[e] = __float_as_uint(v[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    c[e] = (uint32_t)elem<T>::from_f32(v[2 * e]) | ((uint32_t)elem<T>::from_f32(v[2 * e + 1]) << 16);
-            }
+            const u32x4 c = IO::pack(v);
             __builtin_memcpy(yr + at(j), &c, 16);
         }
     }

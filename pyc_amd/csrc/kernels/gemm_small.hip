@@ -496,7 +496,10 @@ static int launch_small(int bm, int bn, int M, int N, int K, const void* A, cons
 extern "C" int pyc_hip_gemm_small_takes(int b_trans, int M, int N, int K, const void* A, const void* B) {
     using namespace pyc;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const size_t kpad = (size_t)K + 16 * kSmBK;  // [K,N] k-rows of stages past K must not wrap round to the first ones
+    // [K,N] k-rows past K that are multiplied (against zeros of A) must read zeros and
+    // not wrap round to the first ones: they end with a slot's last stage, less than
+    // 5 stages past K. Later stages are issued too and may wrap, but nothing reads them.
+    const size_t kpad = (size_t)K + 16 * kSmBK;
     if (K % 8 || (!b_trans && N % 4) || (((uintptr_t)A | (uintptr_t)B) & 15) || (size_t)M * K * 2 > kSmPastEnd ||
         (size_t)N * K * 2 > kSmPastEnd || ((K % kSmBK || !b_trans) && (size_t)N * kpad * 2 > kSmPastEnd))
         return K < 8 || (!b_trans && N < 8) ? 0 : 1;
