@@ -915,7 +915,8 @@ static hipError_t launch_attn_small(int BH, int S, int causal, const void* q, co
 // to back; mean error 3 to 6 %, S from 64 to 4096, B H from 8 to 256). Persistent /
 // QW = 2 / QW = 4 of [B,H,S,D]: [2,16,1000,64] 22.8 / 17.1 / 16.7, [1,32,1196,128]
 // causal 43 / 33 / 26.7, [1,8,1260,64] causal 32 / 11.8 / 18.4, [8,16,583,128]
-// causal 33.7 / 47 / 36.9, [1,32,2551,128] 121 / 157 / 149, [7,32,539,128] causal
+// causal 33.7 / 47 / 36.9, [1,63,1126,64] 45 / 55 / 41, [1,16,3300,64] 63 / 74 / 66,
+// [1,32,2551,128] 121 / 157 / 149, [7,32,539,128] causal
 // 60 / 80 / 66, [8,32,2048,64] causal 190 / 312 / 207, [1,12,64,64] 5.8 / 4.9 / 4.7.
 // The persistent form takes a fixed part and, per round of its grid, a start and
 // one time per 64-key block of its longest workgroup, more with more CUs busy.
@@ -943,8 +944,9 @@ static double attn_cost_small(int BH, int S, int D, int causal, int qw) {
     if (!causal) {
         if (D == 128) return qw == 2 ? 1.5 + r1 * (5.2 + n * 1.19) : 1.1 + r1 * (5.7 + n * 1.04);
         const double r2 = (double)((wgs + 511) / 512);
-        return qw == 2 ? 2.65 + 2.1 * r1 + n * (0.236 * r1 + 0.37 * r2 + 0.18 * per_cu)
-                       : 1.85 + 2.9 * r1 + n * (0.237 * r1 + 0.4 * r2 + 0.086 * per_cu);
+        // 918 shapes: mean error 5 %
+        return qw == 2 ? 2.05 + 2.07 * r1 + n * (0.241 * r1 + 0.518 * r2 + 0.135 * per_cu)
+                       : 2.0 + 2.19 * r1 + n * (0.319 * r1 + 0.375 * r2 + 0.064 * per_cu);
     }
     // q-block q walks (q + 1) bq keys; the steps of all of them
     const double m = nqb, sum = qw == 2 ? (double)((long)(nqb + 1) * (nqb + 1) / 4) : m * (m + 1.0) - (2.0 * m - n);
@@ -967,7 +969,15 @@ static double attn_cost_small(int BH, int S, int D, int causal, int qw) {
     return t + (qw == 2 ? 0.1 : -3.4);
 }
 
-// form: 0 = the cheapest by estimate, 1 = persistent, 2 / 4 = small with that QW
+// The cheapest form by estimate: 1 = persistent, 2 / 4 = small with that QW. The
+// estimates' error: a small form has to be 5 % ahead.
+static int attn_form(int BH, int S, int D, int causal) {
+    const double c1 = attn_cost_persist(BH, S, D, causal), c2 = attn_cost_small(BH, S, D, causal, 2),
+                 c4 = attn_cost_small(BH, S, D, causal, 4);
+    return c1 <= 1.05 * c2 && c1 <= 1.05 * c4 ? 1 : c2 <= c4 ? 2 : 4;
+}
+
+// form: 0 = attn_form's, or one of its forms
 template <typename T, int D>
 static hipError_t launch_attn(int form, int B, int H, int S, int causal, const void* q, const void* k,
                               const void* v, void* o, float scale, hipStream_t s) {
@@ -977,12 +987,7 @@ static hipError_t launch_attn(int form, int B, int H, int S, int causal, const v
     const uint16_t* kk = (const uint16_t*)k;
     const uint16_t* vv = (const uint16_t*)v;
     uint16_t* oo = (uint16_t*)o;
-    if (form == 0) {
-        const double c1 = attn_cost_persist(BH, S, D, causal), c2 = attn_cost_small(BH, S, D, causal, 2),
-                     c4 = attn_cost_small(BH, S, D, causal, 4);
-        // the estimates' error: a small form has to be 5 % ahead
-        form = c1 <= 1.05 * c2 && c1 <= 1.05 * c4 ? 1 : c2 <= c4 ? 2 : 4;
-    }
+    if (form == 0) form = attn_form(BH, S, D, causal);
     if (form == 2) return launch_attn_small<T, D, 2>(BH, S, causal, q, k, v, o, scale_log2, s);
     if (form == 4) return launch_attn_small<T, D, 4>(BH, S, causal, q, k, v, o, scale_log2, s);
     const int bq = kAttnWaves * 32;
@@ -1001,6 +1006,11 @@ static hipError_t launch_attn(int form, int B, int H, int S, int causal, const v
 }
 
 }  // namespace pyc
+
+// attn_form for BH heads of S queries and keys. Host only.
+extern "C" int pyc_hip_attention_form(int BH, int S, int D, int causal) {
+    return (D == 64 || D == 128) && BH > 0 && S > 0 ? pyc::attn_form(BH, S, D, causal) : -1;
+}
 
 // form: see launch_attn; -1 for an unknown form or head dim
 extern "C" int pyc_hip_attention_launch_form(int form, int is_bf16, int B, int H, int S, int D, int causal,

@@ -1,4 +1,4 @@
-"""Which kernel fp32 GEMM and LayerNorm calls take, on the CPU (the choice looks at
+"""Which kernel fp32 GEMM, LayerNorm and attention calls take, on the CPU (the choice looks at
 sizes and at the operands' alignment only)."""
 import ctypes as C
 
@@ -51,3 +51,14 @@ def test_layernorm_row_kernel(dtype, rows, d, off, row):
     f = pyc_amd.lib().pyc_hip_layernorm_row_form
     f.argtypes = [C.c_int] * 3 + [C.c_void_p] * 4
     assert f(dtype, rows, d, BASE + off, BASE, BASE, BASE) == row
+
+
+@pytest.mark.parametrize("bh,s,d,causal,form", [
+    (63, 1126, 64, 0, 4), (16, 3300, 64, 0, 1), (66, 3064, 64, 0, 1), (32, 1000, 64, 0, 4),
+    (256, 2048, 128, 1, 1), (32, 1196, 128, 1, 4), (8, 1260, 64, 1, 2), (32, 2551, 128, 0, 1)])
+def test_attention_form(bh, s, d, causal, form):
+    """The form that is the fastest of the three there, by more than a few percent where
+    it is a small one."""
+    f = pyc_amd.lib().pyc_hip_attention_form
+    f.argtypes = [C.c_int] * 4
+    assert f(bh, s, d, causal) == form
